@@ -78,11 +78,9 @@ public:
     float *value_ = nullptr, *buffer_ = nullptr;
     double *d_sum_ = nullptr;
     // pull rounds (cfg.pull_divisor != UINT32_MAX): the in-edge store, the
-    // frontier bitmaps and pushes of dense rounds, the partial sums of cut
-    // in-lists
+    // push arrays of alternating rounds, the partial sums of cut in-lists
     std::unique_ptr<GraphStore> rev_;
-    uint32_t *fb_[2] = {nullptr, nullptr};
-    uint32_t *pv_ = nullptr;
+    float *pv_[2] = {nullptr, nullptr};
     float *accg_ = nullptr;
 
     uint64_t aux_device_bytes() const override { return rev_ ? rev_->dev_bytes_ : 0; }
@@ -93,19 +91,21 @@ public:
         if (rev_) rev_->mirror_counts(slots, live);
     }
 
+    bool rev_streams() const { return host_edges_ && (cfg_.flags & SG_FLAG_PULL_STREAM); }
+    bool give_back() override { return rev_ && rev_->give_back(); }
     // Whether the engine keeps an in-edge store.
     virtual bool wants_in_store() const { return cfg_.pull_divisor != 0xFFFFFFFFu; }
     void after_load(const uint64_t *row, const uint32_t *col) override {
         if (!wants_in_store()) return;
         const bool pulling = cfg_.pull_divisor != 0xFFFFFFFFu;
-        rev_ = make_in_store(*this, row, col, in_cache_bytes_, pulling, pulling);
+        // a streamed pull reads the slots segment by segment: no plan
+        const bool streams = rev_streams();
+        rev_ = make_in_store(*this, row, col, in_cache_bytes_, pulling && !streams, pulling);
         if (cfg_.pull_divisor == 0xFFFFFFFFu) return;  // the store serves another program only
-        const uint64_t words = ((uint64_t)nv_ + 31) / 32;
-        for (auto &b : fb_) {
-            b = dalloc<uint32_t>(words);
-            fill<uint32_t>(b, words, 0u);
+        for (auto &b : pv_) {
+            b = dalloc<float>((size_t)nv_ + 4);  // read in 16-byte groups
+            fill<uint32_t>((uint32_t *)b, (uint64_t)nv_ + 4, 0u);
         }
-        pv_ = dalloc<uint32_t>(nv_);
         accg_ = dalloc<float>(nv_);
         fill<uint32_t>((uint32_t *)accg_, nv_, 0u);
         sync();
@@ -121,16 +121,31 @@ public:
         const uint64_t div = cfg_.pull_divisor ? cfg_.pull_divisor : (rev_ && rev_->host_edges_ ? 8 : 24);
         return std::max<unsigned long long>(1ull, ne_ / div);
     }
-    bool pulls() const { return pv_ != nullptr; }
-    PullTake take_state(uint32_t R) const { return PullTake{fb_[R & 1], pv_, rev_ ? rev_->relabel_ : nullptr}; }
-    // Round R's frontier bitmap starts empty (it last served round R - 2).
-    void clear_take(uint32_t R) {
-        if (!pulls()) return;
-        const uint64_t words = ((uint64_t)nv_ + 31) / 32;
-        round_launch(k_fill_u32, dim3(grid_for(words, 256, 2048)), dim3(256), fb_[R & 1], words, 0u);
+    bool pulls() const { return accg_ != nullptr; }
+    // Share of a pull pass's waves that take the tiles in host memory
+    // (64ths): the host link saturates with far fewer waves than the HBM
+    // gathers need.
+    static constexpr uint32_t kHostWaves64 = SG_PULL_HOST_WAVES64;
+    PrState pr_state(uint32_t R) const {
+        PrState p{};
+        p.op = op_;
+        p.value = value_;
+        p.res = buffer_;
+        p.pv_in = pv_[R & 1];
+        p.pv_out = pv_[(R + 1) & 1];
+        p.accg = accg_;
+        p.relabel = rev_->relabel_;
+        p.unlabel = rev_->unlabel_;
+        p.deg = deg_;
+        p.cnt_in = pcnt_ + (R % 3);
+        p.cnt_out = pcnt_ + ((R + 1) % 3);
+        p.cnt_zero = pcnt_ + ((R + 2) % 3);
+        p.stamp = stamp_;
+        p.hot = ((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nv_, ne_ / (kPrHotEdges * pr_grid()))) + 3u) & ~3u;
+        p.host_waves64 = kHostWaves64;
+        return p;
     }
     PassIO pr_io(PassIO io) const {
-        if (!pulls()) return io;
         const uint32_t R = io.round;
         io.ecnt_in = ecnt_ + (R % 3);
         io.ecnt_out = ecnt_ + ((R + 1) % 3);
@@ -139,94 +154,109 @@ public:
         io.dense_thr = dense_thr();
         return io;
     }
-    // Share of a pull pass's waves that take the tiles beyond the HBM mirror
-    // (64ths): the host link saturates with far fewer waves than the HBM
-    // gathers need.
-    static constexpr uint32_t kHostWaves64 = SG_PULL_HOST_WAVES64;
-    PullPR pull_state(uint32_t R, bool split = true) const {
-        return PullPR{fb_[R & 1], (const float *)pv_, buffer_, accg_, stamp_, R, (float)cfg_.pr_epsilon,
-                      split && rev_ ? rev_->tile_split() : nullptr, kHostWaves64};
+    // one block per CU: it takes the CU's whole LDS
+    uint32_t pr_grid() const { return (uint32_t)std::max(num_cus_, 1); }
+    PullSlots pr_slots() const {
+        return PullSlots{rev_->gview(), rev_->dpre_, rev_->tiles_, rev_->col_, 0, 0u, nv_, 0, rev_->ntiles()};
     }
-
-    // Pull pass of round R over the whole in-edge store (resident store).
-    // force = 0: the kernels return unless the round is dense (device flag).
-    void pull_resident(const PassIO &io, int force, bool timed) {
-        const uint64_t nt = rev_->ntiles();
-        const uint32_t grid = sweep_grid(k_pr_pull, nt);
-        begin_timed(timed && !batch_, SG_KCLASS_PULL);
-        round_launch(k_pr_pull, dim3(grid), dim3(kSweepBlock), rev_->gview(), (const unsigned long long *)rev_->dpre_,
-                     rev_->tiles_, (const uint32_t *)rev_->col_, (uint64_t)0, 0u, nv_, (uint64_t)0, nt, pull_state(io.round),
-                     io, force);
-        round_launch(k_pr_pull_fix, dim3(grid_for(nt + 1, kBlock, 4096)), dim3(kBlock),
-                     (const unsigned long long *)rev_->dpre_, nv_, rev_->tiles_, pull_state(io.round), io, force);
-        end_timed(timed && !batch_);
+    void pr_step(const PassIO &io, const PrState &p, int mode) {
+        if (rev_->plan_ok_)
+            round_launch(k_pr_step<true>, dim3(pr_grid()), dim3(kPrBlock), gview(), rev_->plan_, PullSlots{}, p, io, mode);
+        else
+            round_launch(k_pr_step<false>, dim3(pr_grid()), dim3(kPrBlock), gview(), PullPlan{}, pr_slots(), p, io, mode);
     }
-    // The same with the store's edges in pinned host memory: its SEGMENT slot
-    // ranges stream through HBM staging buffers while earlier ones are pulled.
-    void pull_streamed(const PassIO &io, bool timed) {
-        const uint64_t nt = rev_->ntiles();
-        const PullPR ps = pull_state(io.round, false);  // segments are staged in HBM: no split
-        GraphView rg = rev_->gview();
-        rg.tail = nullptr;  // the staged segments stand in for the host copy
-        const unsigned long long *rdpre = rev_->dpre_;
-        const SweepTiles rt = rev_->tiles_;
-        begin_timed(timed, SG_KCLASS_PULL);
+    void pr_tail(const PassIO &io, const PrState &p, int mode) {
+        if (rev_->plan_ok_)
+            round_launch(k_pr_tail<true>, dim3(pr_grid()), dim3(kPrBlock), gview(), rev_->plan_,
+                         (const unsigned long long *)nullptr, SweepTiles{}, p, io, mode);
+        else
+            round_launch(k_pr_tail<false>, dim3(pr_grid()), dim3(kPrBlock), gview(), PullPlan{},
+                         (const unsigned long long *)rev_->dpre_, rev_->tiles_, p, io, mode);
+    }
+    // A pull over the store with its edges in pinned host memory: the SEGMENT
+    // slot ranges stream through HBM staging buffers while earlier ones are
+    // pulled.
+    void pull_streamed(const PassIO &io, const PrState &p) {
+        PullSlots sl = pr_slots();
+        const uint64_t nt = sl.t_end;
         const uint64_t b0 = rev_->st_.streamed_bytes;
         const double ms0 = rev_->st_.stream_ms;
         rev_->streamed_sweep([&](const uint32_t *colp, uint64_t slo, uint32_t va, uint32_t vb, uint64_t tlo, uint64_t thi) {
-            const uint32_t grid = sweep_grid(k_pr_pull, thi - tlo);
-            hipLaunchKernelGGL(k_pr_pull, dim3(grid), dim3(kSweepBlock), 0, stream_, rg, rdpre, rt, colp, slo, va, vb, tlo,
-                               std::min<uint64_t>(thi, nt), ps, io, 1);
+            sl.colp = colp;
+            sl.slot_lo = slo;
+            sl.dst_lo = va;
+            sl.dst_hi = vb;
+            sl.t_begin = tlo;
+            sl.t_end = std::min<uint64_t>(thi, nt);
+            hipLaunchKernelGGL(k_pr_step<false>, dim3(pr_grid()), dim3(kPrBlock), 0, stream_, gview(), PullPlan{}, sl, p, io,
+                               (int)kPrPull);
             SG_LAUNCHED();
         });
-        hipLaunchKernelGGL(k_pr_pull_fix, dim3(grid_for(nt + 1, kBlock, 4096)), dim3(kBlock), 0, stream_, rdpre, nv_, rt, ps,
-                           io, 1);
-        SG_LAUNCHED();
-        end_timed(timed);
         st_.streamed_bytes += rev_->st_.streamed_bytes - b0;  // the in-store's segments crossed the host link
         st_.stream_ms += rev_->st_.stream_ms - ms0;
     }
     // The touched sources' amend pushes (type -1: cancel, +1: compensate)
-    // delivered by one pull over the in-store as it stands; what crosses
-    // epsilon joins round R's frontier (stamp R).
-    void amend_pull(uint32_t R, int type) {
-        const uint64_t words = ((uint64_t)nv_ + 31) / 32;
-        const PullTake t = take_state(R - 1);  // the pull of "round R - 1" reads it and stamps R
-        fill<uint32_t>(t.bits, words, 0u);
-        hipLaunchKernelGGL(k_pr_amend_take, dim3(grid_for(nv_, 256, 4096)), dim3(256), 0, stream_,
-                           (const uint32_t *)touched_, (const uint32_t *)&ctl_->tcount, nv_, op_, type, value_, buffer_,
-                           (const uint32_t *)deg_, t);
+    // delivered by one pull over the in-store as it stands.
+    void amend_pull(int type) {
+        rev_->ready();
+        const uint32_t R = R_;
+        PrState p = pr_state(R);
+        p.cnt_zero = nullptr;
+        hipLaunchKernelGGL(k_pr_amend_take, dim3(1024), dim3(256), 0, stream_, (const uint32_t *)touched_,
+                           (const uint32_t *)&ctl_->tcount, nv_, p, type, pv_[R & 1]);
         SG_LAUNCHED();
-        PassIO io = seed_io(R, nullptr, nullptr, 0);
-        io.round = R - 1;
+        PassIO io = base_io();
+        io.round = R;
         // counted as a pull round on the device: the next pr_rounds adds its bytes
-        pull_resident(io, 1, timing(SG_KCLASS_PULL));
+        const bool timed = timing(SG_KCLASS_PULL);
+        begin_timed(timed, SG_KCLASS_PULL);
+        pr_step(io, p, kPrAccum);
+        pr_tail(io, p, kPrAccum);
+        end_timed(timed);
     }
 
-    // One round: push (k_round) or, when the frontier's out-edges pass the
-    // threshold, take + pull + fix-up (the round kernel only takes the
-    // frontier's pushes then).
+    // One round over the in-edge store, in the form the device picks.
     void pr_round(const PassIO &io0, bool do_time) {
         const PassIO io = pr_io(io0);
-        const uint32_t R = io.round;
-        clear_take(R);
-        launch_pass(io, VPageRank{op_, value_, buffer_, take_state(R)},
-                    ERelax<api::PageRank>{op_, buffer_, stamp_, R + 1, 0, 0}, do_time);
-        if (pulls()) pull_resident(io, 0, do_time && timing(SG_KCLASS_PULL));
+        const PrState p = pr_state(io.round);
+        begin_timed(do_time && !batch_);
+        pr_step(io, p, kPrAuto);
+        pr_tail(io, p, kPrAuto);
+        end_timed(do_time && !batch_);
+    }
+    // Rounds given up (cfg.max_rounds): the pushes taken for round R_ are still
+    // delivered, so that values and residuals stay those of some push order.
+    void settle() {
+        PrState p = pr_state(R_);
+        p.cnt_zero = nullptr;
+        PassIO io = base_io();
+        io.round = R_;
+        pr_step(io, p, kPrAccum);
+        pr_tail(io, p, kPrAccum);
+        ++R_;
+        sync();
     }
 
     // Rounds from the frontier of round R_ to convergence.
     uint32_t pr_rounds(bool timed, int phase = -1) {
-        if (pulls()) {  // out-edges of the seeded frontier: the first round's direction
-            hipLaunchKernelGGL(k_list_degsum, dim3(256), dim3(kBlock), 0, stream_, (const uint32_t *)q_[R_ & 1],
-                               (const uint32_t *)(cnt_ + (R_ % 3)), nv_, (const uint32_t *)deg_, ecnt_ + (R_ % 3));
-            SG_LAUNCHED();
-        }
-        if (pulls() && rev_->host_edges_ && (cfg_.flags & SG_FLAG_PULL_STREAM)) return pr_rounds_host(timed);
         const bool do_time = timed && timing(SG_KCLASS_RELAX);
+        if (!pulls())
+            return run_rounds([&](uint32_t sv) {
+                return std::make_pair(VCombine<api::PageRank>{op_, value_, buffer_},
+                                      ERelax<api::PageRank>{op_, buffer_, stamp_, sv, 0, 0});
+            }, timed, phase);
+        rev_->ready();
         const uint64_t p0 = st_.pull_rounds;
-        const uint32_t r = drive_rounds([&](const PassIO &io) { pr_round(io, do_time); }, timed, phase);
-        // the pull kernels of push rounds returned at once: bytes only for the rounds that pulled
+        uint32_t r = 0;
+        try {
+            if (rev_streams()) r = pr_rounds_host(timed);
+            else r = drive_rounds([&](const PassIO &io) { pr_round(io, do_time); }, timed, phase, 0, true);
+        } catch (const Error &) {
+            batch_ = nullptr;
+            settle();
+            throw;
+        }
+        // bytes only for the rounds that pulled
         if (timed && timing(SG_KCLASS_PULL))
             kt_bytes_[SG_KCLASS_PULL] += (st_.pull_rounds - p0) * (8ull * ne_ + 24ull * nv_);
         return r;
@@ -237,12 +267,11 @@ public:
     // the whole store over the host link, so a push round must not start one).
     uint32_t pr_rounds_host(bool timed) {
         const bool do_time = timed && timing(SG_KCLASS_RELAX);
-        const uint64_t p0 = st_.pull_rounds;
         if (timed) fill<unsigned long long>(stats_ + 8, 8, 0ull);
         const uint32_t maxr = cfg_.max_rounds ? cfg_.max_rounds : 1000000u;
         read_block();
         uint32_t rounds = 0;
-        last_appended_ = h_blk_[R_ % 3];
+        last_appended_ = h_blk_[R_ % 3] + h_pcnt()[R_ % 3];
         for (;;) {
             const uint32_t R = R_;
             PassIO io = round_io(R);
@@ -250,26 +279,26 @@ public:
             io.round = R;
             if (timed) io.stats = stats_ + 8;
             io = pr_io(io);
-            const bool dense = h_ecnt()[R % 3] > io.dense_thr;
-            clear_take(R);
-            launch_pass(io, VPageRank{op_, value_, buffer_, take_state(R)},
-                        ERelax<api::PageRank>{op_, buffer_, stamp_, R + 1, 0, 0}, do_time);
-            if (dense) pull_streamed(io, do_time && timing(SG_KCLASS_PULL));
+            const bool pull = h_ecnt()[R % 3] > io.dense_thr && h_pcnt()[R % 3];
+            const PrState p = pr_state(R);
+            begin_timed(do_time, pull ? SG_KCLASS_PULL : SG_KCLASS_RELAX);
+            if (pull) pull_streamed(io, p);
+            else pr_step(io, p, kPrAuto);
+            pr_tail(io, p, kPrAuto);
+            end_timed(do_time);
             ++R_;
             ++rounds;
             read_block();
             if (do_time) harvest_events();
-            const uint32_t front = h_blk_[(R + 1) % 3], spill = h_blk_[3 + R % 3];
+            const uint32_t front = h_blk_[(R + 1) % 3] + h_pcnt()[(R + 1) % 3];
             last_appended_ += front;
-            if (front == 0 && spill == 0) break;
+            if (front == 0) break;
             if (rounds >= maxr) {
                 finish_rounds(timed);
                 fail(SG_EDEVICE, "no convergence within " + std::to_string(maxr) + " rounds");
             }
         }
         finish_rounds(timed);
-        if (timed && timing(SG_KCLASS_PULL))
-            kt_bytes_[SG_KCLASS_PULL] += (st_.pull_rounds - p0) * (8ull * ne_ + 24ull * nv_);
         return rounds;
     }
 
@@ -317,16 +346,28 @@ public:
         hipLaunchKernelGGL(k_init_state<api::PageRank>, dim3(grid_for(nv_, 256, 16384)), dim3(256), 0, stream_, nv_, op_, value_,
                            buffer_);
         SG_LAUNCHED();
-        frontier_reset();
-        hipLaunchKernelGGL(k_seed_active<api::PageRank>, dim3(grid_for(nv_, kBlock, 16384)), dim3(kBlock), 0, stream_, nv_, op_,
-                           value_, buffer_, stamp_, R_, q_[R_ & 1], cnt_ + (R_ % 3), stats_ + 3);
-        SG_LAUNCHED();
+        seed<false>();
         st_.rounds = pr_rounds(false);
         residual();
         init_others();
         cache_rebuild();
         inited_ = true;
         st_.last_phase_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+    // Every vertex with a residual past epsilon (kBothSigns: or below -epsilon)
+    // starts round R_.
+    template <bool kBothSigns>
+    void seed() {
+        frontier_reset();
+        if (pulls()) {
+            PassIO io = base_io();
+            io.ecnt_out = ecnt_ + (R_ % 3);
+            hipLaunchKernelGGL(k_pr_seed<kBothSigns>, dim3(pr_grid()), dim3(kPrBlock), 0, stream_, nv_, pr_state(R_ - 1), io);
+        } else {
+            hipLaunchKernelGGL((k_seed_active<api::PageRank, kBothSigns>), dim3(grid_for(nv_, kBlock, 16384)), dim3(kBlock), 0,
+                               stream_, nv_, op_, value_, buffer_, stamp_, R_, q_[R_ & 1], cnt_ + (R_ % 3), stats_ + 3);
+        }
+        SG_LAUNCHED();
     }
     // Programs that share this engine's stores: their static solve, and their
     // recompute after each committed batch (PageRank's rounds done).
@@ -346,10 +387,10 @@ public:
         const uint32_t *tc = &ctl_->tcount;
         if (pulls()) {
             // cancel over the old in-lists, compensate over the new ones: two pulls
-            amend_pull(R, -1);
+            amend_pull(-1);
             commit(overflow);
             rev_->apply(d_ins, nins, d_del, ndel);
-            amend_pull(R, +1);
+            amend_pull(+1);
         } else {
             {
                 PassIO io = seed_io(R, touched_, tc, 0);
@@ -367,14 +408,15 @@ public:
             }
         }
         if (cfg_.flags & SG_FLAG_DEFER_CONVERGE) {
-            // the long new lists were cut into chunks for the first round: walk
-            // them now. The residual then holds alpha * (A' - A) * value on top
-            // of the old one, exact for any committed value: later snapshots add
-            // theirs and one convergence serves them all
-            drain_seed_spill(R, ERelax<api::PageRank>{op_, buffer_, stamp_, R, 0, 0});
+            // (push form: the long new lists were cut into chunks for the first
+            // round, walk them now.) The residual then holds alpha * (A' - A) *
+            // value on top of the old one, exact for any committed value: later
+            // snapshots add theirs and one convergence serves them all
+            if (!pulls()) drain_seed_spill(R, ERelax<api::PageRank>{op_, buffer_, stamp_, R, 0, 0});
             pending_ = true;
             st_.rounds = 0;
         } else {
+            if (pulls()) seed<true>();  // whatever the two pulls left past +-epsilon
             st_.rounds = pr_rounds(true, kPhaseRelax);
         }
         recompute_others();
@@ -392,10 +434,7 @@ public:
     void converge() override {
         if (!pending_) return;
         auto t0 = std::chrono::steady_clock::now();
-        frontier_reset();
-        hipLaunchKernelGGL((k_seed_active<api::PageRank, true>), dim3(grid_for(nv_, kBlock, 16384)), dim3(kBlock), 0, stream_, nv_, op_,
-                           value_, buffer_, stamp_, R_, q_[R_ & 1], cnt_ + (R_ % 3), stats_ + 3);
-        SG_LAUNCHED();
+        seed<true>();
         st_.rounds = pr_rounds(true, kPhaseRelax);
         pending_ = false;
         residual();

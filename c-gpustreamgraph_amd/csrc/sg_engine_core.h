@@ -667,14 +667,23 @@ public:
     uint64_t budget_used() const {
         return dev_bytes_ + aux_device_bytes() + (budget_peer_ ? budget_peer_->dev_bytes_ : 0);
     }
+    // Frees device memory that only makes the engine faster (a resident pull
+    // plan); false when there is none. Tried before an allocation is refused.
+    virtual bool give_back() { return false; }
     template <class T>
     T *dalloc(size_t count) {
         const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
         const double budget = cfg_.device_budget_gb * 1073741824.0;
-        if (budget > 0 && (double)(budget_used() + bytes) > budget)
+        auto over = [&]() { return budget > 0 && (double)(budget_used() + bytes) > budget; };
+        if (over() && give_back() && !over()) return dalloc<T>(count);
+        if (over())
             fail(SG_EBUDGET, "device budget exceeded: need " + std::to_string(budget_used() + bytes) + " bytes");
         void *p = nullptr;
         hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            if (give_back()) return dalloc<T>(count);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             fail(SG_EBUDGET, std::string("hipMalloc of ") + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
@@ -785,8 +794,9 @@ public:
     //   [0] edges (light), [1] vertices, [2] edges (spilled chunks), [3] overflow
     //   flags, [4] pull rounds, [5] edges read from the HBM cache, [6..7] cache
     //   rebuild counts, [8..15] the same as [0..7] for timed rounds.
-    //   Then u64 ecnt[4]: out-edges of the frontiers of rounds R % 3 (direction choice).
-    static constexpr size_t kCtlBlockBytes = (8 + 2 * kRoundLog) * 4 + 16 * 8 + 4 * 8;
+    //   Then u64 ecnt[4]: out-edges of the frontiers of rounds R % 3 (direction choice),
+    //   and u32 pcnt[4]: sources of the frontiers kept as push arrays (PageRank).
+    static constexpr size_t kCtlBlockBytes = (8 + 2 * kRoundLog) * 4 + 16 * 8 + 4 * 8 + 4 * 4;
     uint32_t *cnt_ = nullptr;    // [3] rotating round counters
     uint32_t *hcnt_ = nullptr;   // [3] rotating spill counters
     uint32_t *rlog_ = nullptr;
@@ -796,6 +806,7 @@ public:
     size_t heavy_cap_ = 0;
     unsigned long long *stats_ = nullptr;  // [0..3] pass stats, [4] inval count
     unsigned long long *ecnt_ = nullptr;   // [3] rotating frontier out-edge counters
+    uint32_t *pcnt_ = nullptr;             // [3] rotating counters of push-array frontiers
     uint32_t *stamp_ = nullptr;
     uint32_t *inval_ = nullptr;   // bitmap of invalidated vertices
     uint32_t *coarse_ = nullptr;  // coarse filter of inval_: one bit per 2^cshift_ vertices
@@ -875,6 +886,7 @@ public:
     unsigned long long *h_u64_ = nullptr;  // [16]
     const unsigned long long *h_stats() const { return (const unsigned long long *)(h_blk_ + 8 + 2 * kRoundLog); }
     const unsigned long long *h_ecnt() const { return h_stats() + 16; }
+    const uint32_t *h_pcnt() const { return (const uint32_t *)(h_ecnt() + 4); }
 
     // --- kernel timing --------------------------------------------------------
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events_;
@@ -1016,18 +1028,23 @@ public:
         leaf_dirty_ = dalloc<uint8_t>(nleaves_);
         chosen_ = dalloc<uint8_t>(2 * nleaves_);
         maximal_ = dalloc<uint8_t>(2 * nleaves_);
-        q_[0] = dalloc<uint32_t>(nv);
-        q_[1] = dalloc<uint32_t>(nv);
+        if (has_rounds()) {
+            q_[0] = dalloc<uint32_t>(nv);
+            q_[1] = dalloc<uint32_t>(nv);
+        }
         // control block: counters, round log and stats, read back by one copy
         cnt_ = (uint32_t *)dalloc<unsigned long long>(kCtlBlockBytes / 8);
         hcnt_ = cnt_ + 3;
         rlog_ = cnt_ + 8;
         stats_ = (unsigned long long *)(cnt_ + 8 + 2 * kRoundLog);
         ecnt_ = stats_ + 16;
-        stamp_ = dalloc<uint32_t>(nv);
-        inval_ = dalloc<uint32_t>(((size_t)nv + 31) / 32);
+        pcnt_ = (uint32_t *)(ecnt_ + 4);
         cshift_ = coarse_shift_for(nv);
-        coarse_ = dalloc<uint32_t>(coarse_words(nv, cshift_));
+        if (has_rounds()) {
+            stamp_ = dalloc<uint32_t>(nv);
+            inval_ = dalloc<uint32_t>(((size_t)nv + 31) / 32);
+            coarse_ = dalloc<uint32_t>(coarse_words(nv, cshift_));
+        }
         mark_ = dalloc<uint32_t>(((size_t)nv + 31) / 32);
         tidx_ = dalloc<uint32_t>(nv);
         br_.ins_b = dalloc<uint32_t>(nv);
@@ -1074,13 +1091,15 @@ public:
         fill<uint8_t>(chosen_, 2 * nleaves_, 0);
         fill<uint8_t>(maximal_, 2 * nleaves_, 0);
         fill<uint32_t>(mark_, ((uint64_t)nv + 31) / 32, 0u);
-        fill<uint32_t>(inval_, ((uint64_t)nv + 31) / 32, 0u);
-        fill<uint32_t>(coarse_, coarse_words(nv, cshift_), 0u);
+        if (has_rounds()) {
+            fill<uint32_t>(inval_, ((uint64_t)nv + 31) / 32, 0u);
+            fill<uint32_t>(coarse_, coarse_words(nv, cshift_), 0u);
+            fill<uint32_t>(stamp_, nv, 0);
+        }
         fill<uint32_t>(br_.ins_b, nv, 0u);
         fill<uint32_t>(br_.ins_e, nv, 0u);
         fill<uint32_t>(br_.del_b, nv, 0u);
         fill<uint32_t>(br_.del_e, nv, 0u);
-        fill<uint32_t>(stamp_, nv, 0);
         fill<uint32_t>(cnt_, kCtlBlockBytes / 4, 0u);
         fill<uint8_t>((uint8_t *)ctl_, sizeof(Ctl), 0);
         if (cache_slots_) {
@@ -1105,9 +1124,12 @@ public:
     virtual uint64_t aux_device_bytes() const { return 0; }
     virtual uint64_t aux_host_bytes() const { return 0; }
     virtual uint64_t in_capacity() const { return 0; }
+    // A store without a vertex program keeps no frontiers, stamps or spill queues.
+    virtual bool has_rounds() const { return true; }
     virtual void in_mirror(uint64_t &slots, uint64_t &live) { slots = live = 0; }
 
     void ensure_heavy(uint64_t edges) {
+        if (!has_rounds()) return;
         // every list past a wave's budget becomes >= 1 descriptor: at most one per
         // vertex plus one per kChunk edges, per pass
         const size_t need = (size_t)(edges / kChunk + nv_ + 4096);
@@ -1129,10 +1151,9 @@ public:
     // GraphStore): the tile sweeps read those edges from HBM.
     uint32_t *mirror_ = nullptr;
     uint64_t mirror_live_ = 0;
-    uint32_t *tail_ = nullptr;  // gap-free host copy of the live edges past the mirror (GraphStore)
-    uint32_t mbits_ = 32;       // bits per id in the mirror and the tail
+    uint32_t mbits_ = 32;       // bits per id in the mirror
     GraphView gview() const {
-        GraphView g{nv_, off_, deg_, col_, nullptr, nullptr, cap_, nullptr, mirror_, std::min(mirror_live_, ne_), tail_, mbits_};
+        GraphView g{nv_, off_, deg_, col_, nullptr, nullptr, cap_, nullptr, mirror_, std::min(mirror_live_, ne_), mbits_};
         if (cache_slots_) {
             g.ccol = ccol_[ccur_];
             g.coff = coff_;
@@ -1198,7 +1219,7 @@ public:
     // round R's frontier and spill into hq[(R + 2) % 3].
     void frontier_reset() {  // word 7 stays zero: an empty list count
         fill<uint32_t>(cnt_, 8, 0);
-        fill<unsigned long long>(ecnt_, 4, 0ull);
+        fill<unsigned long long>(ecnt_, 6, 0ull);  // and pcnt
     }
 
     PassIO base_io() const {
@@ -1432,9 +1453,12 @@ public:
     // runs longer continues with batches of 4, 8, ...
     // limit > 0: stop after about `limit` rounds (whole batches) even if work
     // remains (stopped_ tells which); the frontier and spills stay for the next call.
+    // pr: PageRank rounds over an in-edge store. They leave no spilled work to
+    // the next round, and the log's second word says whether a round pulled
+    // (one timed event pair per round: pull or relax class).
     bool stopped_ = false;
     template <class Launch>
-    uint32_t drive_rounds(Launch launch, bool timed, int phase = -1, uint32_t limit = 0) {
+    uint32_t drive_rounds(Launch launch, bool timed, int phase = -1, uint32_t limit = 0, bool pr = false) {
         stopped_ = false;
         uint32_t k0 = cfg_.rounds_per_sync ? cfg_.rounds_per_sync : 4;
         const bool adaptive = !cfg_.rounds_per_sync && phase >= 0 && last_rounds_[phase];
@@ -1470,6 +1494,10 @@ public:
                 end_timed(do_time);
             }
             read_block();
+            if (do_time && pr && !graphs) {
+                for (uint32_t i = 0; i < k && ev_used_ >= k; ++i)
+                    if (h_blk_[8 + 2 * ((R0 + i) % kRoundLog) + 1]) ev_cls_[ev_used_ - k + i] = SG_KCLASS_PULL;
+            }
             if (do_time) harvest_events();
             if (first) {  // what the seed passes put on the first frontier (logged by the first round)
                 last_appended_ += h_blk_[8 + 2 * ((R0 + kRoundLog - 1) % kRoundLog)];
@@ -1483,9 +1511,10 @@ public:
                     front = h_blk_[8 + 2 * (R % kRoundLog)];
                     spill = h_blk_[8 + 2 * (R % kRoundLog) + 1];
                 } else {
-                    front = h_blk_[(R + 1) % 3];
+                    front = h_blk_[(R + 1) % 3] + h_pcnt()[(R + 1) % 3];
                     spill = h_blk_[3 + R % 3];
                 }
+                if (pr) spill = 0;
                 last_appended_ += front;
                 if (front == 0 && spill == 0) {
                     finish_rounds(timed);
@@ -2130,119 +2159,181 @@ public:
         commit(overflow);
         finish_batch();
         st_.snapshots += 1;
+        refresh();
+    }
+    bool has_rounds() const override { return false; }
+    // What the owner's pulls read, after a load or a batch: the pull plan, or
+    // the merge-path tiles (and the HBM mirror).
+    void refresh() {
+        tiles_stale_ = true;
+        if (want_plan_ && refresh_plan()) return;
+        ready();
+    }
+    bool tiles_stale_ = true;
+    // Tiles for a pull without a plan (the plan may have been given back since).
+    void ready() {
+        if (plan_ok_ || !tiles_stale_) return;
         refresh_tiles();
         refresh_mirror();
+        tiles_stale_ = false;
     }
-    // With the store in pinned host memory, the device edge budget holds an
-    // HBM copy of its leading live edges, gaps left out (every pull round
-    // reads the whole store; those edges then come from HBM instead of over
-    // the host link). Rebuilt after every batch from the live slots (the
-    // live-edge order shifts with every insert and delete).
-    uint64_t mirror_extra_bytes_ = 0;  // HBM beyond the edge budget the owner gives the mirror
-    // With want_tail_ (an owner whose pull rounds read every in-edge), the
-    // live edges past the mirror also get a gap-free copy in pinned host
-    // memory: a pull then reads them as contiguous runs over the host link
-    // instead of short lists scattered between gaps. Rebuilt with the mirror.
-    bool want_tail_ = false;
-    uint64_t tail_cap_ = 0;
-    // Ids are packed at ceil(log2 nv) bits (27 at 2^27 vertices): the same
-    // HBM holds 32 / 27 as many edges, and the host link moves that much less
-    // per tail edge. Packed words are ORed together at run ends, so the copies
-    // are zeroed first. The tail is packed in windows of an HBM stage (at most
-    // kTailStageWords, taken out of the mirror's budget) and each window
-    // copied out before the next is packed, so no more of the store than the
-    // budget allows is held in HBM.
-    static constexpr uint64_t kTailStageWords = 16ull << 20;  // 64 MiB
-    static constexpr uint64_t kTailStageMinWords = 1024;
-    static constexpr uint64_t kCopySlack = 4;
-    uint32_t *tail_stage_ = nullptr;
-    uint64_t tail_stage_cap_ = 0;
+    // Traversal owners: with the store in pinned host memory, the device edge
+    // budget holds an HBM copy of its leading live edges, gaps left out, ids
+    // packed at ceil(log2 nv) bits (the tile sweeps read those from HBM).
+    // Rebuilt after every batch from the live slots (the live-edge order shifts
+    // with every insert and delete). Packed words are ORed together at run
+    // ends, so the copy is zeroed first.
+    uint64_t mirror_extra_bytes_ = 0;  // HBM beyond the edge budget the owner gives the ids
     static uint64_t packed_words(uint64_t n, uint32_t b) { return (n * b + 31) / 32 + 1; }
     static uint64_t ids_in_words(uint64_t words, uint32_t b) { return words > 1 ? (words - 1) * 32 / b : 0; }
+    uint64_t budget_words() const {
+        return (uint64_t)((std::max(0.0, cfg_.edge_budget_gb) * 1073741824.0 + (double)mirror_extra_bytes_) / 4.0);
+    }
+    uint32_t id_bits() const {
+        const uint32_t b = nv_ > 1 ? 32 - (uint32_t)__builtin_clz(nv_ - 1) : 1;
+        return b > 31 ? 32 : b;
+    }
     void refresh_mirror() {
         mirror_live_ = 0;
-        if (!host_edges_) return;
-        const uint32_t b = nv_ > 1 ? 32 - (uint32_t)__builtin_clz(nv_ - 1) : 1;
-        mbits_ = b > 31 ? 32 : b;
-        const double bytes = std::max(0.0, cfg_.edge_budget_gb) * 1073741824.0 + (double)mirror_extra_bytes_;
-        uint64_t cap_words = (uint64_t)(bytes / 4.0);
-        // the tile sweeps read whole 16-byte groups: 4 words of slack past the last id
-        auto fits = [&](uint64_t words) { return ids_in_words(words > kCopySlack ? words - kCopySlack : 0, mbits_); };
-        // a tail needs a stage: its words come out of the mirror's share
-        uint64_t stage_words = 0;
-        if (want_tail_ && ne_ > fits(cap_words)) {
-            stage_words = std::max(kTailStageMinWords, std::min(kTailStageWords, cap_words / 2));
-            cap_words = cap_words > stage_words ? cap_words - stage_words : 0;
-        }
-        const uint64_t want = std::min<uint64_t>(ne_, fits(cap_words));
-        const uint64_t rest = want_tail_ ? ne_ - want : 0;
-        if (want == 0 && rest == 0) return;
-        const uint64_t mwords = want ? packed_words(want, mbits_) : 0;
-        if (mwords && mwords + kCopySlack > mirror_cap_) {
+        if (!host_edges_ || want_plan_) return;
+        mbits_ = id_bits();
+        const uint64_t cap_words = budget_words();
+        const uint64_t want = std::min<uint64_t>(ne_, ids_in_words(cap_words, mbits_));
+        if (want == 0) return;
+        const uint64_t mwords = packed_words(want, mbits_);
+        if (mwords > mirror_cap_) {
             dfree(mirror_);
             mirror_ = nullptr;
-            mirror_cap_ = std::min<uint64_t>(cap_words, mwords + std::max<uint64_t>(kCopySlack, mwords / 8));  // room for growth
-            mirror_ = dalloc<uint32_t>(mirror_cap_);
+            mirror_cap_ = 0;
+            const uint64_t cap = std::min<uint64_t>(cap_words, mwords + mwords / 8);  // room for growth
+            mirror_ = dalloc<uint32_t>(cap);
+            mirror_cap_ = cap;
         }
-        const uint64_t twords = rest ? packed_words(rest, mbits_) : 0;
-        if (twords && twords + kCopySlack > tail_cap_) {
-            hfree(tail_);
-            tail_ = nullptr;
-            tail_cap_ = twords + twords / 8 + kCopySlack;
-            tail_ = halloc<uint32_t>(tail_cap_);
-        }
-        if (rest) {
-            stage_words = std::min(stage_words, twords);
-            if (stage_words > tail_stage_cap_) {
-                dfree(tail_stage_);
-                tail_stage_ = nullptr;
-                tail_stage_ = dalloc<uint32_t>(stage_words);
-                tail_stage_cap_ = stage_words;
-            }
-        }
-        GraphView g = gview();  // without copies: the fill reads the host store
+        GraphView g = gview();  // without the copy: the fill reads the host store
         g.mirror = nullptr;
         g.mlive = 0;
-        g.tail = nullptr;
-        const uint32_t grid = sweep_grid(k_mirror_fill, ntiles());
-        if (want) {
-            if (mbits_ < 32) fill<uint32_t>(mirror_, mwords, 0u);
-            hipLaunchKernelGGL(k_mirror_fill, dim3(grid), dim3(kSweepBlock), 0, stream_, g,
-                               (const unsigned long long *)dpre_, tiles_, mirror_, (uint64_t)want, (uint32_t *)nullptr,
-                               (uint64_t)0, (uint64_t)0, mbits_);
-            SG_LAUNCHED();
-        }
-        // tail windows of win ids (a multiple of 32: each starts on a word)
-        const uint64_t win = rest ? std::max<uint64_t>(32, ids_in_words(stage_words, mbits_) & ~31ull) : 0;
-        for (uint64_t lo = 0; lo < rest; lo += win) {
-            const uint64_t hi = std::min(rest, lo + win);
-            const uint64_t used = ((hi - lo) * mbits_ + 31) / 32;  // words holding the window's bits
-            if (used > tail_stage_cap_) fail(SG_EDEVICE, "tail window exceeds its stage");
-            if (mbits_ < 32) fill<uint32_t>(tail_stage_, used, 0u);
-            hipLaunchKernelGGL(k_mirror_fill, dim3(grid), dim3(kSweepBlock), 0, stream_, g,
-                               (const unsigned long long *)dpre_, tiles_, (uint32_t *)nullptr, (uint64_t)want,
-                               tail_stage_, lo, hi, mbits_);
-            SG_LAUNCHED();
-            SG_HIP(hipMemcpyAsync(tail_ + lo * mbits_ / 32, tail_stage_, used * 4, hipMemcpyDeviceToHost, stream_));
-        }
-        if (!tsplit_) tsplit_ = dalloc<unsigned long long>(1);
-        hipLaunchKernelGGL(k_tile_split, dim3(1), dim3(1), 0, stream_, tiles_, (const unsigned long long *)dpre_, nv_,
-                           (unsigned long long)want, tsplit_);
+        if (mbits_ < 32) fill<uint32_t>(mirror_, mwords, 0u);
+        hipLaunchKernelGGL(k_mirror_fill, dim3(sweep_grid(k_mirror_fill, ntiles())), dim3(kSweepBlock), 0, stream_, g,
+                           (const unsigned long long *)dpre_, tiles_, mirror_, (uint64_t)want, mbits_);
         SG_LAUNCHED();
         mirror_live_ = want;
     }
     uint64_t mirror_cap_ = 0;
-    unsigned long long *tsplit_ = nullptr;  // first tile past the mirror (k_tile_split)
-    // The tile split for pull passes: null without a mirror, or with every
-    // live edge in it.
-    const unsigned long long *tile_split() const {
-        return host_edges_ && mirror_live_ && mirror_live_ < ne_ ? tsplit_ : nullptr;
+
+    // PageRank owners: the pull plan (sg_pull.h). Resident store: all its ids,
+    // where the device budget has room (it is given back when something else
+    // needs the memory; pulls then read the slots). Store in pinned host
+    // memory: HBM holds as many tiles of ids as the edge budget allows, the
+    // rest are packed straight into pinned host memory.
+    bool want_plan_ = false, plan_ok_ = false, plan_refused_ = false;
+    PullPlan plan_{};
+    uint32_t *pl_ids_ = nullptr, *pl_tail_ = nullptr, *pl_heads_ = nullptr, *pl_dst_ = nullptr;
+    PullTileMeta *pl_meta_ = nullptr;
+    uint32_t *pl_n_ = nullptr;
+    unsigned long long *pl_cnt_ = nullptr;
+    size_t pl_ids_cap_ = 0, pl_tail_cap_ = 0, pl_heads_cap_ = 0, pl_meta_cap_ = 0, pl_cnt_cap_ = 0;
+    // A plan buffer of at least need elements: with an eighth to spare, or
+    // exactly where the budget has no room for that.
+    template <class T>
+    void plan_buf(T *&p, size_t &cap, size_t need, uint64_t most = ~0ull) {
+        if (p && need <= cap) return;
+        dfree(p);
+        p = nullptr;
+        cap = 0;
+        const size_t roomy = (size_t)std::min<uint64_t>(most, need + need / 8);
+        try {
+            p = dalloc<T>(roomy);
+            cap = roomy;
+        } catch (const Error &) {
+            p = dalloc<T>(need);
+            cap = need;
+        }
+    }
+    void drop_plan() {
+        for (void *p : {(void *)pl_ids_, (void *)pl_heads_, (void *)pl_dst_, (void *)pl_meta_}) dfree(p);
+        pl_ids_ = pl_heads_ = pl_dst_ = nullptr;
+        pl_meta_ = nullptr;
+        pl_ids_cap_ = pl_heads_cap_ = pl_meta_cap_ = 0;
+        plan_ok_ = false;
+        plan_refused_ = true;
+    }
+    bool plan_building_ = false;
+    bool give_back() override {
+        if (!plan_ok_ || plan_building_ || host_edges_) return false;
+        sync();  // queued pulls read it
+        drop_plan();
+        return true;
+    }
+    bool refresh_plan() {
+        plan_ok_ = false;
+        if (plan_refused_) return false;
+        const uint32_t b = mbits_ = id_bits();
+        const uint64_t nt = (ne_ + kPullTile - 1) / kPullTile, words = pull_tile_words(b);
+        const uint64_t in_hbm = host_edges_ ? std::min(nt, budget_words() / words) : nt;
+        plan_building_ = true;
+        try {
+            plan_buf(pl_heads_, pl_heads_cap_, (size_t)std::max<uint64_t>(1, nt) * (kPullTile / 32));
+            plan_buf(pl_meta_, pl_meta_cap_, (size_t)std::max<uint64_t>(1, nt));
+            if (!pl_dst_) pl_dst_ = dalloc<uint32_t>((size_t)nv_ + kWave);
+            if (!pl_n_) pl_n_ = dalloc<uint32_t>(1);
+            if (in_hbm) plan_buf(pl_ids_, pl_ids_cap_, in_hbm * words, host_edges_ ? budget_words() : ~0ull);
+        } catch (const Error &e) {
+            plan_building_ = false;
+            if (host_edges_) throw;
+            drop_plan();
+            return false;
+        }
+        plan_building_ = false;
+        if (nt > in_hbm && (nt - in_hbm) * words > pl_tail_cap_) {
+            hfree(pl_tail_);
+            pl_tail_ = nullptr;
+            pl_tail_cap_ = 0;
+            const size_t cap = (nt - in_hbm) * words + (nt - in_hbm) * words / 8;
+            pl_tail_ = halloc<uint32_t>(cap);
+            pl_tail_cap_ = cap;
+        }
+        const uint32_t nb = (uint32_t)(((uint64_t)nv_ + kScanSpan - 1) / kScanSpan);
+        ensure(bsum_, bsum_cap_, (size_t)nb + 1);
+        ensure(pl_cnt_, pl_cnt_cap_, (size_t)nb + 1);
+        hipLaunchKernelGGL(k_plan_sums, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, bsum_, pl_cnt_);
+        SG_LAUNCHED();
+        hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, bsum_);
+        SG_LAUNCHED();
+        hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, pl_cnt_);
+        SG_LAUNCHED();
+        fill<uint32_t>(pl_heads_, std::max<uint64_t>(1, nt) * (kPullTile / 32), 0u);
+        unsigned long long *const start = dpre_;  // nv + 1 words: the first edge of every list
+        hipLaunchKernelGGL(k_plan_lists, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, (const unsigned long long *)bsum_,
+                           (const unsigned long long *)pl_cnt_, start, pl_dst_, pl_heads_, pl_n_);
+        SG_LAUNCHED();
+        plan_ = PullPlan{pl_ids_, pl_tail_, pl_heads_, pl_dst_, pl_meta_, nt, in_hbm, ne_, b};
+        if (nt) {
+            hipLaunchKernelGGL(k_plan_meta, dim3(grid_for(nt, 256, 4096)), dim3(256), 0, stream_, nt, ne_,
+                               (const unsigned long long *)start, (const uint32_t *)pl_n_, (const uint32_t *)pl_heads_, pl_meta_);
+            SG_LAUNCHED();
+            auto pack = [&](uint64_t t0, uint64_t t1, uint32_t *out) {
+                hipLaunchKernelGGL(k_plan_ids, dim3(grid_for(t1 - t0, kWavesPerBlock, 8 * std::max(num_cus_, 1))),
+                                   dim3(kBlock), 0, stream_, gview(), plan_, (const unsigned long long *)start, t0, t1, out);
+                SG_LAUNCHED();
+            };
+            if (in_hbm) pack(0, in_hbm, pl_ids_);
+            if (nt > in_hbm) pack(in_hbm, nt, pl_tail_);
+        }
+        plan_ok_ = true;
+        return true;
     }
 
-    // Mirror capacity (ids) and the live edges it holds.
+    // HBM copy of a host-resident store's ids: its capacity and the live edges it holds.
     void mirror_counts(uint64_t &slots, uint64_t &live) {
-        slots = mirror_ && mirror_cap_ > 1 ? (mirror_cap_ - 1) * 32 / mbits_ : 0;
-        live = std::min(mirror_live_, ne_);
+        slots = live = 0;
+        if (!host_edges_) return;
+        if (want_plan_) {
+            slots = pl_ids_cap_ / pull_tile_words(mbits_) * kPullTile;
+            live = plan_ok_ ? std::min(plan_.split * kPullTile, ne_) : 0;
+        } else {
+            slots = mirror_ && mirror_cap_ > 1 ? (mirror_cap_ - 1) * 32 / mbits_ : 0;
+            live = std::min(mirror_live_, ne_);
+        }
     }
     void refresh_tiles() { tiles_ = sweep_tiles(); }
     uint64_t ntiles() const { return ((uint64_t)nv_ + ne_ + kSweepTile - 1) / kSweepTile; }
@@ -2261,15 +2352,18 @@ public:
 };
 
 // In-lists of a CSR (counting sort by target; sources ascending in each list).
-static void transpose_csr(uint32_t nv, uint64_t ne, const uint64_t *row, const uint32_t *col, std::vector<uint64_t> &trow,
-                          std::vector<uint32_t> &tcol) {
+// order (null: identity): the source of each id the in-lists record.
+static void transpose_csr(uint32_t nv, uint64_t ne, const uint64_t *row, const uint32_t *col, const uint32_t *order,
+                          std::vector<uint64_t> &trow, std::vector<uint32_t> &tcol) {
     trow.assign((size_t)nv + 1, 0);
     for (uint64_t e = 0; e < ne; ++e) ++trow[(size_t)col[e] + 1];
     for (uint32_t v = 0; v < nv; ++v) trow[(size_t)v + 1] += trow[v];
     std::vector<uint64_t> pos(trow.begin(), trow.end() - 1);
     tcol.resize(std::max<uint64_t>(ne, 1));
-    for (uint32_t u = 0; u < nv; ++u)
-        for (uint64_t e = row[u]; e < row[(size_t)u + 1]; ++e) tcol[pos[col[e]]++] = u;
+    for (uint32_t i = 0; i < nv; ++i) {
+        const uint32_t u = order ? order[i] : i;
+        for (uint64_t e = row[u]; e < row[(size_t)u + 1]; ++e) tcol[pos[col[e]]++] = i;
+    }
 }
 
 // keys[e] = target << 32 | source of every edge e (one wave per source).
@@ -2352,16 +2446,16 @@ static void transpose_csr_device(hipStream_t st, uint32_t nv, uint64_t ne, const
 // The in-edge store of an engine, built from the CSR it loads (its own device
 // budget counted with the owner's, its work on the owner's stream). In-lists
 // are built on the host for small graphs, on the device from 2^24 edges.
-// mirror_extra_bytes: HBM beyond the edge budget for the store's mirror when
-// its edges live in host memory.
-// tail: the owner's pull rounds read every in-edge (a gap-free host copy of
-// the edges past the mirror pays for its rebuild).
+// mirror_extra_bytes: HBM beyond the edge budget for the ids the store keeps
+// there when its edges live in host memory.
+// plan: the owner's pull rounds read every in-edge (a pull plan pays for its
+// rebuild after every batch).
 // relabel: the in-lists record each source by its rank in descending
 // out-degree instead of its id (hubs first), so the per-in-edge gathers of a
 // pull pass (frontier bit and push of the source) fall on a few hot words
 // that stay in the caches; the store translates batches and queries.
 static std::unique_ptr<GraphStore> make_in_store(Engine &owner, const uint64_t *row, const uint32_t *col,
-                                                 uint64_t mirror_extra_bytes = 0, bool tail = false, bool relabel = false) {
+                                                 uint64_t mirror_extra_bytes = 0, bool plan = false, bool relabel = false) {
     const uint32_t nv = owner.nv_;
     std::vector<uint32_t> rank, unrank;
     if (relabel) {  // counting sort by out-degree, descending; ties by id
@@ -2383,10 +2477,7 @@ static std::unique_ptr<GraphStore> make_in_store(Engine &owner, const uint64_t *
     if (owner.ne_ >= (1ull << 24)) {
         transpose_csr_device(owner.stream_, nv, owner.ne_, row, col, relabel ? rank.data() : nullptr, trow, tcol);
     } else {
-        transpose_csr(nv, owner.ne_, row, col, trow, tcol);
-        if (relabel) {
-            for (uint64_t i = 0; i < owner.ne_; ++i) tcol[i] = rank[tcol[i]];
-        }
+        transpose_csr(nv, owner.ne_, row, col, relabel ? unrank.data() : nullptr, trow, tcol);
     }
     sg_config rc = owner.cfg_;
     rc.flags &= SG_FLAG_HOST_EDGES;  // no timing, graphs or deferral of its own
@@ -2404,9 +2495,8 @@ static std::unique_ptr<GraphStore> make_in_store(Engine &owner, const uint64_t *
         in->sync();  // the host vectors die with this call
     }
     in->mirror_extra_bytes_ = mirror_extra_bytes;
-    in->want_tail_ = tail;
-    in->refresh_tiles();
-    in->refresh_mirror();
+    in->want_plan_ = plan;
+    in->refresh();
     return in;
 }
 
@@ -2511,7 +2601,7 @@ struct TravProgram {
             // round R's frontier bitmap starts empty (it last served round R - 2)
             const uint64_t words = ((uint64_t)e.nv_ + 31) / 32;
             e.round_launch(k_fill_u32, dim3(grid_for(words, 256, 2048)), dim3(256), fb[R & 1], words, 0u);
-            e.launch_pass(io, VCombinePull<Op>{op, value, buffer, PullTake{fb[R & 1], pv, nullptr}},
+            e.launch_pass(io, VCombinePull<Op>{op, value, buffer, PullTake{fb[R & 1], pv}},
                           ERelax<Op>{op, buffer, e.stamp_, R + 1, e.cfg_.weight_mode, e.cfg_.weight_seed}, do_time);
             // the pull kernel returns at once unless the round is dense (device flag)
             const uint64_t nt = pull_in->ntiles();

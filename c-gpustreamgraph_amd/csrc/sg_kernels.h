@@ -57,10 +57,6 @@ struct GraphView {
     // walks and updates use col. mlive = 0: none.
     const uint32_t *mirror;
     uint64_t mlive;
-    // Gap-free packed copy of the live edges [mlive, E) in pinned host memory
-    // (id k - mlive = edge k), read by the tile sweeps instead of col's gappy
-    // slots; null: none.
-    const uint32_t *tail;
     uint32_t mbits;  // bits per packed id (32: plain words)
 };
 
@@ -134,23 +130,69 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     const uint32_t l = lane_id();
     return l ? (~0ull >> (64 - l)) : 0ull;
 }
+// Lane moves on the VALU (DPP): lane i takes x of another lane of its row of 16
+// (row_shr) or of an earlier row's last lane (row_bcast); lanes without a
+// source, or outside kRowMask's rows, take `old`. A shuffle goes through the
+// LDS crossbar instead. Every lane of the wave must be active.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t dpp_mov(uint32_t old, uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, kCtrl, kRowMask, 0xf, false);
+}
+constexpr int kDppRowShr = 0x110, kDppWaveShr1 = 0x138, kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+// x of the previous lane (lane 0: 0)
+__device__ __forceinline__ uint32_t wave_shr1(uint32_t x) { return dpp_mov<kDppWaveShr1, 0xf>(0u, x); }
+// Six steps of an inclusive scan: step(shift lanes within a row, then across rows).
+#define SG_DPP_SCAN(STEP)      \
+    STEP(kDppRowShr + 1, 0xf)  \
+    STEP(kDppRowShr + 2, 0xf)  \
+    STEP(kDppRowShr + 4, 0xf)  \
+    STEP(kDppRowShr + 8, 0xf)  \
+    STEP(kDppBcast15, 0xa)     \
+    STEP(kDppBcast31, 0xc)
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-    const uint32_t lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, kWave);
-        if (lane >= (uint32_t)d) x += y;
-    }
+#define SG_STEP(C, M) x += dpp_mov<C, M>(0u, x);
+    SG_DPP_SCAN(SG_STEP)
+#undef SG_STEP
     return x;
 }
 __device__ __forceinline__ unsigned long long wave_incl_scan(unsigned long long x) {
-    const uint32_t lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const unsigned long long y = __shfl_up(x, d, kWave);
-        if (lane >= (uint32_t)d) x += y;
-    }
+#define SG_STEP(C, M)                                                                                   \
+    x += ((unsigned long long)dpp_mov<C, M>(0u, (uint32_t)(x >> 32)) << 32) | dpp_mov<C, M>(0u, (uint32_t)x);
+    SG_DPP_SCAN(SG_STEP)
+#undef SG_STEP
     return x;
+}
+__device__ __forceinline__ uint32_t wave_max_scan(uint32_t x) {
+#define SG_STEP(C, M) x = max(x, dpp_mov<C, M>(0u, x));
+    SG_DPP_SCAN(SG_STEP)
+#undef SG_STEP
+    return x;
+}
+// Inclusive segmented sum: lanes with head != 0 start a segment.
+__device__ __forceinline__ float wave_seg_scan(float x, uint32_t head) {
+#define SG_STEP(C, M)                                                    \
+    {                                                                    \
+        const float y = __uint_as_float(dpp_mov<C, M>(0u, __float_as_uint(x))); \
+        const uint32_t h = dpp_mov<C, M>(0u, head);                      \
+        x = head ? x : x + y;                                            \
+        head |= h;                                                       \
+    }
+    SG_DPP_SCAN(SG_STEP)
+#undef SG_STEP
+    return x;
+}
+// Sum over the wave (in every lane).
+__device__ __forceinline__ float wave_sum_f32(float x) {
+#define SG_STEP(C, M) x += __uint_as_float(dpp_mov<C, M>(0u, __float_as_uint(x)));
+    SG_DPP_SCAN(SG_STEP)
+#undef SG_STEP
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), kWave - 1));
+}
+// LDS of one wave: what its lanes stored before is read by the loads after
+// (the hardware keeps a wave's LDS operations in order; the compiler must too).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 // Wave-aggregated append: one atomicAdd per wave. Every active lane of the
 // wave must call it (pred may differ per lane).
@@ -298,14 +340,13 @@ struct WaveStats {
     unsigned long long edges = 0, verts = 0, hedges = 0, cedges = 0;
 };
 
-// LDS of the light tier (per block).
-struct LightShared {
-    uint64_t start[kWavesPerBlock][kWave];
-    uint32_t excl[kWavesPerBlock][kWave];
-    uint32_t src[kWavesPerBlock][kWave];
-    uint32_t push[kWavesPerBlock][kWave];
-    uint32_t out[kWavesPerBlock][kOutStage];
-    unsigned long long red[kWavesPerBlock][4];
+// LDS of the light tier (per wave).
+struct LightWave {
+    uint64_t start[kWave];
+    uint32_t excl[kWave];
+    uint32_t src[kWave];
+    uint32_t push[kWave];
+    uint32_t out[kOutStage];
 };
 
 // Owner of edge k among the 64 staged lists: the largest j with excl[j] <= k
@@ -364,9 +405,9 @@ __device__ __forceinline__ uint32_t light_width(uint32_t n, uint64_t nwaves) {
 // budget + heavy_deg edges per batch.
 template <class VFn, class EFn>
 __device__ __forceinline__ void light_body(const GraphView &g, const PassIO &io, const VFn &vfn, const EFn &efn,
-                                           uint32_t n, uint64_t gwave, uint64_t nwaves, LightShared &sh, OutStage &st,
+                                           uint32_t n, uint64_t gwave, uint64_t nwaves, LightWave &sh, OutStage &st,
                                            WaveStats &ws) {
-    const uint32_t w = threadIdx.x / kWave, lane = lane_id();
+    const uint32_t lane = lane_id();
     // frontier vertices per wave batch: 64 when the frontier fills every wave,
     // fewer (a power of two, down to 1) when it is small, so that its lists
     // spread over all waves instead of a few waves walking 64 lists each
@@ -380,7 +421,14 @@ __device__ __forceinline__ void light_body(const GraphView &g, const PassIO &io,
         uint32_t u = 0, d = 0, push = 0;
         uint64_t start = 0;
         bool self = false, sched = false;
-        if (lane < per && idx < n) {
+        if constexpr (VFn::kItems) {  // the functor names the vertex of item idx and its push
+            if (lane < per && idx < n) sched = vfn.item((uint32_t)idx, u, push);
+            if (__ballot(sched) == 0) continue;
+            if (sched) {
+                d = g.deg[u];
+                start = list_start(g, u);
+            }
+        } else if (lane < per && idx < n) {
             u = io.in_list ? io.in_list[idx] : io.range_lo + (uint32_t)idx;
             const uint32_t du = g.deg[u];
             sched = vfn(u, du, push, self);
@@ -428,12 +476,12 @@ __device__ __forceinline__ void light_body(const GraphView &g, const PassIO &io,
         if (heavy) d = 0;
         const uint32_t incl = wave_incl_scan(d);
         const uint32_t total = __shfl(incl, kWave - 1, kWave);
-        sh.start[w][lane] = start;
-        sh.excl[w][lane] = incl - d;
-        sh.src[w][lane] = u;
-        sh.push[w][lane] = push;
+        sh.start[lane] = start;
+        sh.excl[lane] = incl - d;
+        sh.src[lane] = u;
+        sh.push[lane] = push;
         __builtin_amdgcn_wave_barrier();
-        walk_staged(g, io, efn, total, sh.excl[w], sh.start[w], sh.src[w], sh.push[w], st);
+        walk_staged(g, io, efn, total, sh.excl, sh.start, sh.src, sh.push, st);
         ws.edges += total;
         if (g.coff) ws.cedges += wave_sum_u64(start >= g.cap ? d : 0u);
         __builtin_amdgcn_wave_barrier();
@@ -471,19 +519,20 @@ __device__ __forceinline__ void heavy_body(const GraphView &g, const PassIO &io,
 }
 
 // One atomic per block for the pass counters.
-__device__ __forceinline__ void block_stats(const WaveStats &ws, LightShared &sh, unsigned long long *stats) {
+template <int kWaves>
+__device__ __forceinline__ void block_stats(const WaveStats &ws, unsigned long long (*red)[4], unsigned long long *stats) {
     const uint32_t w = threadIdx.x / kWave;
     const unsigned long long v = wave_sum_u64(ws.verts);
     if (lane_id() == 0) {
-        sh.red[w][0] = ws.edges;
-        sh.red[w][1] = v;
-        sh.red[w][2] = ws.hedges;
-        sh.red[w][3] = ws.cedges;  // lane 0 holds the wave's cached-edge total
+        red[w][0] = ws.edges;
+        red[w][1] = v;
+        red[w][2] = ws.hedges;
+        red[w][3] = ws.cedges;  // lane 0 holds the wave's cached-edge total
     }
     __syncthreads();
     if (threadIdx.x < 4) {
         unsigned long long t = 0;
-        for (int i = 0; i < kWavesPerBlock; ++i) t += sh.red[i][threadIdx.x];
+        for (int i = 0; i < kWaves; ++i) t += red[i][threadIdx.x];
         // [0] edges, [1] vertices, [2] spilled-chunk edges, [5] edges read from the cache
         const int slot = threadIdx.x == 3 ? 5 : (int)threadIdx.x;
         if (t) atomicAdd(stats + slot, t);
@@ -497,7 +546,8 @@ __device__ __forceinline__ void block_stats(const WaveStats &ws, LightShared &sh
 // and whatever they activate joins round R+1.
 template <class VFn, class EFn>
 __global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vfn, EFn efn) {
-    __shared__ LightShared sh;
+    __shared__ LightWave s_wave[kWavesPerBlock];
+    __shared__ unsigned long long s_red[kWavesPerBlock][4];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (io.zero_cnt) *io.zero_cnt = 0;
         if (io.heavy_zero) *io.heavy_zero = 0;
@@ -513,13 +563,13 @@ __global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vf
     const uint32_t nh = io.hin ? min(*io.hin_cnt, io.heavy_cap) : 0;
     const uint32_t w = threadIdx.x / kWave;
     const uint64_t gwave = (uint64_t)blockIdx.x * kWavesPerBlock + w, nwaves = (uint64_t)gridDim.x * kWavesPerBlock;
-    OutStage st{sh.out[w], 0};
+    OutStage st{s_wave[w].out, 0};
     WaveStats ws;
-    light_body(g, io, vfn, efn, n, gwave, nwaves, sh, st, ws);
+    light_body(g, io, vfn, efn, n, gwave, nwaves, s_wave[w], st, ws);
     heavy_body(g, io, efn, nh, gwave, nwaves, st, ws);
     stage_flush(st, io);
     stage_count_flush(st, io);
-    block_stats(ws, sh, io.stats);
+    block_stats<kWavesPerBlock>(ws, s_red, io.stats);
 }
 
 // ---- vertex functors ---------------------------------------------------------
@@ -530,6 +580,7 @@ __global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vf
 template <class Op>
 struct VCombine {
     static constexpr bool kDense = false;
+    static constexpr bool kItems = false;
     Op op;
     typename Op::value_t *value;
     typename Op::buffer_t *buffer;
@@ -546,6 +597,7 @@ struct VCombine {
 template <class Op>
 struct VAmend {
     static constexpr bool kDense = false;
+    static constexpr bool kItems = false;
     Op op;
     int type;
     typename Op::value_t *value;
@@ -566,6 +618,7 @@ struct VAmend {
 template <class Op>
 struct VSweep {
     static constexpr bool kDense = false;
+    static constexpr bool kItems = false;
     Op op;
     typename Op::value_t *value;
     typename Op::buffer_t *buffer;
@@ -586,6 +639,7 @@ struct VSweep {
 // Invalidation propagation: expand every invalidated vertex.
 struct VAll {
     static constexpr bool kDense = false;
+    static constexpr bool kItems = false;
     __device__ bool operator()(uint32_t u, uint32_t, uint32_t &push, bool &self) const {
         self = false;
         push = u;

@@ -649,12 +649,8 @@ __global__ void __launch_bounds__(kSweepBlock) k_msweep(GraphView g, const unsig
     uint32_t n_edges = 0;
     const uint32_t cs = ms.cshift;
     load_filter(s_filter, ms.coarse, coarse_words(g.nv, cs));
-    TilePipe tp;
-    tp.tend = min_u64(ntiles, tiles.cap - 1);
-    tp.nw = (unsigned long long)gridDim.x * kSweepWaves;
-    tp.t = (unsigned long long)blockIdx.x * kSweepWaves + w;
-    tp.start(g, dpre, tiles);
-    while (tp.t < tp.tend) {
+    TilePipe tp(TileWalk(0, min_u64(ntiles, tiles.cap - 1), kSweepWaves), g, dpre, tiles);
+    while (tp.more) {
         uint32_t vv[kSweepPerLane];
         const uint32_t v0 = tp.h.v0;
         sweep_tile(g, dpre, tp.h, tp.pre, g.col, 0, 0, g.nv, sh, vv, n_edges);

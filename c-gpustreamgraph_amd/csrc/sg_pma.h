@@ -528,14 +528,18 @@ constexpr uint32_t kSweepOutStage = 128;
 constexpr int kSweepWaves = 4;                    // waves per block of the sweep kernels
 constexpr int kSweepBlock = kSweepWaves * kWave;
 
-struct SweepWave {
+// A tile's LDS: owners (16-byte groups of 8 positions) and slot bases; base[]
+// is dead once the tile's edges are loaded.
+struct alignas(16) SweepTileLds {
     uint16_t own[kSweepTile];
-    int32_t base[kSweepTile + 1];
+    int32_t base[kSweepTile + 4];
+};
+struct SweepWave : SweepTileLds {
     uint32_t out[kSweepOutStage];
 };
-// base[] also holds a tile's packed words (ids of at most 31 bits, 16-byte groups)
-static_assert(kSweepTile + 1 >= (kSweepTile * 31 + 31) / 32 + 8, "base[] holds a tile's packed words");
-
+// 16-byte LDS accesses to arrays of another type
+typedef uint32_t lds_u32x4 __attribute__((ext_vector_type(4), may_alias));
+typedef float lds_f32x4 __attribute__((ext_vector_type(4), may_alias));
 // Bounds of tile t, loaded by lanes 0-3 with vector loads so that the load
 // stays in flight while the wave works on the current tile: lane 0 v[t],
 // lane 1 v[t + 1], lane 2 e[t], lane 3 e[t + 1].
@@ -589,22 +593,18 @@ __device__ __forceinline__ TilePre tile_pre(const GraphView &g, const unsigned l
     return p;
 }
 
-// colp / slot_lo: where slot s of the tile's sources is read (colp[s - slot_lo]:
-// the edge array itself, or one streamed segment of it); only sources in
-// [src_lo, src_hi) are walked. pre = tile_pre(h, lane). vv[j] = target at tile
-// position j * 64 + lane (kGap when none); the owner index of a position stays
-// in sh.own.
-template <bool kStagePacked = false>
-__device__ __forceinline__ void sweep_tile(const GraphView &g, const unsigned long long *dpre, const TileHead &h,
-                                           const TilePre &pre, const uint32_t *colp, uint64_t slot_lo, uint32_t src_lo,
-                                           uint32_t src_hi, SweepWave &sh, uint32_t vv[kSweepPerLane],
-                                           uint32_t &n_edges) {
+// Owners and slot bases of the tile's positions into sh; pre = tile_pre(h,
+// lane). Returns the owners of the lane's positions [8 * lane, 8 * lane + 8)
+// as 16-bit pairs; wide: the slot range does not fit base[].
+__device__ __forceinline__ lds_u32x4 sweep_owners(const GraphView &g, const unsigned long long *dpre, const TileHead &h,
+                                                  const TilePre &pre, SweepTileLds &sh, bool &wide) {
     const uint32_t lane = lane_id();
     const uint32_t v0 = h.v0, span = h.span, ne = h.ne;
     const unsigned long long e0 = h.e0;
-#pragma unroll
-    for (int j = 0; j < kSweepPerLane; ++j) sh.own[j * kWave + lane] = 0;
-    __builtin_amdgcn_wave_barrier();
+    // lane k owns positions [k * 8, k * 8 + 8): one 16-byte group of own[]
+    lds_u32x4 *const own8 = reinterpret_cast<lds_u32x4 *>(sh.own) + lane;
+    *own8 = lds_u32x4{0u, 0u, 0u, 0u};
+    wave_lds_sync();
     const uint64_t off0 = read_lane_u64(pre.ov, 0);
     bool far = false;
     for (uint32_t i0 = 0; i0 <= span; i0 += kWave) {
@@ -619,85 +619,40 @@ __device__ __forceinline__ void sweep_tile(const GraphView &g, const unsigned lo
             if (b > p.a && p.a >= e0 && p.a < e0 + ne) sh.own[p.a - e0] = (uint16_t)i;
         }
     }
-    const bool wide = __ballot(far) != 0;
-    __builtin_amdgcn_wave_barrier();
-    // forward fill of the owners: lane k holds positions [k * P, k * P + P)
-    uint32_t own[kSweepPerLane];
+    wide = __ballot(far) != 0;
+    wave_lds_sync();
+    // forward fill of the owners: the running maximum in the lane's group, on
+    // top of the largest owner before it (a scan over the lanes)
+    lds_u32x4 o = *own8;
     uint32_t m = 0;
 #pragma unroll
-    for (int j = 0; j < kSweepPerLane; ++j) {
-        own[j] = sh.own[lane * kSweepPerLane + j];
-        m = max(m, own[j]);
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t lo = max(m, o[j] & 0xFFFFu), hi = max(lo, o[j] >> 16);
+        o[j] = lo | (hi << 16);
+        m = hi;
     }
-    uint32_t x = m;
+    const uint32_t prev = wave_shr1(wave_max_scan(m));
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, kWave);
-        if (lane >= (uint32_t)d) x = max(x, y);
-    }
-    uint32_t prev = __shfl_up(x, 1, kWave);
-    if (lane == 0) prev = 0;
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int j = 0; j < kSweepPerLane; ++j) {
-        prev = max(prev, own[j]);
-        sh.own[lane * kSweepPerLane + j] = (uint16_t)prev;
-    }
-    __builtin_amdgcn_wave_barrier();
-    // kStagePacked: a tile whose edges all lie in one packed copy (the HBM
-    // mirror or the host tail) loads the words it spans with at most two
-    // 16-byte loads per lane into LDS (base[] is not needed for such a tile)
-    // and unpacks its ids there: each word crosses the bus once, where reading
-    // id by id loads two overlapping words per id. The copies keep 4 words of
-    // slack past their last id for the aligned loads. Kernels that seldom
-    // read a copy leave it off (it costs registers).
-    const uint32_t b = g.mbits;
-    const bool in_mirror = g.mlive && e0 + ne <= g.mlive;
-    const bool packed_tile = kStagePacked && b < 32 && ne && (in_mirror || (g.tail && e0 >= g.mlive));
-    uint32_t *const lw = reinterpret_cast<uint32_t *>(sh.base);
-    uint32_t bit0 = 0;  // bit of the tile's first id in lw
-    if (packed_tile) {
-        const uint32_t *cp = in_mirror ? g.mirror : g.tail;
-        const unsigned long long i0 = in_mirror ? e0 : e0 - g.mlive;
-        const unsigned long long wa = ((i0 * b) >> 5) & ~3ull;
-        // words [wa, end]: end is the word after the one holding the last bit (<= 501 words)
-        const uint32_t nw = (uint32_t)(((i0 + ne) * b + 31) / 32 + 1 - wa);
-        bit0 = (uint32_t)(i0 * b - wa * 32);
-        const uint32_t q0 = lane * 4, q1 = q0 + kWave * 4;
-        uint4 x0 = make_uint4(0u, 0u, 0u, 0u), x1 = x0;
-        if (q0 < nw) x0 = *reinterpret_cast<const uint4 *>(cp + wa + q0);
-        if (q1 < nw) x1 = *reinterpret_cast<const uint4 *>(cp + wa + q1);
-        if (q0 < nw) {
-            lw[q0] = x0.x;
-            lw[q0 + 1] = x0.y;
-            lw[q0 + 2] = x0.z;
-            lw[q0 + 3] = x0.w;
-        }
-        if (q1 < nw) {
-            lw[q1] = x1.x;
-            lw[q1 + 1] = x1.y;
-            lw[q1 + 2] = x1.z;
-            lw[q1 + 3] = x1.w;
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (packed_tile) {
-#pragma unroll
-        for (int j = 0; j < kSweepPerLane; ++j) {
-            const uint32_t p = j * kWave + lane;
-            vv[j] = kGap;
-            if (p < ne) {
-                const uint32_t src = v0 + sh.own[p];
-                if (src >= src_lo && src < src_hi) {
-                    ++n_edges;
-                    const uint32_t bit = bit0 + p * b;
-                    const uint64_t x = ((uint64_t)lw[(bit >> 5) + 1] << 32) | lw[bit >> 5];
-                    vv[j] = (uint32_t)(x >> (bit & 31u)) & ((1u << b) - 1u);
-                }
-            }
-        }
-        return;
-    }
+    for (int j = 0; j < 4; ++j) o[j] = max(o[j] & 0xFFFFu, prev) | (max(o[j] >> 16, prev) << 16);
+    *own8 = o;
+    wave_lds_sync();
+    return o;
+}
+
+// colp / slot_lo: where slot s of the tile's sources is read (colp[s - slot_lo]:
+// the edge array itself, or one streamed segment of it); only sources in
+// [src_lo, src_hi) are walked. vv[j] = target at tile position j * 64 + lane
+// (kGap when none); the owner index of a position stays in sh.own.
+__device__ __forceinline__ void sweep_tile(const GraphView &g, const unsigned long long *dpre, const TileHead &h,
+                                           const TilePre &pre, const uint32_t *colp, uint64_t slot_lo, uint32_t src_lo,
+                                           uint32_t src_hi, SweepTileLds &sh, uint32_t vv[kSweepPerLane],
+                                           uint32_t &n_edges) {
+    const uint32_t lane = lane_id();
+    const uint32_t v0 = h.v0, ne = h.ne, b = g.mbits;
+    const unsigned long long e0 = h.e0;
+    const uint64_t off0 = read_lane_u64(pre.ov, 0);
+    bool wide;
+    sweep_owners(g, dpre, h, pre, sh, wide);
 #pragma unroll
     for (int j = 0; j < kSweepPerLane; ++j) {
         const uint32_t p = j * kWave + lane;
@@ -710,38 +665,70 @@ __device__ __forceinline__ void sweep_tile(const GraphView &g, const unsigned lo
                 const uint64_t slot = !wide ? off0 + (uint64_t)((long long)sh.base[o] + (long long)p)
                                             : g.off[src] + (e0 + p - dpre[src]);
                 const unsigned long long k = e0 + p;
-                vv[j] = k < g.mlive ? packed_at(g.mirror, k, b)
-                        : g.tail    ? packed_at(g.tail, k - g.mlive, b)
-                                    : colp[slot - slot_lo];
+                vv[j] = k < g.mlive ? packed_at(g.mirror, k, b) : colp[slot - slot_lo];
             }
         }
     }
 }
 
-// Tile pipeline of one wave over tiles t, t + nw, ... < tend: the bounds are
-// loaded two tiles ahead and the first sources' words one tile ahead, so they
-// are in flight while the current tile's edges are loaded and tested.
+// The tiles of one wave. Blocks go to the 8 XCDs in turn, and each XCD has its
+// own L2: the tiles [t0, tend) are dealt out in runs of kTileRun, run r to the
+// waves of XCD r mod 8, so that the lines neighbouring tiles share (per-vertex
+// words; a pull's scattered pushes) are completed in one L2 instead of being
+// fetched, and written back in parts, by several.
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kTileRun = 64;
+struct TileWalk {
+    unsigned long long t0, tend;
+    unsigned long long k;      // index among the tiles of this wave's group
+    uint32_t group, ngroups, step;
+    __device__ __forceinline__ TileWalk(unsigned long long lo, unsigned long long hi, uint32_t waves)
+        : t0(lo), tend(hi) {
+        ngroups = gridDim.x % kXcds == 0 ? kXcds : 1u;
+        group = blockIdx.x % ngroups;
+        const uint32_t blocks = gridDim.x / ngroups;
+        // consecutive waves of a group on different CUs
+        k = (unsigned long long)(threadIdx.x / kWave) * blocks + blockIdx.x / ngroups;
+        step = blocks * waves;
+    }
+    __device__ __forceinline__ unsigned long long at(unsigned long long i) const {
+        return t0 + ((i / kTileRun) * ngroups + group) * kTileRun + i % kTileRun;
+    }
+    __device__ __forceinline__ unsigned long long tile() const { return at(k); }
+    __device__ __forceinline__ unsigned long long ahead(uint32_t n) const { return at(k + (unsigned long long)n * step); }
+};
+
+// Tile pipeline of one wave: the bounds are loaded two tiles ahead and the
+// first sources' words one tile ahead, so they are in flight while the current
+// tile's edges are loaded and tested.
 struct TilePipe {
-    unsigned long long t, nw, tend;
-    unsigned long long raw_next;  // tile_head_load(t + nw)
-    TileHead h;                   // tile t
-    TilePre pre;                  // tile_pre of tile t
-    __device__ __forceinline__ void start(const GraphView &g, const unsigned long long *dpre, const SweepTiles &tiles) {
-        raw_next = t + nw < tend ? tile_head_load(tiles, t + nw) : 0;
-        if (t < tend) {
+    TileWalk w;
+    unsigned long long raw_next;  // tile_head_load(next tile)
+    TileHead h;                   // this tile
+    TilePre pre;                  // tile_pre of this tile
+    bool more;                    // this tile exists
+    __device__ __forceinline__ TilePipe(const TileWalk &walk, const GraphView &g, const unsigned long long *dpre,
+                                        const SweepTiles &tiles)
+        : w(walk) {
+        const unsigned long long t = w.tile(), t1 = w.ahead(1);
+        more = t < w.tend;
+        raw_next = t1 < w.tend ? tile_head_load(tiles, t1) : 0;
+        if (more) {
             h = tile_head(tile_head_load(tiles, t));
             pre = tile_pre(g, dpre, h, lane_id());
         }
     }
     // after the current tile's edges are loaded: start the next tile's loads
     __device__ __forceinline__ void advance(const GraphView &g, const unsigned long long *dpre, const SweepTiles &tiles) {
-        const unsigned long long raw2 = t + 2 * nw < tend ? tile_head_load(tiles, t + 2 * nw) : 0;
-        if (t + nw < tend) {
+        const unsigned long long t2 = w.ahead(2);
+        const unsigned long long raw2 = t2 < w.tend ? tile_head_load(tiles, t2) : 0;
+        more = w.ahead(1) < w.tend;
+        if (more) {
             h = tile_head(raw_next);
             pre = tile_pre(g, dpre, h, lane_id());
         }
         raw_next = raw2;
-        t += nw;
+        w.k += w.step;
     }
 };
 
@@ -782,12 +769,8 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_edges(GraphView g, const 
     uint32_t n_edges = 0;
     const uint32_t cs = efn.cshift;
     load_filter(s_filter, efn.coarse, coarse_words(g.nv, cs));
-    TilePipe tp;
-    tp.tend = min_u64(min_u64(t_end, ntiles), tiles.cap - 1);
-    tp.nw = (unsigned long long)gridDim.x * kSweepWaves;
-    tp.t = t_begin + (unsigned long long)blockIdx.x * kSweepWaves + w;
-    tp.start(g, dpre, tiles);
-    while (tp.t < tp.tend) {
+    TilePipe tp(TileWalk(t_begin, min_u64(min_u64(t_end, ntiles), tiles.cap - 1), kSweepWaves), g, dpre, tiles);
+    while (tp.more) {
         uint32_t vv[kSweepPerLane];
         const uint32_t v0 = tp.h.v0;
         sweep_tile(g, dpre, tp.h, tp.pre, colp, slot_lo, src_lo, src_hi, sh, vv, n_edges);
