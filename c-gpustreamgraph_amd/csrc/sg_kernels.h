@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "sg_operators.h"
 #include "../host/sg_rng.h"
 
@@ -79,7 +81,8 @@ __device__ __forceinline__ uint64_t list_start(const GraphView &g, uint32_t u) {
     return g.off[u];
 }
 __device__ __forceinline__ uint32_t edge_at(const GraphView &g, uint64_t s) {
-    return s < g.cap ? g.col[s] : g.ccol[s - g.cap];
+    const uint32_t *const p = s < g.cap ? g.col + s : g.ccol + (s - g.cap);
+    return *p;
 }
 // Activation count of the cache's hotness window (non-atomic and saturating,
 // like the reference's hotness[0]++ in RelaxCTADB, sync_push_dd.cuh:196-230).
@@ -327,6 +330,65 @@ __device__ __forceinline__ void stage_push(bool pred, uint32_t item, OutStage &s
     st.n += c;
 }
 
+// item[j] of the lanes with pred[j], N per lane.
+template <int N>
+__device__ __forceinline__ void stage_push_n(const bool (&pred)[N], const uint32_t (&item)[N], OutStage &st,
+                                             const PassIO &io) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) c += pred[j] ? 1u : 0u;
+    if (__ballot(c != 0) == 0) return;
+    if (io.fdeg) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (pred[j]) st.fedges += io.fdeg[item[j]];
+    }
+    const uint32_t incl = wave_incl_scan(c);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    if (st.n + total > st.cap) stage_flush(st, io);
+    if (total > st.cap) {  // more than a slice at once
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const uint64_t m = __ballot(pred[j]);
+            const uint32_t n = (uint32_t)__popcll(m);
+            if (st.n + n > st.cap) stage_flush(st, io);
+            if (pred[j]) st.buf[st.n + (uint32_t)__popcll(m & lanemask_lt())] = item[j];
+            st.n += n;
+        }
+        return;
+    }
+    uint32_t at = st.n + incl - c;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (pred[j]) st.buf[at++] = item[j];
+    st.n += total;
+}
+
+// The waves of a block append what they still hold with one atomic (every
+// thread of a block of kWaves waves; s_n: kWaves + 1 words).
+template <int kWaves>
+__device__ __forceinline__ void block_flush(OutStage &st, const PassIO &io, uint32_t *s_n) {
+    const uint32_t w = threadIdx.x / kWave;
+    if (lane_id() == 0) s_n[w] = st.n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int i = 0; i < kWaves; ++i) {
+            const uint32_t c = s_n[i];
+            s_n[i] = t;
+            t += c;
+        }
+        s_n[kWaves] = t ? atomicAdd(io.out_cnt, t) : 0u;
+    }
+    __syncthreads();
+    const uint32_t base = s_n[kWaves] + s_n[w];
+    for (uint32_t i = lane_id(); i < st.n; i += kWave) {
+        if (base + i < io.out_cap) io.out_list[base + i] = st.buf[i];
+        else atomicOr(io.stats + 3, 1ull);
+    }
+    st.n = 0;
+}
+
 // One atomic per wave: the out-edges of what the wave appended (io.ecnt_out).
 __device__ __forceinline__ void stage_count_flush(OutStage &st, const PassIO &io) {
     if (!io.ecnt_out) return;
@@ -340,53 +402,86 @@ struct WaveStats {
     unsigned long long edges = 0, verts = 0, hedges = 0, cedges = 0;
 };
 
-// LDS of the light tier (per wave).
-struct LightWave {
-    uint64_t start[kWave];
-    uint32_t excl[kWave];
-    uint32_t src[kWave];
-    uint32_t push[kWave];
+// LDS of the light tier (per wave). own: list of each of the kIlp * 64 edges
+// of a step.
+struct StagedList {
+    uint64_t base;  // slot of edge k of the staged union: base + k
+    uint32_t src, push;
+};
+struct alignas(16) LightWave {
+    StagedList list[kWave];
+    uint8_t own[kIlp * kWave];
     uint32_t out[kOutStage];
 };
+// LDS accesses of another width than the array's
+typedef uint32_t lds_u32x2 __attribute__((ext_vector_type(2), may_alias));
 
-// Owner of edge k among the 64 staged lists: the largest j with excl[j] <= k
-// (six unrolled LDS probes, so the kIlp searches of a lane interleave).
-__device__ __forceinline__ uint32_t staged_owner(const uint32_t *excl, uint32_t k) {
-    uint32_t lo = 0;
+// One step of edges: all their updates, then what they activate. Nothing
+// waits between the edges of a lane: the loads, the destination updates and
+// the stamp exchanges of a step are each in flight together.
+template <class EFn>
+__device__ __forceinline__ void apply_edges(const PassIO &io, const EFn &efn, const uint32_t (&src)[kIlp],
+                                            const uint32_t (&v)[kIlp], const uint32_t (&push)[kIlp], OutStage &st) {
+    uint64_t peek[kIlp];
 #pragma unroll
-    for (uint32_t step = kWave / 2; step > 0; step >>= 1)
-        if (excl[lo + step] <= k) lo += step;
-    return lo;
+    for (int j = 0; j < kIlp; ++j) peek[j] = efn.load(v[j] != kGap ? v[j] : 0u);
+    bool enq[kIlp];
+    efn.template apply_n<kIlp>(src, v, push, peek, enq);
+    if constexpr (EFn::kAppendSource) stage_push_n<kIlp>(enq, src, st, io);
+    else stage_push_n<kIlp>(enq, v, st, io);
 }
 
-// Edge loop of one wave over `total` edges whose owners are staged in LDS,
-// kIlp edges per lane per step: all target ids are loaded, then all functor
-// peeks, then the updates.
+// Edge loop of one wave over the union of its lanes' lists: lane i's list has
+// d edges from slot start, the union's edges [excl, excl + d); total edges.
+// kIlp edges per lane per step. The list of each edge of a step comes from
+// marks at the list starts, filled forward by a maximum scan (a binary search
+// per edge is six dependent LDS reads, and was half of a step).
 template <class EFn>
 __device__ __forceinline__ void walk_staged(const GraphView &g, const PassIO &io, const EFn &efn, uint32_t total,
-                                            const uint32_t *s_excl, const uint64_t *s_start, const uint32_t *s_src,
-                                            const uint32_t *s_push, OutStage &st) {
+                                            uint32_t excl, uint32_t d, uint64_t start, uint32_t src_l, uint32_t push_l,
+                                            LightWave &sh, OutStage &st) {
+    if (total == 0) return;
     const uint32_t lane = lane_id();
+    sh.list[lane] = StagedList{start - excl, src_l, push_l};
+    lds_u32x2 *const own8 = reinterpret_cast<lds_u32x2 *>(sh.own) + lane;
     for (uint32_t k0 = 0; k0 < total; k0 += kIlp * kWave) {
+        *own8 = lds_u32x2{0u, 0u};
+        wave_lds_sync();
+        if (d && excl > k0 && excl - k0 < kIlp * kWave) sh.own[excl - k0] = (uint8_t)lane;
+        // the list open at k0: the last non-empty one that starts at or before it
+        const uint32_t open = 63u - (uint32_t)__builtin_clzll(__ballot(d != 0 && excl <= k0) | 1ull);
+        wave_lds_sync();
+        lds_u32x2 o = *own8;
+        uint32_t m = 0;
+        uint32_t b[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            m = max(m, (o[j / 4] >> (8 * (j & 3))) & 0xFFu);
+            b[j] = m;
+        }
+        const uint32_t before = max(wave_shr1(wave_max_scan(m)), open);
+        o = lds_u32x2{0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j / 4] |= max(b[j], before) << (8 * (j & 3));
+        *own8 = o;
+        wave_lds_sync();
         uint32_t v[kIlp], src[kIlp], push[kIlp];
-        uint64_t peek[kIlp];
-        bool act[kIlp];
+        uint64_t slot[kIlp];
 #pragma unroll
         for (int j = 0; j < kIlp; ++j) {
-            const uint32_t k = k0 + j * kWave + lane;
-            act[j] = k < total;
-            const uint32_t o = staged_owner(s_excl, act[j] ? k : 0);
-            src[j] = s_src[o];
-            push[j] = s_push[o];
-            v[j] = act[j] ? edge_at(g, s_start[o] + (k - s_excl[o])) : kGap;
+            const uint32_t k = min(k0 + j * kWave + lane, total - 1);
+            const StagedList l = sh.list[sh.own[min(j * kWave + lane, total - 1 - k0)]];
+            src[j] = l.src;
+            push[j] = l.push;
+            slot[j] = l.base + k;
         }
 #pragma unroll
-        for (int j = 0; j < kIlp; ++j) peek[j] = (v[j] != kGap) ? efn.load(v[j]) : 0;
-        bool enq[kIlp];
+        for (int j = 0; j < kIlp; ++j) v[j] = edge_at(g, slot[j]);
 #pragma unroll
-        for (int j = 0; j < kIlp; ++j) enq[j] = v[j] != kGap && efn.apply(src[j], v[j], push[j], peek[j]);
-#pragma unroll
-        for (int j = 0; j < kIlp; ++j) stage_push(enq[j], EFn::kAppendSource ? src[j] : v[j], st, io);
+        for (int j = 0; j < kIlp; ++j)
+            if (k0 + j * kWave + lane >= total) v[j] = kGap;
+        wave_lds_sync();
+        apply_edges(io, efn, src, v, push, st);
     }
 }
 
@@ -476,12 +571,8 @@ __device__ __forceinline__ void light_body(const GraphView &g, const PassIO &io,
         if (heavy) d = 0;
         const uint32_t incl = wave_incl_scan(d);
         const uint32_t total = __shfl(incl, kWave - 1, kWave);
-        sh.start[lane] = start;
-        sh.excl[lane] = incl - d;
-        sh.src[lane] = u;
-        sh.push[lane] = push;
-        __builtin_amdgcn_wave_barrier();
-        walk_staged(g, io, efn, total, sh.excl, sh.start, sh.src, sh.push, st);
+        wave_lds_sync();
+        walk_staged(g, io, efn, total, incl - d, d, start, u, push, sh, st);
         ws.edges += total;
         if (g.coff) ws.cedges += wave_sum_u64(start >= g.cap ? d : 0u);
         __builtin_amdgcn_wave_barrier();
@@ -498,20 +589,17 @@ __device__ __forceinline__ void heavy_body(const GraphView &g, const PassIO &io,
         const uint64_t hstart = hd.start_len >> kLenBits;
         const uint32_t hlen = (uint32_t)(hd.start_len & ((1u << kLenBits) - 1)) + 1;
         for (uint32_t k0 = 0; k0 < hlen; k0 += kIlp * kWave) {
-            uint32_t v[kIlp];
-            uint64_t peek[kIlp];
-            bool enq[kIlp];
+            uint32_t v[kIlp], src[kIlp], push[kIlp];
 #pragma unroll
             for (int j = 0; j < kIlp; ++j) {
-                const uint32_t k = k0 + j * kWave + lane;
-                v[j] = k < hlen ? edge_at(g, hstart + k) : kGap;
+                src[j] = hd.u;
+                push[j] = hd.push;
+                v[j] = edge_at(g, hstart + min(k0 + j * kWave + lane, hlen - 1));
             }
 #pragma unroll
-            for (int j = 0; j < kIlp; ++j) peek[j] = v[j] != kGap ? efn.load(v[j]) : 0;
-#pragma unroll
-            for (int j = 0; j < kIlp; ++j) enq[j] = v[j] != kGap && efn.apply(hd.u, v[j], hd.push, peek[j]);
-#pragma unroll
-            for (int j = 0; j < kIlp; ++j) stage_push(enq[j], EFn::kAppendSource ? hd.u : v[j], st, io);
+            for (int j = 0; j < kIlp; ++j)
+                if (k0 + j * kWave + lane >= hlen) v[j] = kGap;
+            apply_edges(io, efn, src, v, push, st);
         }
         ws.hedges += hlen;
         if (hstart >= g.cap) ws.cedges += hlen;
@@ -548,6 +636,7 @@ template <class VFn, class EFn>
 __global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vfn, EFn efn) {
     __shared__ LightWave s_wave[kWavesPerBlock];
     __shared__ unsigned long long s_red[kWavesPerBlock][4];
+    __shared__ uint32_t s_n[kWavesPerBlock + 1];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (io.zero_cnt) *io.zero_cnt = 0;
         if (io.heavy_zero) *io.heavy_zero = 0;
@@ -567,7 +656,7 @@ __global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vf
     WaveStats ws;
     light_body(g, io, vfn, efn, n, gwave, nwaves, s_wave[w], st, ws);
     heavy_body(g, io, efn, nh, gwave, nwaves, st, ws);
-    stage_flush(st, io);
+    block_flush<kWavesPerBlock>(st, io, s_n);
     stage_count_flush(st, io);
     block_stats<kWavesPerBlock>(ws, s_red, io.stats);
 }
@@ -648,9 +737,35 @@ struct VAll {
 };
 
 // ---- edge functors -------------------------------------------------------------
-// load(v) peeks the destination state (issued for kIlp edges at once);
-// apply(u, v, push, peek) updates it and returns whether v joins the output
-// (u, the walked list's owner, when kAppendSource: a pull over in-lists).
+// load(v) peeks the destination state; apply_n(src, v, push, peek, enq) updates
+// N destinations of the lane (v[j] = kGap: none) and says which join the output
+// (src[j], the walked list's owner, when kAppendSource: a pull over in-lists).
+
+// How the built-in programs fold the offer of an edge, a word pack(key, src),
+// into the destination's: kFoldMin takes the smaller word, kFoldKey a smaller
+// key only. Any other operator (also one derived from these) is called through
+// its own AccumulateBuffer.
+enum : int { kFoldNone = 0, kFoldMin = 1, kFoldKey = 2 };
+template <class Op>
+struct EdgeFold {
+    static constexpr int kKind = kFoldNone;
+    __device__ static uint32_t key(uint32_t, uint32_t) { return 0; }
+};
+template <>
+struct EdgeFold<api::SSSP> {
+    static constexpr int kKind = kFoldMin;
+    __device__ static uint32_t key(uint32_t weight, uint32_t pushed) { return pushed + weight; }
+};
+template <>
+struct EdgeFold<api::BFS> {
+    static constexpr int kKind = kFoldMin;
+    __device__ static uint32_t key(uint32_t, uint32_t pushed) { return pushed; }
+};
+template <>
+struct EdgeFold<api::CC> {
+    static constexpr int kKind = kFoldKey;
+    __device__ static uint32_t key(uint32_t, uint32_t pushed) { return pushed; }
+};
 
 template <class Op>
 struct ERelax {
@@ -678,6 +793,66 @@ struct ERelax {
         }
         if (!op.AccumulateBuffer(u, v, w, &buffer[v], p)) return false;
         return atomicExch(&stamp[v], stamp_val) != stamp_val;
+    }
+    template <int N>
+    __device__ __forceinline__ void apply_n(const uint32_t (&u)[N], const uint32_t (&v)[N], const uint32_t (&push)[N],
+                                            const uint64_t (&peek)[N], bool (&enq)[N]) const {
+        if constexpr (!Op::kTraversal) {  // PageRank: the crossing rule of AccumulateBuffer
+            float old[N];
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                old[j] = 0.0f;
+                if (v[j] != kGap) old[j] = unsafeAtomicAdd(&buffer[v[j]], from_bits<float>(push[j]));
+            }
+#pragma unroll
+            for (int j = 0; j < N; ++j) enq[j] = v[j] != kGap && op.Crosses(old[j], from_bits<float>(push[j]));
+        } else {
+            uint32_t w[N];
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                w[j] = Op::kWeighted ? sg_weight(wmode, wseed, u[j], v[j]) : 0u;
+                enq[j] = v[j] != kGap && op.MayImprove(u[j], w[j], from_bits<typename Op::push_t>(push[j]), peek[j]);
+            }
+            if constexpr (EdgeFold<Op>::kKind == kFoldMin) {
+                unsigned long long old[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    old[j] = 0;
+                    if (enq[j]) old[j] = atomicMin(&buffer[v[j]], api::pack(EdgeFold<Op>::key(w[j], push[j]), u[j]));
+                }
+#pragma unroll
+                for (int j = 0; j < N; ++j) enq[j] = enq[j] && EdgeFold<Op>::key(w[j], push[j]) < api::hi32(old[j]);
+            } else if constexpr (EdgeFold<Op>::kKind == kFoldKey) {
+                unsigned long long old[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    old[j] = 0;
+                    if (enq[j]) old[j] = atomicCAS(&buffer[v[j]], peek[j], api::pack(EdgeFold<Op>::key(w[j], push[j]), u[j]));
+                }
+#pragma unroll
+                for (int j = 0; j < N; ++j)  // another offer came between: fold as usual
+                    if (enq[j] && old[j] != peek[j])
+                        enq[j] = op.AccumulateBuffer(u[j], v[j], w[j], &buffer[v[j]], from_bits<typename Op::push_t>(push[j]));
+            } else {
+#pragma unroll
+                for (int j = 0; j < N; ++j)
+                    if (enq[j])
+                        enq[j] = op.AccumulateBuffer(u[j], v[j], w[j], &buffer[v[j]], from_bits<typename Op::push_t>(push[j]));
+            }
+        }
+        claim<N>(v, enq);
+    }
+    // of the vertices to append, those not yet on the next frontier
+    template <int N>
+    __device__ __forceinline__ void claim(const uint32_t (&v)[N], bool (&enq)[N]) const {
+        uint32_t was[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            was[j] = stamp_val;
+            if (enq[j]) was[j] = atomicExch(&stamp[v[j]], stamp_val);
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) enq[j] = was[j] != stamp_val;
     }
 };
 
@@ -715,15 +890,24 @@ struct EInvalidate {
     uint32_t cshift;
     __device__ EInvalidate with_round(uint32_t) const { return *this; }
     __device__ uint64_t load(uint32_t v) const { return ld_relaxed(&buffer[v]); }
-    __device__ bool apply(uint32_t u, uint32_t v, uint32_t, uint64_t b) const {
-        if (Op::Parent(b) != u) return false;
-        const uint32_t bit = 1u << (v & 31);
-        if (atomicOr(&inval[v >> 5], bit) & bit) return false;
-        coarse_mark(coarse, cshift, v);
-        typename Op::buffer_t bb = b;
-        op.AccumulateBuffer_del(u, v, &bb, &value[v]);
-        buffer[v] = bb;
-        return true;  // counted by the frontier it joins
+    template <int N>
+    __device__ __forceinline__ void apply_n(const uint32_t (&u)[N], const uint32_t (&v)[N], const uint32_t (&)[N],
+                                            const uint64_t (&b)[N], bool (&enq)[N]) const {
+        uint32_t was[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            was[j] = ~0u;
+            if (v[j] != kGap && Op::Parent(b[j]) == u[j]) was[j] = atomicOr(&inval[v[j] >> 5], 1u << (v[j] & 31));
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            enq[j] = !((was[j] >> (v[j] & 31)) & 1u);  // each child once; counted by the frontier it joins
+            if (!enq[j]) continue;
+            coarse_mark(coarse, cshift, v[j]);
+            typename Op::buffer_t bb = b[j];
+            op.AccumulateBuffer_del(u[j], v[j], &bb, &value[v[j]]);
+            buffer[v[j]] = bb;
+        }
     }
 };
 

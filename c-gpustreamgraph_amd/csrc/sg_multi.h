@@ -379,6 +379,15 @@ __device__ void mwalk(const GraphView &g, const MultiState &ms, const PassIO &io
     }
 }
 
+// Owner of edge k among 64 staged lists: the largest j with excl[j] <= k.
+__device__ __forceinline__ uint32_t staged_owner(const uint32_t *excl, uint32_t k) {
+    uint32_t lo = 0;
+#pragma unroll
+    for (uint32_t step = kWave / 2; step > 0; step >>= 1)
+        if (excl[lo + step] <= k) lo += step;
+    return lo;
+}
+
 // LDS of the light path (per wave): 64 items of a wave batch.
 constexpr uint32_t kMLightQS = 16;  // light path for one group of at most this many slots
 struct MLight {

@@ -265,7 +265,9 @@ struct PageRank {
     // when |residual| crosses the threshold (the crossing rule of
     // hybrid_pr_host.cu:96-99, extended to negative residuals)
     __device__ bool AccumulateBuffer(uint32_t, uint32_t, uint32_t, buffer_t *p_buffer, push_t pushed) const {
-        const float old = unsafeAtomicAdd(p_buffer, pushed);
+        return Crosses(unsafeAtomicAdd(p_buffer, pushed), pushed);
+    }
+    __device__ bool Crosses(float old, float pushed) const {
         const float now = old + pushed;
         const float e = (float)m_error;
         return fabsf(now) > e && !(fabsf(old) > e);

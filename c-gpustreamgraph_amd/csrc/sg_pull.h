@@ -531,6 +531,7 @@ struct PrShared {
         LightWave light[kPrWaves];
     };
     unsigned long long red[kPrWaves][4];
+    uint32_t n[kPrWaves + 1];
 };
 static_assert(sizeof(PrShared<true>) <= 160 * 1024 && sizeof(PrShared<false>) <= 160 * 1024, "one block's LDS");
 
@@ -615,7 +616,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_step(GraphView g, PullPlan pl, 
         light_body(g, io, VPrRanks{p.pv_in, p.unlabel}, efn, g.nv, gwave, nwaves, sh.light[w], st, ws);
     else
         light_body(g, io, VPrList{p.op, p.value, p.res}, efn, rd.n_list, gwave, nwaves, sh.light[w], st, ws);
-    stage_flush(st, io);
+    block_flush<kPrWaves>(st, io, sh.n);
     stage_count_flush(st, io);
     block_stats<kPrWaves>(ws, sh.red, io.stats);
 }
@@ -632,6 +633,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_tail(GraphView g, PullPlan pl, 
     if (rd.idle) return;
     __shared__ uint32_t s_out[kPrWaves][kOutStage];
     __shared__ unsigned long long s_red[kPrWaves][4];
+    __shared__ uint32_t s_n[kPrWaves + 1];
     const uint32_t w = threadIdx.x / kWave;
     const uint64_t first = (uint64_t)blockIdx.x * kPrBlock + threadIdx.x, stride = (uint64_t)gridDim.x * kPrBlock;
     if (rd.n_pv) {
@@ -675,7 +677,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_tail(GraphView g, PullPlan pl, 
     const uint32_t nh = min(*io.heavy_cnt, io.heavy_cap);
     const ERelax<api::PageRank> efn{p.op, p.res, p.stamp, io.round + 1, 0, 0};
     heavy_body(g, hio, efn, nh, (uint64_t)w * gridDim.x + blockIdx.x, (uint64_t)gridDim.x * kPrWaves, st, ws);
-    stage_flush(st, io);
+    block_flush<kPrWaves>(st, io, s_n);
     stage_count_flush(st, io);
     block_stats<kPrWaves>(ws, s_red, io.stats);
 }
@@ -955,14 +957,22 @@ struct EPullSeed {
     const uint32_t *unlabel;  // vertex of each in-list id (null: ids are vertices)
     __device__ uint32_t vertex(uint32_t x) const { return unlabel ? unlabel[x] : x; }
     __device__ uint64_t load(uint32_t x) const { return ld_peek(&buffer[vertex(x)]); }
-    // v: the invalidated vertex whose in-list is walked; x: one in-list entry
-    __device__ bool apply(uint32_t v, uint32_t x, uint32_t, uint64_t bu) const {
-        const uint32_t u = vertex(x);
-        const uint32_t w = Op::kWeighted ? sg_weight(wmode, wseed, u, v) : 0u;
-        const auto p = op.PushValue(bu);
-        if (!op.MayImprove(u, w, p, ld_peek(&buffer[v]))) return false;
-        if (!op.AccumulateBuffer(u, v, w, &buffer[v], p)) return false;
-        return atomicExch(&stamp[v], stamp_val) != stamp_val;
+    // v: the invalidated vertices whose in-lists are walked; x: in-list entries
+    template <int N>
+    __device__ __forceinline__ void apply_n(const uint32_t (&v)[N], const uint32_t (&x)[N], const uint32_t (&)[N],
+                                            const uint64_t (&bu)[N], bool (&enq)[N]) const {
+        uint32_t u[N], w[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            u[j] = x[j] != kGap ? vertex(x[j]) : 0u;
+            w[j] = Op::kWeighted ? sg_weight(wmode, wseed, u[j], v[j]) : 0u;
+            enq[j] = x[j] != kGap && op.MayImprove(u[j], w[j], op.PushValue(bu[j]), ld_peek(&buffer[v[j]]));
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (enq[j])
+                enq[j] = op.AccumulateBuffer(u[j], v[j], w[j], &buffer[v[j]], op.PushValue(bu[j])) &&
+                         atomicExch(&stamp[v[j]], stamp_val) != stamp_val;
     }
 };
 
