@@ -123,97 +123,6 @@ __device__ __forceinline__ void reset_children(const MultiState &ms, const PassI
     stage_push(app, v, st, io);
 }
 
-// Walk for a sparse slot mask (at most kSparseSlots queries active at u):
-// one lane per edge, each lane trying the few active slots in turn, instead
-// of QS lanes per edge of which most would idle. kMode as mwalk.
-constexpr int kSparseSlots = 4;
-constexpr int kSparseUnroll = 4;  // edges per lane in flight
-template <int kMode>
-__device__ void mwalk_sparse(const GraphView &g, const MultiState &ms, const PassIO &io, OutStage &st, uint32_t *stamp,
-                             uint32_t stamp_val, uint32_t u, uint32_t grp, uint64_t mask, uint64_t start, uint32_t len,
-                             unsigned long long &edges) {
-    uint32_t sl[kSparseSlots], dus[kSparseSlots];
-    bool unit[kSparseSlots], live[kSparseSlots];
-    bool any = false;
-    uint64_t m = mask;
-#pragma unroll
-    for (int a = 0; a < kSparseSlots; ++a) {  // the active slots and u's distances (wave-uniform)
-        sl[a] = 0;
-        dus[a] = kInf;
-        unit[a] = false;
-        live[a] = false;
-        if (m) {
-            const uint32_t s = (uint32_t)__builtin_ctzll(m);
-            m &= m - 1;
-            const uint32_t qi = grp * ms.QS + s;
-            const uint8_t kind = ms.kind[qi];
-            sl[a] = s;
-            unit[a] = kind == kQUnit;
-            if (kMode == 0) {
-                dus[a] = kind == kQNone ? kInf : hi32(ld_relaxed(&ms.best[(uint64_t)u * ms.KP + qi]));
-                live[a] = dus[a] != kInf;
-            } else {
-                live[a] = kind != kQNone;
-            }
-            any = any || live[a];
-        }
-    }
-    if (!any) return;
-    edges += len;
-    const uint32_t lane = lane_id();
-    for (uint32_t e0 = 0; e0 < len; e0 += kWave * kSparseUnroll) {
-        uint32_t vv[kSparseUnroll];
-#pragma unroll
-        for (int j = 0; j < kSparseUnroll; ++j) {
-            const uint32_t e = e0 + j * kWave + lane;
-            vv[j] = e < len ? edge_at(g, start + e) : kGap;
-        }
-#pragma unroll
-        for (int j = 0; j < kSparseUnroll; ++j) {
-            const uint32_t v = vv[j];
-            bool app = false;
-            if (v != kGap) {
-                if (kMode == 0) {
-                    const uint32_t w = sg_weight(ms.wmode, ms.wseed, u, v);
-                    uint64_t better = 0;
-#pragma unroll
-                    for (int a = 0; a < kSparseSlots; ++a) {
-                        if (!live[a]) continue;
-                        const uint32_t cand = dus[a] + (unit[a] ? 1u : w);
-                        unsigned long long *p = &ms.best[(uint64_t)v * ms.KP + grp * ms.QS + sl[a]];
-                        const unsigned long long nw = pack(cand, u);
-                        if (nw < ld_peek(p) && cand < hi32(atomicMin(p, nw))) better |= 1ull << sl[a];
-                    }
-                    if (better) {
-                        atomicOr(&ms.act[(uint64_t)v * ms.G + grp], better);
-                        app = atomicExch(&stamp[v], stamp_val) != stamp_val;
-                    }
-                } else {
-                    // slots of v whose tree parent is u: claim them once, reset them
-                    uint64_t child = 0;
-#pragma unroll
-                    for (int a = 0; a < kSparseSlots; ++a) {
-                        if (!live[a]) continue;
-                        const unsigned long long b = ld_relaxed(&ms.best[(uint64_t)v * ms.KP + grp * ms.QS + sl[a]]);
-                        if (lo32(b) == u && hi32(b) != kInf) child |= 1ull << sl[a];
-                    }
-                    uint64_t fresh = 0;
-                    if (child) fresh = child & ~atomicOr(&ms.inv[(uint64_t)v * ms.G + grp], child);
-                    if (fresh) {
-                        atomicOr(&ms.ninv[(uint64_t)v * ms.G + grp], fresh);
-                        atomicOr(&ms.invbit[v >> 5], 1u << (v & 31));
-                        coarse_mark(ms.coarse, ms.cshift, v);
-                        app = atomicExch(&stamp[v], stamp_val) != stamp_val;
-                        for (uint64_t f = fresh; f; f &= f - 1)
-                            ms.best[(uint64_t)v * ms.KP + grp * ms.QS + (uint32_t)__builtin_ctzll(f)] = ~0ull;
-                    }
-                }
-            }
-            stage_push(app, v, st, io);
-        }
-    }
-}
-
 // Position of the r-th (0-based) set bit of m; r < popcount(m).
 __device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r) {
     uint32_t pos = 0;
@@ -229,152 +138,225 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r) {
     return pos;
 }
 
-// Walk for a mid-density slot mask (W/2 < popcount <= W, W = 8, 16 or 32
-// below the group's QS): the active slots are packed into W lanes, so a wave
-// step covers 64 / W edges instead of 64 / QS with most lanes idle. Lane
-// rank r takes the r-th active slot; the slot bits of an edge's hits are
-// OR-reduced over its W lanes before the one atomic per item. kMode as mwalk.
+// A wave takes the lists of up to 64 (vertex, group) items at a time: lane i
+// holds item i's words, the lists are then walked one after the other, each
+// item's ids and distances loaded while the one before it is walked.
+struct MItem {
+    uint32_t u, grp, len;
+    uint64_t mask, start;
+};
+
+// Slot bits of rank bits (packed lanes).
+__device__ __forceinline__ uint64_t rank_to_slots(uint64_t bits, uint64_t mask) {
+    uint64_t s = 0;
+    while (bits) {
+        s |= 1ull << nth_set_bit(mask, (uint32_t)__builtin_ctzll(bits));
+        bits &= bits - 1;
+    }
+    return s;
+}
+
+// What the edges of a step did, one edge per lane: hit = slots of v that
+// dropped (kMode 0) or whose tree parent is the walked vertex (kMode 1).
 template <int kMode>
-__device__ __forceinline__ void mwalk_compact(const GraphView &g, const MultiState &ms, const PassIO &io, OutStage &st, uint32_t *stamp,
-                              uint32_t stamp_val, uint32_t u, uint32_t grp, uint64_t mask, uint32_t wlog, uint64_t start,
-                              uint32_t len, unsigned long long &edges) {
+__device__ __forceinline__ void mfinish(const MultiState &ms, const PassIO &io, OutStage &st, uint32_t *stamp,
+                                        uint32_t stamp_val, uint32_t grp, uint32_t v, uint64_t hit) {
+    bool app = false;
+    if (hit) {
+        if (kMode == 0) {
+            atomicOr(&ms.act[(uint64_t)v * ms.G + grp], hit);
+            app = atomicExch(&stamp[v], stamp_val) != stamp_val;
+        } else {  // claim the slots once, queue them, reset their words
+            const uint64_t fresh = hit & ~atomicOr(&ms.inv[(uint64_t)v * ms.G + grp], hit);
+            if (fresh) {
+                atomicOr(&ms.ninv[(uint64_t)v * ms.G + grp], fresh);
+                atomicOr(&ms.invbit[v >> 5], 1u << (v & 31));
+                coarse_mark(ms.coarse, ms.cshift, v);
+                app = atomicExch(&stamp[v], stamp_val) != stamp_val;
+                for (uint64_t f = fresh; f; f &= f - 1)
+                    ms.best[(uint64_t)v * ms.KP + grp * ms.QS + (uint32_t)__builtin_ctzll(f)] = ~0ull;
+            }
+        }
+    }
+    stage_push(app, v, st, io);
+}
+
+// Walk one item for a sparse slot mask (at most kSparseSlots queries active at
+// u): one lane per edge, the few active slots side by side, instead of QS
+// lanes per edge of which most would idle.
+constexpr int kSparseSlots = 4;
+template <int kMode>
+__device__ __forceinline__ void mwalk_sparse(const GraphView &g, const MultiState &ms, const PassIO &io, OutStage &st,
+                                             uint32_t *stamp, uint32_t stamp_val, uint32_t u, uint32_t grp, uint64_t mask,
+                                             uint64_t start, uint32_t len, uint32_t vv, uint32_t du, uint64_t units) {
+    uint32_t sl[kSparseSlots], dus[kSparseSlots];
+    bool unit[kSparseSlots], live[kSparseSlots];
+    uint64_t m = mask;
+#pragma unroll
+    for (int a = 0; a < kSparseSlots; ++a) {  // the active slots and u's distances (wave-uniform)
+        live[a] = m != 0;
+        sl[a] = m ? (uint32_t)__builtin_ctzll(m) : 0u;
+        m &= m - 1;
+        unit[a] = (units >> sl[a]) & 1ull;
+        dus[a] = (uint32_t)__builtin_amdgcn_readlane((int)du, (int)sl[a]);
+    }
     const uint32_t lane = lane_id();
-    const uint32_t W = 1u << wlog;
-    const uint32_t r = lane & (W - 1);  // rank among the active slots
-    const uint32_t sub = lane >> wlog;   // edge of the wave step
-    const uint32_t per = kWave >> wlog;  // edges per wave step
-    const bool on = r < (uint32_t)__popcll(mask);
-    const uint32_t slot = on ? nth_set_bit(mask, r) : 0u;
-    const uint32_t qi = grp * ms.QS + slot;
-    const uint8_t kind = on ? ms.kind[qi] : (uint8_t)kQNone;
-    uint32_t du = kInf;
-    if (kMode == 0 && on) du = hi32(ld_relaxed(&ms.best[(uint64_t)u * ms.KP + qi]));
-    const bool live = on && kind != kQNone && (kMode == 1 || du != kInf);
-    if (!__any(live)) return;
-    edges += len;
-    for (uint32_t e0 = 0; e0 < len; e0 += per * kMUnroll) {
-        uint32_t vv[kMUnroll];
+    for (uint32_t e0 = 0; e0 < len; e0 += kWave) {
+        const bool in = e0 + lane < len;
+        const uint32_t v = e0 == 0 ? vv : edge_at(g, start + min(e0 + lane, len - 1));
+        unsigned long long *const p = &ms.best[(uint64_t)v * ms.KP + grp * ms.QS];
+        unsigned long long b[kSparseSlots];
 #pragma unroll
-        for (int j = 0; j < kMUnroll; ++j) {
-            const uint32_t e = e0 + j * per + sub;
-            vv[j] = e < len ? edge_at(g, start + e) : kGap;
+        for (int a = 0; a < kSparseSlots; ++a) {
+            b[a] = 0;
+            if (live[a]) b[a] = kMode == 0 ? ld_peek(p + sl[a]) : ld_relaxed(p + sl[a]);
         }
-        uint64_t pk[kMUnroll];
-        uint32_t cand[kMUnroll];
+        uint64_t hit = 0;
+        if (kMode == 0) {
+            const uint32_t w = sg_weight(ms.wmode, ms.wseed, u, v);
+            uint32_t cand[kSparseSlots];
 #pragma unroll
-        for (int j = 0; j < kMUnroll; ++j) {
-            const bool ok = live && vv[j] != kGap;
-            if (kMode == 0) {
-                cand[j] = ok ? du + qweight(ms, kind, u, vv[j]) : kInf;
-                pk[j] = ok ? ld_peek(&ms.best[(uint64_t)vv[j] * ms.KP + qi]) : 0ull;
-            } else {
-                cand[j] = 0;
-                pk[j] = ok ? ld_relaxed(&ms.best[(uint64_t)vv[j] * ms.KP + qi]) : 0ull;
+            for (int a = 0; a < kSparseSlots; ++a) {
+                cand[a] = dus[a] + (unit[a] ? 1u : w);
+                const unsigned long long nw = pack(cand[a], u);
+                const bool ok = in && live[a] && nw < b[a];
+                b[a] = 0;
+                if (ok) b[a] = atomicMin(p + sl[a], nw);
             }
-        }
 #pragma unroll
-        for (int j = 0; j < kMUnroll; ++j) {
-            const uint32_t v = vv[j];
-            bool hit = false;
-            if (kMode == 0) {
-                const unsigned long long nw = pack(cand[j], u);
-                if (cand[j] != kInf && nw < pk[j]) {
-                    const unsigned long long old = atomicMin(&ms.best[(uint64_t)v * ms.KP + qi], nw);
-                    hit = cand[j] < hi32(old);
-                }
-            } else {
-                hit = live && v != kGap && lo32(pk[j]) == u && hi32(pk[j]) != kInf;
-            }
-            // slot bits of this edge's hits, gathered in every lane of its W-lane group
-            unsigned long long bits = hit ? (1ull << slot) : 0ull;
-            for (uint32_t o = 1; o < W; o <<= 1) bits |= __shfl_xor(bits, (int)o, kWave);
-            bool app = false;
-            if (kMode == 0) {
-                if (r == 0 && bits) {
-                    atomicOr(&ms.act[(uint64_t)v * ms.G + grp], bits);
-                    app = atomicExch(&stamp[v], stamp_val) != stamp_val;
-                }
-            } else {
-                unsigned long long fresh = 0;
-                if (r == 0 && bits) fresh = bits & ~atomicOr(&ms.inv[(uint64_t)v * ms.G + grp], bits);
-                fresh = __shfl(fresh, (int)(sub << wlog), kWave);
-                if (r == 0 && fresh) {
-                    atomicOr(&ms.ninv[(uint64_t)v * ms.G + grp], fresh);
-                    atomicOr(&ms.invbit[v >> 5], 1u << (v & 31));
-                    coarse_mark(ms.coarse, ms.cshift, v);
-                    app = atomicExch(&stamp[v], stamp_val) != stamp_val;
-                }
-                if (on && ((fresh >> slot) & 1u)) ms.best[(uint64_t)v * ms.KP + qi] = ~0ull;
-            }
-            stage_push(app, v, st, io);
+            for (int a = 0; a < kSparseSlots; ++a)
+                if (live[a] && cand[a] < hi32(b[a])) hit |= 1ull << sl[a];
+        } else {
+#pragma unroll
+            for (int a = 0; a < kSparseSlots; ++a)
+                if (in && live[a] && lo32(b[a]) == u && hi32(b[a]) != kInf) hit |= 1ull << sl[a];
         }
+        mfinish<kMode>(ms, io, st, stamp, stamp_val, grp, v, hit);
     }
 }
 
-// Walk len edges of u from slot position start for the slots in mask.
-// kMode 0: relax (activations go to act); kMode 1: reset tree children whose
-// parent is u (resets go to inv / ninv and the vertex bitmaps).
+// Relax (kMode 0: activations go to act) or reset the tree children (kMode 1:
+// resets go to inv / ninv and the vertex bitmaps) along the lists of the
+// wave's items, lane i holding item i; n items.
+// 64 edges at a time: their ids and weights are loaded and computed one edge
+// per lane, then kMUnroll edges (QS = 64; more with fewer lanes per edge) are
+// tested and updated at once, the updates in flight together, and what the 64
+// edges did is marked one edge per lane. With a weight in every lane and a
+// wait for every edge's update, a dense round of 64 queries over 8 M edges
+// took 2.1 ms, bound by instruction issue and those waits.
 template <int kMode>
-__device__ void mwalk(const GraphView &g, const MultiState &ms, const PassIO &io, OutStage &st, uint32_t *stamp,
-                      uint32_t stamp_val, uint32_t u, uint32_t grp, uint64_t mask, uint64_t start, uint32_t len,
-                      unsigned long long &edges) {
-    const uint32_t np = (uint32_t)__popcll(mask);
-    if (ms.QS > kSparseSlots && np <= kSparseSlots) {
-        mwalk_sparse<kMode>(g, ms, io, st, stamp, stamp_val, u, grp, mask, start, len, edges);
-        return;
-    }
-    if (ms.QS >= 16 && 2 * np <= ms.QS) {  // 8, 16 or 32 lanes per edge instead of QS
-        const uint32_t wlog = np <= 8 ? 3u : np <= 16 ? 4u : 5u;
-        mwalk_compact<kMode>(g, ms, io, st, stamp, stamp_val, u, grp, mask, wlog, start, len, edges);
-        return;
-    }
-    const QLane q = qlane(ms);
-    const bool on = (mask >> q.slot) & 1u;
-    const uint32_t qi = grp * ms.QS + q.slot;
-    const uint8_t kind = ms.kind[qi];
-    uint32_t du = kInf;
-    if (kMode == 0 && on) du = hi32(ld_relaxed(&ms.best[(uint64_t)u * ms.KP + qi]));
-    const bool live = on && kind != kQNone && (kMode == 1 || du != kInf);
-    if (!__any(live)) return;
-    edges += len;
-    for (uint32_t e0 = 0; e0 < len; e0 += q.per * kMUnroll) {
-        uint32_t vv[kMUnroll];
-#pragma unroll
-        for (int j = 0; j < kMUnroll; ++j) {
-            const uint32_t e = e0 + j * q.per + q.sub;
-            vv[j] = e < len ? edge_at(g, start + e) : kGap;
+__device__ __forceinline__ void mwalk_items(const GraphView &g, const MultiState &ms, const PassIO &io, OutStage &st,
+                                            uint32_t *stamp, uint32_t stamp_val, const MItem &it, uint32_t n,
+                                            unsigned long long &edges) {
+    const uint32_t lane = lane_id(), ql = min(lane, ms.QS - 1);
+    const uint64_t slots = ms.QS == 64 ? ~0ull : (1ull << ms.QS) - 1;
+    uint32_t kgrp = ~0u;  // the group units / used describe
+    uint64_t units = 0, used = 0;
+    // item i's first 64 ids and u's distance in slot `lane`; the mask was taken
+    // before, and the distance is read past the caches: an improvement that
+    // comes later sets its bit again
+    auto ids = [&](uint32_t i) {
+        const uint32_t len = (uint32_t)__builtin_amdgcn_readlane((int)it.len, (int)i);
+        return len ? edge_at(g, read_lane_u64(it.start, (int)i) + min(lane, len - 1)) : 0u;
+    };
+    auto dist = [&](uint32_t i) {
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)it.u, (int)i);
+        const uint32_t grp = (uint32_t)__builtin_amdgcn_readlane((int)it.grp, (int)i);
+        return kMode == 0 ? hi32(ld_relaxed(&ms.best[(uint64_t)u * ms.KP + grp * ms.QS + ql])) : 0u;
+    };
+    uint32_t vn = ids(0), dn = dist(0);
+    for (uint32_t i = 0; i < n; ++i) {
+        uint32_t vv = vn;
+        const uint32_t du0 = dn;
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)it.u, (int)i);
+        const uint32_t grp = (uint32_t)__builtin_amdgcn_readlane((int)it.grp, (int)i);
+        const uint32_t len = (uint32_t)__builtin_amdgcn_readlane((int)it.len, (int)i);
+        const uint64_t start = read_lane_u64(it.start, (int)i);
+        uint64_t mask = read_lane_u64(it.mask, (int)i);
+        if (i + 1 < n) {
+            vn = ids(i + 1);
+            dn = dist(i + 1);
         }
-        if (kMode == 0) {
-            // all peeks in flight before the first atomic
-            uint64_t pk[kMUnroll];
-            uint32_t cand[kMUnroll];
+        if (grp != kgrp) {
+            const uint8_t kind = ms.kind[grp * ms.QS + ql];
+            units = __ballot(kind == kQUnit);
+            used = __ballot(kind != kQNone) & slots;
+            kgrp = grp;
+        }
+        mask &= used;
+        if (kMode == 0) mask &= __ballot(du0 != kInf);
+        if (mask == 0 || len == 0) continue;
+        edges += len;
+        const uint32_t np = (uint32_t)__popcll(mask);
+        if (ms.QS > kSparseSlots && np <= kSparseSlots) {
+            mwalk_sparse<kMode>(g, ms, io, st, stamp, stamp_val, u, grp, mask, start, len, vv, du0, units);
+            continue;
+        }
+        // W = 2^wlog lanes per edge: rank r of an edge's lanes takes the r-th
+        // active slot (packed) or slot r
+        const bool packed = ms.QS >= 16 && 2 * np <= ms.QS;
+        const uint32_t wlog = packed ? (np <= 8 ? 3u : np <= 16 ? 4u : 5u) : ms.qs_log;
+        const uint32_t r = lane & ((1u << wlog) - 1u);
+        const bool live = packed ? r < np : ((mask >> r) & 1ull) != 0;
+        const uint32_t slot = packed ? (live ? nth_set_bit(mask, r) : 0u) : r;
+        const bool unit = (units >> slot) & 1ull;
+        const uint32_t du = __shfl(du0, (int)slot, kWave);
+        unsigned long long *const col = ms.best + grp * ms.QS + slot;
+        const uint32_t per = kWave >> wlog, sub = lane >> wlog;
+        const uint64_t ones = wlog == 6 ? ~0ull : (1ull << (1u << wlog)) - 1;
+        for (uint32_t e0 = 0; e0 < len; e0 += kWave) {
+            const uint32_t ne = min(len - e0, (uint32_t)kWave);
+            const uint32_t wv = kMode == 0 ? sg_weight(ms.wmode, ms.wseed, u, vv) : 0u;
+            const uint32_t vnext = e0 + kWave < len ? edge_at(g, start + min(e0 + kWave + lane, len - 1)) : 0u;
+            uint64_t hit = 0;  // ranks of this lane's edge
+            // edges past the last repeat it (lanes past ne hold its id): their
+            // updates change nothing, their marks fall on the same vertex
+            for (uint32_t s0 = 0; s0 < ne; s0 += per * kMUnroll) {
+                uint64_t pk[kMUnroll];
+                uint32_t cand[kMUnroll];
+                unsigned long long *p[kMUnroll];
+                bool ok[kMUnroll];
 #pragma unroll
-            for (int j = 0; j < kMUnroll; ++j) {
-                const bool ok = live && vv[j] != kGap;
-                cand[j] = ok ? du + qweight(ms, kind, u, vv[j]) : kInf;
-                pk[j] = ok ? ld_peek(&ms.best[(uint64_t)vv[j] * ms.KP + qi]) : 0ull;
-            }
-#pragma unroll
-            for (int j = 0; j < kMUnroll; ++j) {
-                bool hit = false;
-                const unsigned long long nw = pack(cand[j], u);
-                if (cand[j] != kInf && nw < pk[j]) {
-                    const unsigned long long old = atomicMin(&ms.best[(uint64_t)vv[j] * ms.KP + qi], nw);
-                    hit = cand[j] < hi32(old);
+                for (int j = 0; j < kMUnroll; ++j) {
+                    uint32_t v, w;
+                    if (wlog == 6) {
+                        v = (uint32_t)__builtin_amdgcn_readlane((int)vv, (int)(s0 + j));
+                        w = (uint32_t)__builtin_amdgcn_readlane((int)wv, (int)(s0 + j));
+                    } else {
+                        const uint32_t e = min(s0 + j * per + sub, (uint32_t)kWave - 1);
+                        v = __shfl(vv, (int)e, kWave);
+                        w = kMode == 0 ? __shfl(wv, (int)e, kWave) : 0u;
+                    }
+                    cand[j] = du + (unit ? 1u : w);
+                    p[j] = col + (uint64_t)v * ms.KP;
                 }
-                mark_items(ms, io, st, q, ms.act, grp, vv[j], hit, stamp, stamp_val);
-            }
-        } else {
-            uint64_t peek[kMUnroll];
 #pragma unroll
-            for (int j = 0; j < kMUnroll; ++j)
-                peek[j] = (live && vv[j] != kGap) ? ld_relaxed(&ms.best[(uint64_t)vv[j] * ms.KP + qi]) : 0ull;
+                for (int j = 0; j < kMUnroll; ++j) pk[j] = kMode == 0 ? ld_peek(p[j]) : ld_relaxed(p[j]);
+                if (kMode == 0) {
 #pragma unroll
-            for (int j = 0; j < kMUnroll; ++j) {
-                const uint32_t v = vv[j];
-                const bool child = live && v != kGap && lo32(peek[j]) == u && hi32(peek[j]) != kInf;
-                reset_children(ms, io, st, q, grp, v, child, stamp, stamp_val);
+                    for (int j = 0; j < kMUnroll; ++j) {
+                        const unsigned long long nw = pack(cand[j], u);
+                        // (a step's positions past 63 must not win an update that edge 63 marks)
+                        ok[j] = live && nw < pk[j] && (wlog == 6 || s0 + j * per + sub < (uint32_t)kWave);
+                        if (ok[j]) pk[j] = atomicMin(p[j], nw);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < kMUnroll; ++j) {
+                    const bool h = kMode == 0 ? ok[j] && cand[j] < hi32(pk[j])
+                                              : live && lo32(pk[j]) == u && hi32(pk[j]) != kInf;
+                    const uint64_t b = __ballot(h);
+                    if (wlog == 6) {
+                        hit = lane == s0 + j ? b : hit;
+                    } else if (b) {
+                        const uint32_t at = lane - (s0 + j * per);  // the lane's edge among the step's
+                        if (at < per) hit = (b >> (at << wlog)) & ones;
+                    }
+                }
             }
+            if (packed) hit = rank_to_slots(hit, mask);
+            mfinish<kMode>(ms, io, st, stamp, stamp_val, grp, vv, hit);
+            vv = vnext;
         }
     }
 }
@@ -515,6 +497,7 @@ __global__ void __launch_bounds__(kBlock) k_mround(GraphView g, MultiState ms, P
     __shared__ uint32_t s_out[kWavesPerBlock][kOutStage];
     __shared__ unsigned long long s_red[kWavesPerBlock], s_red2[kWavesPerBlock];
     __shared__ MLight s_light[kWavesPerBlock];
+    __shared__ uint32_t s_n[kWavesPerBlock + 1];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (io.zero_cnt) *io.zero_cnt = 0;
         if (io.heavy_zero) *io.heavy_zero = 0;
@@ -534,46 +517,55 @@ __global__ void __launch_bounds__(kBlock) k_mround(GraphView g, MultiState ms, P
     const bool light = ms.G == 1 && ms.QS <= kMLightQS;
     if (light) mlight<kMode>(g, ms, io, st, s_light[w], spill, spill_cap, stamp, n, gw, nw, edges, verts);
     // (frontier vertex, group) items, then the previous round's spilled
-    // descriptors, in one loop with one walk call site
+    // descriptors, in one loop: a wave takes up to 64 of them at a time, dealt
+    // out in turn (neighbours in the frontier are alike: a run of hubs would
+    // be one wave's work)
     const uint64_t items = light ? 0 : (uint64_t)n * ms.G;
-    for (uint64_t it = gw; it < items + nh; it += nw) {
-        uint32_t u, grp, len;
-        unsigned long long m;
-        uint64_t start;
-        if (it < items) {
-            u = io.in_list[it / ms.G];
-            grp = (uint32_t)(it % ms.G);
-            m = 0;
-            if (lane == 0) m = atomicExch(&masks[(uint64_t)u * ms.G + grp], 0ull);
-            m = __shfl(m, 0, kWave);
-            if (m == 0) continue;
-            ++verts;
-            start = list_start(g, u);
-            if (lane == 0) count_hot(g, u);
-            const uint32_t deg = g.deg[u];
-            len = min(deg, kMEdgeChunk);
-            if (deg > len) {
-                const uint32_t nch = (deg - len + kMEdgeChunk - 1) / kMEdgeChunk;
-                uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(io.heavy_cnt, nch);
-                base = __shfl(base, 0, kWave);
-                for (uint32_t c = lane; c < nch; c += kWave) {
-                    const uint32_t lo = len + c * kMEdgeChunk;
-                    if (base + c < spill_cap) spill[base + c] = MDesc{start + lo, m, u, min(kMEdgeChunk, deg - lo), grp, 0};
+    for (uint64_t i0 = gw; i0 < items + nh; i0 += nw * kWave) {
+        const uint64_t i = i0 + lane * nw;
+        MItem it{0, 0, 0, 0, 0};
+        uint32_t nch = 0, deg = 0;
+        if (i < items) {
+            it.u = io.in_list[i / ms.G];
+            it.grp = (uint32_t)(i % ms.G);
+            it.mask = atomicExch(&masks[(uint64_t)it.u * ms.G + it.grp], 0ull);
+            if (it.mask) {
+                it.start = list_start(g, it.u);
+                count_hot(g, it.u);
+                deg = g.deg[it.u];
+                it.len = min(deg, kMEdgeChunk);
+                nch = (deg - it.len + kMEdgeChunk - 1) / kMEdgeChunk;
+            }
+        } else if (i < items + nh) {
+            const MDesc d = sin[i - items];
+            it = MItem{d.u, d.grp, d.len, d.mask, d.start};
+        }
+        verts += (uint32_t)__popcll(__ballot(i < items && it.mask != 0));
+        const uint32_t incl = wave_incl_scan(nch);
+        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        if (tot) {  // the tails of long lists go to the next round
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(io.heavy_cnt, tot);
+            base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+            for (uint64_t m = __ballot(nch != 0); m; m &= m - 1) {  // lane by lane, its chunks side by side
+                const int l = __builtin_ctzll(m);
+                const uint32_t c1 = (uint32_t)__builtin_amdgcn_readlane((int)incl, l);
+                const uint32_t cn = (uint32_t)__builtin_amdgcn_readlane((int)nch, l), at = base + c1 - cn;
+                const MDesc d{read_lane_u64(it.start, l) + kMEdgeChunk, read_lane_u64(it.mask, l),
+                              (uint32_t)__builtin_amdgcn_readlane((int)it.u, l),
+                              (uint32_t)__builtin_amdgcn_readlane((int)deg, l) - kMEdgeChunk,
+                              (uint32_t)__builtin_amdgcn_readlane((int)it.grp, l), 0};
+                for (uint32_t c = lane; c < cn; c += kWave) {
+                    const uint32_t lo = c * kMEdgeChunk;
+                    if (at + c < spill_cap) spill[at + c] = MDesc{d.start + lo, d.mask, d.u, min(kMEdgeChunk, d.len - lo), d.grp, 0};
                     else atomicOr(io.stats + 3, 2ull);
                 }
             }
-        } else {
-            const MDesc d = sin[it - items];
-            u = d.u;
-            grp = d.grp;
-            m = d.mask;
-            start = d.start;
-            len = d.len;
         }
-        mwalk<kMode>(g, ms, io, st, stamp, io.round + 1, u, grp, m, start, len, edges);
+        mwalk_items<kMode>(g, ms, io, st, stamp, io.round + 1, it,
+                           (uint32_t)min_u64(kWave, (items + nh - i0 + nw - 1) / nw), edges);
     }
-    stage_flush(st, io);
+    block_flush<kWavesPerBlock>(st, io, s_n);
     // one atomic per counter and block
     if (lane == 0) {
         s_red[w] = edges;
@@ -641,6 +633,7 @@ __global__ void __launch_bounds__(kBlock) k_mpairs(MultiState ms, BatchView bv, 
     stage_flush(st, io);
 }
 
+constexpr int kSweepSlots = 4;
 // Edge-centric sweep for the batch: every live edge (u, v) whose target has a
 // reset slot relaxes v's reset slots from u (the sweep hits). Same wave tiles
 // as k_sweep_edges: the tile's hits are compacted in place in the wave's LDS
@@ -702,19 +695,36 @@ __global__ void __launch_bounds__(kSweepBlock) k_msweep(GraphView g, const unsig
                 for (uint32_t grp = 0; grp < ms.G; ++grp) {
                     uint64_t m = ms.inv[(uint64_t)v * ms.G + grp];
                     uint64_t better = 0;
-                    while (m) {
-                        const uint32_t slot = (uint32_t)__builtin_ctzll(m);
-                        m &= m - 1;
-                        const uint32_t qi = grp * ms.QS + slot;
-                        const uint8_t kind = ms.kind[qi];
-                        if (kind == kQNone) continue;
-                        const uint32_t du = hi32(ld_relaxed(&ms.best[(uint64_t)u * ms.KP + qi]));
-                        if (du == kInf) continue;
-                        const uint32_t cand = du + (kind == kQUnit ? 1u : wt);
-                        unsigned long long *p = &ms.best[(uint64_t)v * ms.KP + qi];
-                        const unsigned long long nw = pack(cand, u);
-                        if (nw >= ld_peek(p)) continue;
-                        if (cand < hi32(atomicMin(p, nw))) better |= 1ull << slot;
+                    unsigned long long *const bu = &ms.best[(uint64_t)u * ms.KP + grp * ms.QS];
+                    unsigned long long *const bv = &ms.best[(uint64_t)v * ms.KP + grp * ms.QS];
+                    while (m) {  // kSweepSlots slots at a time, their loads and updates in flight together
+                        uint32_t sl[kSweepSlots], cand[kSweepSlots];
+                        uint8_t kind[kSweepSlots];
+                        unsigned long long du[kSweepSlots], cur[kSweepSlots];
+#pragma unroll
+                        for (int a = 0; a < kSweepSlots; ++a) {  // past the last: the last again
+                            sl[a] = m ? (uint32_t)__builtin_ctzll(m) : sl[a ? a - 1 : 0];
+                            m &= m - 1;
+                        }
+#pragma unroll
+                        for (int a = 0; a < kSweepSlots; ++a) {
+                            kind[a] = ms.kind[grp * ms.QS + sl[a]];
+                            du[a] = ld_relaxed(bu + sl[a]);
+                            cur[a] = ld_peek(bv + sl[a]);
+                        }
+#pragma unroll
+                        for (int a = 0; a < kSweepSlots; ++a) {
+                            const uint32_t d = hi32(du[a]);
+                            const bool on = kind[a] != kQNone && d != kInf && (a == 0 || sl[a] != sl[a - 1]);
+                            cand[a] = d + (kind[a] == kQUnit ? 1u : wt);
+                            const unsigned long long nw = pack(cand[a], u);
+                            const bool ok = on && nw < cur[a];
+                            cur[a] = 0;
+                            if (ok) cur[a] = atomicMin(bv + sl[a], nw);
+                        }
+#pragma unroll
+                        for (int a = 0; a < kSweepSlots; ++a)
+                            if (cand[a] < hi32(cur[a])) better |= 1ull << sl[a];
                     }
                     if (better) {
                         atomicOr(&ms.act[(uint64_t)v * ms.G + grp], better);
