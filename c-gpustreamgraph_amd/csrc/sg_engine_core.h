@@ -32,6 +32,7 @@
 #include "sg_kernels.h"
 #include "sg_operators.h"
 #include "sg_pma.h"
+#include "sg_sort.h"
 #include "sg_multi.h"
 #include "sg_pull.h"
 
@@ -824,6 +825,9 @@ public:
     size_t raw_ins_cap_ = 0, raw_del_cap_ = 0;
     uint32_t *ins_k_ = nullptr, *ins_v_ = nullptr, *ins_k2_ = nullptr, *ins_v2_ = nullptr;
     size_t ins_cap_ = 0, ins_cap2_ = 0, ins_cap3_ = 0, ins_cap4_ = 0;
+    unsigned long long *sort_tmp_ = nullptr, *sort_split_ = nullptr;  // batch sort (sg_sort.h)
+    uint32_t *sort_hist_ = nullptr;
+    size_t sort_tmp_cap_ = 0, sort_split_cap_ = 0, sort_hist_cap_ = 0;
     unsigned long long *del_k_ = nullptr, *del_k2_ = nullptr;
     size_t del_cap_ = 0, del_cap2_ = 0;
     uint8_t *cub_tmp_ = nullptr;
@@ -1571,6 +1575,59 @@ public:
         d_del = raw_del_;
     }
 
+    // ins_k2_ / ins_v2_ and del_k2_ from the batch's pairs (sg_sort.h).
+    void sort_batch(const uint32_t *d_ins, uint32_t nins, const uint32_t *d_del, uint32_t ndel) {
+        if (nins + ndel == 0) return;
+        SortBatch sb{};
+        sb.nv = nv_;
+        sb.a = swap_pairs_ ? 1 : 0;
+        sb.b = swap_pairs_ ? 0 : 1;
+        sb.dropped = &ctl_->dropped;
+        const uint32_t *const pairs[2] = {d_ins, d_del};
+        const uint32_t n[2] = {nins, ndel};
+        uint64_t keys = 0, hist = 0;
+        for (int i = 0; i < 2; ++i) {
+            SortSide &x = sb.side[i];
+            x.pairs = pairs[i];
+            x.n = n[i];
+            if (n[i] <= kSortOne) continue;
+            x.nsplit = std::min(kSortMaxSplit, (n[i] + kSortBucket - 1) / kSortBucket);
+            x.tile = std::max<uint32_t>(1024, (n[i] + kSortRows - 1) / kSortRows);
+            x.rows = (n[i] + x.tile - 1) / x.tile;
+            keys += n[i];
+            hist += (uint64_t)x.rows * x.nbuckets() + x.nbuckets() + 1;
+        }
+        ensure(sort_tmp_, sort_tmp_cap_, std::max<uint64_t>(keys, 1));
+        ensure(sort_hist_, sort_hist_cap_, std::max<uint64_t>(hist, 1));
+        ensure(sort_split_, sort_split_cap_, 2 * kSortMaxSplit);
+        uint64_t at = 0, hat = 0;
+        for (int i = 0; i < 2; ++i) {
+            SortSide &x = sb.side[i];
+            x.tmp = sort_tmp_ + at;
+            x.hist = sort_hist_ + hat;
+            x.split = sort_split_ + i * kSortMaxSplit;
+            if (x.nsplit) {
+                at += x.n;
+                hat += (uint64_t)x.rows * x.nbuckets();
+                x.start = sort_hist_ + hat;
+                hat += x.nbuckets() + 1;
+            }
+        }
+        sb.side[0].out_key = ins_k2_;
+        sb.side[0].out_val = ins_v2_;
+        sb.side[1].out_del = del_k2_;
+        const uint32_t rows = sb.side[0].rows + sb.side[1].rows;
+        if (rows) {
+            hipLaunchKernelGGL(k_sort_count, dim3(rows), dim3(kSortBlock), 0, stream_, sb);
+            SG_LAUNCHED();
+            hipLaunchKernelGGL(k_sort_move, dim3(rows), dim3(kSortBlock), 0, stream_, sb);
+            SG_LAUNCHED();
+        }
+        const uint32_t nb = (nins ? sb.side[0].nsplit + 1 : 0u) + (ndel ? sb.side[1].nsplit + 1 : 0u);
+        hipLaunchKernelGGL(k_sort_buckets, dim3(nb), dim3(kSortBlock), 0, stream_, sb);
+        SG_LAUNCHED();
+    }
+
     // Sort the batch, list touched sources, cut their lists into chunks, count
     // survivors and new degrees. Leaves the graph unchanged.
     bool prepare(const uint32_t *d_ins, uint64_t nins64, const uint32_t *d_del, uint64_t ndel64) {
@@ -1578,12 +1635,15 @@ public:
         const uint32_t nins = (uint32_t)nins64, ndel = (uint32_t)ndel64;
         nins_ = nins;
         ndel_ = ndel;
-        ensure(ins_k_, ins_cap_, nins + 1);
-        ensure(ins_v_, ins_cap2_, nins + 1);
+        const bool own_sort = nins <= kSortMost && ndel <= kSortMost;
         ensure(ins_k2_, ins_cap3_, nins + 1);
         ensure(ins_v2_, ins_cap4_, nins + 1);
-        ensure(del_k_, del_cap_, ndel + 1);
         ensure(del_k2_, del_cap2_, ndel + 1);
+        if (!own_sort) {
+            ensure(ins_k_, ins_cap_, nins + 1);
+            ensure(ins_v_, ins_cap2_, nins + 1);
+            ensure(del_k_, del_cap_, ndel + 1);
+        }
         ensure_heavy(ne_ + nins);
         // chunks: sum over touched vertices of ceil(deg/CH) (with deletes) + ceil(ins/CH)
         const uint64_t chunk_bound = (ne_ + nins) / kMergeChunk + (uint64_t)nins + ndel + 64;
@@ -1598,23 +1658,27 @@ public:
         ensure(cpos_, cpos_cap_, chunk_bound + 1);
         fill<uint8_t>((uint8_t *)ctl_, sizeof(Ctl), 0);
         fill<unsigned long long>(ccount_, chunk_bound + 1, 0ull);
-        if (nins + ndel) {
-            hipLaunchKernelGGL(k_split, dim3(grid_for((uint64_t)nins + ndel, 256, 8192)), dim3(256), 0, stream_, nv_, d_ins, nins,
-                               d_del, ndel, ins_k_, ins_v_, del_k_, ctl_, swap_pairs_ ? 1 : 0);
-            SG_LAUNCHED();
-        }
+        size_t b1 = 0, b2 = 0, b3 = 0;
+        SG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, b3, ccount_, cpos_, (int)(chunk_bound + 1), stream_));
         // sort only the bits ids can hold: kb = bit length of nv, so a masked
         // kGap / ~0 (dropped pair) still compares above every valid key
         const int kb = nv_ ? 32 - __builtin_clz(nv_) : 1;
-        size_t b1 = 0, b2 = 0, b3 = 0;
-        SG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b1, ins_k_, ins_k2_, ins_v_, ins_v2_, (int)nins, 0, kb, stream_));
-        SG_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, b2, del_k_, del_k2_, (int)ndel, 0, 32 + kb, stream_));
-        SG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, b3, ccount_, cpos_, (int)(chunk_bound + 1), stream_));
+        if (!own_sort) {
+            SG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b1, ins_k_, ins_k2_, ins_v_, ins_v2_, (int)nins, 0, kb, stream_));
+            SG_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, b2, del_k_, del_k2_, (int)ndel, 0, 32 + kb, stream_));
+        }
         ensure(cub_tmp_, cub_cap_, std::max({b1, b2, b3}) + 256);
         size_t b = cub_cap_;
-        if (nins) SG_HIP(hipcub::DeviceRadixSort::SortPairs(cub_tmp_, b, ins_k_, ins_k2_, ins_v_, ins_v2_, (int)nins, 0, kb, stream_));
-        b = cub_cap_;
-        if (ndel) SG_HIP(hipcub::DeviceRadixSort::SortKeys(cub_tmp_, b, del_k_, del_k2_, (int)ndel, 0, 32 + kb, stream_));
+        if (own_sort) {
+            sort_batch(d_ins, nins, d_del, ndel);
+        } else {
+            hipLaunchKernelGGL(k_split, dim3(grid_for((uint64_t)nins + ndel, 256, 8192)), dim3(256), 0, stream_, nv_, d_ins, nins,
+                               d_del, ndel, ins_k_, ins_v_, del_k_, ctl_, swap_pairs_ ? 1 : 0);
+            SG_LAUNCHED();
+            if (nins) SG_HIP(hipcub::DeviceRadixSort::SortPairs(cub_tmp_, b, ins_k_, ins_k2_, ins_v_, ins_v2_, (int)nins, 0, kb, stream_));
+            b = cub_cap_;
+            if (ndel) SG_HIP(hipcub::DeviceRadixSort::SortKeys(cub_tmp_, b, del_k_, del_k2_, (int)ndel, 0, 32 + kb, stream_));
+        }
         bv_.ins_key = ins_k2_;
         bv_.ins_val = ins_v2_;
         bv_.nins = nins;
