@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_msweep(GraphView g, const unsig
         tp.advance(g, dpre, tiles);
         bool pass[kSweepPerLane];
 #pragma unroll
-        for (int j = 0; j < kSweepPerLane; ++j) pass[j] = vv[j] != kGap && coarse_test(s_filter, cs, vv[j]);
+        for (int j = 0; j < kSweepPerLane; ++j) pass[j] = coarse_test(s_filter, cs, vv[j] != kGap ? vv[j] : 0u) && vv[j] != kGap;
         uint32_t word[kSweepPerLane];
 #pragma unroll
         for (int j = 0; j < kSweepPerLane; ++j) word[j] = pass[j] ? ms.invbit[vv[j] >> 5] : 0u;

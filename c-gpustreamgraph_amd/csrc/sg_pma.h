@@ -574,23 +574,19 @@ __device__ __forceinline__ TileHead tile_head(unsigned long long raw) {
     return h;
 }
 
-// Per-source words of the tile's first kWave sources (lane i: source v0 + i,
-// off and dpre; position span is the vertex after the last source: its off
-// is the width check and its dpre the last source's end). Loaded one tile
-// ahead.
+// Per-source words of the tile's source v0 + i (position span is the vertex
+// after the last source: its off is the width check): its first slot, its
+// first edge and the edge after its last. The first kWave sources' words are
+// loaded one tile ahead.
 struct TilePre {
     uint64_t ov;
-    unsigned long long a;
+    unsigned long long a, b;
 };
 
 __device__ __forceinline__ TilePre tile_pre(const GraphView &g, const unsigned long long *dpre, const TileHead &h,
                                             uint32_t i) {
-    TilePre p{0, 0};
-    if (i <= h.span) {
-        p.ov = g.off[h.v0 + i];
-        p.a = dpre[h.v0 + i];
-    }
-    return p;
+    const uint32_t v = h.v0 + min(i, h.span), w = h.v0 + min(i + 1, h.span);
+    return TilePre{g.off[v], dpre[v], dpre[w]};
 }
 
 // Owners and slot bases of the tile's positions into sh; pre = tile_pre(h,
@@ -607,17 +603,20 @@ __device__ __forceinline__ lds_u32x4 sweep_owners(const GraphView &g, const unsi
     wave_lds_sync();
     const uint64_t off0 = read_lane_u64(pre.ov, 0);
     bool far = false;
-    for (uint32_t i0 = 0; i0 <= span; i0 += kWave) {
-        const uint32_t i = i0 + lane;
-        const TilePre p = i0 == 0 ? pre : tile_pre(g, dpre, h, i);
+    auto source = [&](uint32_t i, const TilePre &p) {
         far |= i <= span && p.ov - off0 >= 0x40000000ull;
-        // end of source i = start of source i + 1 (the next lane, or one more load on the last lane)
-        unsigned long long b = __shfl_down(p.a, 1, kWave);
-        if (lane == kWave - 1 && i < span) b = dpre[v0 + i + 1];
         if (i < span) {
             sh.base[i] = (int32_t)((long long)(p.ov - off0) - (long long)(p.a - e0));
-            if (b > p.a && p.a >= e0 && p.a < e0 + ne) sh.own[p.a - e0] = (uint16_t)i;
+            if (p.b > p.a && p.a >= e0 && p.a < e0 + ne) sh.own[p.a - e0] = (uint16_t)i;
         }
+    };
+    source(lane, pre);
+    for (uint32_t i0 = kWave; i0 <= span; i0 += 4 * kWave) {  // short lists: more sources, 256 in flight
+        TilePre p[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) p[c] = tile_pre(g, dpre, h, i0 + c * kWave + lane);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) source(i0 + c * kWave + lane, p[c]);
     }
     wide = __ballot(far) != 0;
     wave_lds_sync();
@@ -651,23 +650,65 @@ __device__ __forceinline__ void sweep_tile(const GraphView &g, const unsigned lo
     const uint32_t v0 = h.v0, ne = h.ne, b = g.mbits;
     const unsigned long long e0 = h.e0;
     const uint64_t off0 = read_lane_u64(pre.ov, 0);
+#pragma unroll
+    for (int j = 0; j < kSweepPerLane; ++j) vv[j] = kGap;
+    if (h.span == 1 && e0 >= g.mlive) {  // the whole tile lies in one list: consecutive slots, one owner
+        reinterpret_cast<lds_u32x4 *>(sh.own)[lane] = lds_u32x4{0u, 0u, 0u, 0u};
+        if (ne && v0 >= src_lo && v0 < src_hi) {
+            const uint32_t *const cp = colp + (off0 + (e0 - read_lane_u64(pre.a, 0)) - slot_lo);
+            uint32_t x[kSweepPerLane];
+#pragma unroll
+            for (int j = 0; j < kSweepPerLane; ++j) x[j] = cp[min(j * kWave + lane, ne - 1)];
+#pragma unroll
+            for (int j = 0; j < kSweepPerLane; ++j) {
+                vv[j] = j * kWave + lane < ne ? x[j] : kGap;
+                n_edges += j * kWave + lane < ne ? 1u : 0u;
+            }
+        }
+        wave_lds_sync();
+        return;
+    }
     bool wide;
     sweep_owners(g, dpre, h, pre, sh, wide);
+    if (ne == 0) return;
+    if (!wide && e0 >= g.mlive) {
+        // no branch and no wait between the loads: positions past the tile, and
+        // sources out of range, load a slot that exists and drop it (behind a
+        // branch per position the loads could come one at a time: 190 to 330 us
+        // a sweep of 65 M edges, by the compiler's luck)
+        uint64_t slot[kSweepPerLane];
+        bool in[kSweepPerLane];
 #pragma unroll
-    for (int j = 0; j < kSweepPerLane; ++j) {
+        for (int j = 0; j < kSweepPerLane; ++j) {
+            const uint32_t p = j * kWave + lane, q = min(p, ne - 1), o = sh.own[q];
+            in[j] = p < ne && v0 + o >= src_lo && v0 + o < src_hi;
+            slot[j] = in[j] ? off0 + (uint64_t)((long long)sh.base[o] + (long long)q) - slot_lo : 0ull;
+        }
+        uint32_t x[kSweepPerLane];
+#pragma unroll
+        for (int j = 0; j < kSweepPerLane; ++j) x[j] = colp[slot[j]];
+#pragma unroll
+        for (int j = 0; j < kSweepPerLane; ++j) {
+            vv[j] = in[j] ? x[j] : kGap;
+            n_edges += in[j] ? 1u : 0u;
+        }
+        return;
+    }
+    for (int j = 0; j < kSweepPerLane; ++j) {  // a tile with edges in the mirror, or a slot range past 32 bits
         const uint32_t p = j * kWave + lane;
-        vv[j] = kGap;
+        uint32_t x = kGap;
         if (p < ne) {
-            const uint32_t o = sh.own[p];
-            const uint32_t src = v0 + o;
+            const uint32_t o = sh.own[p], src = v0 + o;
             if (src >= src_lo && src < src_hi) {
                 ++n_edges;
                 const uint64_t slot = !wide ? off0 + (uint64_t)((long long)sh.base[o] + (long long)p)
                                             : g.off[src] + (e0 + p - dpre[src]);
                 const unsigned long long k = e0 + p;
-                vv[j] = k < g.mlive ? packed_at(g.mirror, k, b) : colp[slot - slot_lo];
+                x = k < g.mlive ? packed_at(g.mirror, k, b) : colp[slot - slot_lo];
             }
         }
+#pragma unroll
+        for (int i = 0; i < kSweepPerLane; ++i) vv[i] = i == j ? x : vv[i];
     }
 }
 
@@ -688,7 +729,7 @@ struct TileWalk {
         group = blockIdx.x % ngroups;
         const uint32_t blocks = gridDim.x / ngroups;
         // consecutive waves of a group on different CUs
-        k = (unsigned long long)(threadIdx.x / kWave) * blocks + blockIdx.x / ngroups;
+        k = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)) * blocks + blockIdx.x / ngroups;
         step = blocks * waves;
     }
     __device__ __forceinline__ unsigned long long at(unsigned long long i) const {
@@ -777,7 +818,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_edges(GraphView g, const 
         tp.advance(g, dpre, tiles);
         bool pass[kSweepPerLane];
 #pragma unroll
-        for (int j = 0; j < kSweepPerLane; ++j) pass[j] = vv[j] != kGap && coarse_test(s_filter, cs, vv[j]);
+        for (int j = 0; j < kSweepPerLane; ++j) pass[j] = coarse_test(s_filter, cs, vv[j] != kGap ? vv[j] : 0u) && vv[j] != kGap;
         decltype(efn.load(0u)) peek[kSweepPerLane];
 #pragma unroll
         for (int j = 0; j < kSweepPerLane; ++j) peek[j] = pass[j] ? efn.load(vv[j]) : 0;
