@@ -82,6 +82,9 @@ public:
     std::unique_ptr<GraphStore> rev_;
     float *pv_[2] = {nullptr, nullptr};
     float *accg_ = nullptr;
+    PrSums *sums_ = nullptr;  // [3] rotating, as the round counters
+    PrPace *pace_ = nullptr;  // [2]
+    static constexpr size_t kPaceBytes = 3 * sizeof(PrSums) + 2 * sizeof(PrPace);
 
     uint64_t aux_device_bytes() const override { return rev_ ? rev_->dev_bytes_ : 0; }
     uint64_t aux_host_bytes() const override { return rev_ ? rev_->host_bytes_ : 0; }
@@ -108,6 +111,10 @@ public:
         }
         accg_ = dalloc<float>(nv_);
         fill<uint32_t>((uint32_t *)accg_, nv_, 0u);
+        if (!streams) {  // host-driven rounds (streamed pulls) are plain
+            sums_ = (PrSums *)dalloc<unsigned long long>(kPaceBytes / 8);
+            pace_ = (PrPace *)(sums_ + 3);
+        }
         sync();
     }
 
@@ -143,6 +150,13 @@ public:
         p.stamp = stamp_;
         p.hot = ((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nv_, ne_ / (kPrHotEdges * pr_grid()))) + 3u) & ~3u;
         p.host_waves64 = kHostWaves64;
+        if (pace_) {
+            p.sums_in = sums_ + (R % 3);
+            p.sums_out = sums_ + ((R + 1) % 3);
+            p.sums_zero = sums_ + ((R + 2) % 3);
+            p.pace_in = pace_ + (R & 1);
+            p.pace_out = pace_ + ((R + 1) & 1);
+        }
         return p;
     }
     PassIO pr_io(PassIO io) const {
@@ -360,6 +374,7 @@ public:
     void seed() {
         frontier_reset();
         if (pulls()) {
+            if (pace_) fill<unsigned long long>((unsigned long long *)sums_, kPaceBytes / 8, 0ull);
             PassIO io = base_io();
             io.ecnt_out = ecnt_ + (R_ % 3);
             hipLaunchKernelGGL(k_pr_seed<kBothSigns>, dim3(pr_grid()), dim3(kPrBlock), 0, stream_, nv_, pr_state(R_ - 1), io);

@@ -219,6 +219,45 @@ __device__ __forceinline__ float pr_eps(const api::PageRank &op, int mode) {
     return mode == kPrAccum ? __builtin_huge_valf() : (float)op.m_error;
 }
 
+// ---- fewer rounds: the slow part of the residual taken in one step ------------------
+// A round that takes d and delivers alpha * d / outdeg leaves
+//     residual = (1 - alpha) - (I - A) value
+// whatever d is, so a round may take more of a residual than is there. Plain
+// rounds (d = r) shrink the residual by alpha a round at best: its part along
+// the graph's dominant eigenvector, eigenvalue l, shrinks by l only (R-MAT:
+// 0.84), everything else much faster (0.2 to 0.4). Taking d = r / (1 - l) once
+// removes that part and leaves the rest a few times larger, which two or three
+// plain rounds make good. l is what the sums of the residuals taken in
+// successive rounds show. Rounds of a static solve of R-MAT graphs of 2^14 to
+// 2^18 vertices: 91 dense ones without, 17 with; of a snapshot: 41 and 16; the
+// error against 64 bits is a fifth (solve) and the same (snapshot).
+//
+// A step is taken when two successive ratios agree (the dominant part leads),
+// kPrStepWait rounds after the last one (their plain rounds shrink what the
+// step enlarged), and only while each step finds half of the residual the one
+// before it found: so there are finitely many, and plain rounds between them
+// converge as ever. One that left more than plain rounds would have (a graph
+// with more than one slow part: a tree, a star) is the last: such graphs take
+// 10 to 20 rounds more than without.
+constexpr uint32_t kPrStepWait = 5;
+constexpr double kPrStepAgree = 0.3;   // ratios may differ by this share of 1 - l
+// Sums over the residuals that one round took (of their magnitudes: mag).
+struct PrSums {
+    double sum, mag;
+};
+// What a round hands the next (all zero before the first).
+struct PrPace {
+    double sum;      // of the frontier before this one
+    double ratio;    // of that one's sum to the one's before
+    double found;    // magnitude at the last step (0: none yet)
+    double bound;    // what plain rounds would have left of it by now
+    double l;        // the last step's l
+    uint32_t since;  // rounds since then, or since the first
+    uint32_t off;    // no more steps
+    uint32_t pull;   // the frontier was taken in a step: only a pull finds what the step left behind
+    uint32_t pad;
+};
+
 struct PrState {
     api::PageRank op;
     float *value, *res;             // committed ranks, residuals
@@ -235,12 +274,19 @@ struct PrState {
     // waves take those, the others the tiles in HBM, so that both run at once
     // instead of every wave stalling on the host link in turn.
     uint32_t host_waves64;
+    // sums of this round's frontier, of the next (added to), of a later one (to
+    // clear); pace of this round and the next. null: plain rounds.
+    const PrSums *sums_in;
+    PrSums *sums_out, *sums_zero;
+    const PrPace *pace_in;
+    PrPace *pace_out;
 };
 
 // What a thread took: sources and their out-edges.
 struct PrTaken {
     uint32_t n = 0;
     unsigned long long edges = 0;
+    float sum = 0.0f, mag = 0.0f;
 };
 
 // A destination's words.
@@ -252,27 +298,30 @@ __device__ __forceinline__ PrDest pr_dest(const PrState &p, uint32_t v) {
     return PrDest{p.res[v], p.value[v], p.deg[v], p.relabel[v]};
 }
 // CombineValueBuffer (hybrid_pr.cu:66-85) on a residual already known: commit
-// it and record the push of the next round.
-__device__ __forceinline__ void pr_take(const PrState &p, uint32_t v, float r, const PrDest &d, PrTaken &tk) {
-    p.value[v] = d.value + r;
-    p.res[v] = 0.0f;
-    if (d.deg == 0) return;  // dangling: mass dropped
-    const float push = (float)(p.op.m_alpha * (double)r / (double)d.deg);
+// it and record the push of the next round. step: the multiple of r to take.
+__device__ __forceinline__ void pr_take(const PrState &p, uint32_t v, float r, const PrDest &d, float step, PrTaken &tk) {
+    float x = step * r;
+    float push = d.deg ? (float)(p.op.m_alpha * (double)x / (double)d.deg) : 0.0f;
+    if (push == 0.0f) x = r;  // dangling: mass dropped, nothing comes back
+    p.value[v] = d.value + x;
+    p.res[v] = r - x;
     if (push == 0.0f) return;
     p.pv_out[d.rank] = push;
     ++tk.n;
     tk.edges += d.deg;
+    tk.sum += r;
+    tk.mag += fabsf(r);
 }
 // total: what v's in-edges delivered this round. cut: the list goes on in
 // another tile; k_pr_tail finishes v from the partial sums.
 __device__ __forceinline__ void pr_finish(const PrState &p, uint32_t v, float total, bool cut, const PrDest &d, float eps,
-                                          PrTaken &tk) {
+                                          float step, PrTaken &tk) {
     if (cut) {
         if (total != 0.0f) unsafeAtomicAdd(&p.accg[v], total);
         return;
     }
     const float r = total != 0.0f ? d.res + total : d.res;
-    if (fabsf(r) > eps) pr_take(p, v, r, d, tk);
+    if (fabsf(r) > eps) pr_take(p, v, r, d, step, tk);
     else if (total != 0.0f) p.res[v] = r;
 }
 
@@ -281,10 +330,13 @@ template <int kWaves>
 __device__ __forceinline__ void pr_count(const PrTaken &tk, const PrState &p, const PassIO &io,
                                          unsigned long long (*red)[4]) {
     const unsigned long long n = wave_sum_u64(tk.n), e = wave_sum_u64(tk.edges);
+    const float s = wave_sum_f32(tk.sum), m = wave_sum_f32(tk.mag);
     const uint32_t w = threadIdx.x / kWave;
     if (lane_id() == 0) {
         red[w][0] = n;
         red[w][1] = e;
+        red[w][2] = (unsigned long long)__double_as_longlong((double)s);
+        red[w][3] = (unsigned long long)__double_as_longlong((double)m);
     }
     __syncthreads();
     if (threadIdx.x < 2) {
@@ -294,6 +346,10 @@ __device__ __forceinline__ void pr_count(const PrTaken &tk, const PrState &p, co
             if (threadIdx.x == 0) atomicAdd(p.cnt_out, (uint32_t)t);
             else atomicAdd(io.ecnt_out, t);
         }
+    } else if (threadIdx.x < 4 && p.sums_out) {
+        double t = 0.0;
+        for (int i = 0; i < kWaves; ++i) t += __longlong_as_double((long long)red[i][threadIdx.x]);
+        if (t != 0.0) unsafeAtomicAdd(threadIdx.x == 2 ? &p.sums_out->sum : &p.sums_out->mag, t);
     }
 }
 
@@ -329,12 +385,39 @@ struct VPrRanks {
 struct PrRound {
     uint32_t n_list, n_pv;
     bool idle, dense, pull;
+    float step = 1.0f;  // the multiple of their residuals that destinations of a pull take
+    PrPace next{};
     __device__ __forceinline__ PrRound(const PrState &p, const PassIO &io, int mode) {
         n_list = mode == kPrAuto ? min(*io.in_cnt, io.in_cap) : 0u;
         n_pv = mode == kPrAuto ? *p.cnt_in : 1u;
         idle = n_list == 0 && n_pv == 0;
         dense = mode != kPrAuto || *io.ecnt_in > io.dense_thr;
+        const bool paced = mode == kPrAuto && p.pace_in;
+        if (paced && p.pace_in->pull) dense = true;
         pull = dense && n_pv != 0;
+        if (paced && !idle) pace(*p.pace_in, *p.sums_in, p.op.m_alpha);
+    }
+    // Frontiers that a push made have no sums: their ratios are 0 and agree with none.
+    __device__ __forceinline__ void pace(const PrPace &a, const PrSums &f, double alpha) {
+        next = a;
+        next.pull = 0;
+        next.since = a.since + 1;
+        next.sum = f.sum;
+        next.ratio = a.sum != 0.0 ? f.sum / a.sum : 0.0;
+        next.bound = a.bound * a.l;
+        if (!pull || a.off || next.since < kPrStepWait) return;
+        if (a.found > 0.0 && f.mag > next.bound) {
+            next.off = 1;
+            return;
+        }
+        const double l = next.ratio;  // an eigenvalue is at most alpha
+        if (!(l > 0.0 && l < 0.5 * (1.0 + alpha)) || !(fabs(l - a.ratio) < kPrStepAgree * (1.0 - l))) return;
+        if (a.found > 0.0 && !(f.mag <= 0.5 * a.found)) return;
+        step = (float)(1.0 / (1.0 - l));
+        next.found = next.bound = f.mag;
+        next.l = l;
+        next.since = 0;
+        next.pull = 1;
     }
 };
 
@@ -376,7 +459,7 @@ __device__ __forceinline__ PullRaw pull_load(const PullPlan &pl, uint64_t t, con
 // (Adding every push to its destination in LDS serialises on the long lists:
 // 64 lanes on one address.)
 __device__ __forceinline__ void pull_tiles(const PullPlan &pl, const PrState &p, TileWalk walk, const float *hot,
-                                           uint32_t nhot, float eps, PullWave &sh, PrTaken &tk) {
+                                           uint32_t nhot, float eps, float step, PullWave &sh, PrTaken &tk) {
     const uint32_t lane = lane_id(), b = pl.bits;
     const uint32_t mask = b == 32 ? ~0u : (1u << b) - 1u, shift = (lane * b) & 31u;
     const uint32_t *const lw = sh.words + ((lane * b) >> 5);  // position 64 * j + lane starts 2 * b * j words on
@@ -434,7 +517,7 @@ __device__ __forceinline__ void pull_tiles(const PullPlan &pl, const PrState &p,
 #pragma unroll
             for (int j = 0; j < kPullPerLane; ++j) s += c[j];
             s = wave_sum_f32(s);
-            if (lane == 0) pr_finish(p, v, s, cur.meta.flags != 0, d, eps, tk);
+            if (lane == 0) pr_finish(p, v, s, cur.meta.flags != 0, d, eps, step, tk);
         } else {
 #pragma unroll
             for (int j = 0; j < kPullPerLane; ++j) acc[j * kWave + lane] = c[j];
@@ -466,10 +549,10 @@ __device__ __forceinline__ void pull_tiles(const PullPlan &pl, const PrState &p,
             for (uint32_t i = lane; i < nl; i += kWave) {
                 const bool cut = (i == 0 && cont) || (i + 1 == nl && (cur.meta.flags & kPullOn));
                 if (i == lane) {
-                    pr_finish(p, v, acc[i], cut, d, eps, tk);
+                    pr_finish(p, v, acc[i], cut, d, eps, step, tk);
                 } else {
                     const uint32_t u = pl.dst[cur.meta.first + i];
-                    pr_finish(p, u, acc[i], cut, pr_dest(p, u), eps, tk);
+                    pr_finish(p, u, acc[i], cut, pr_dest(p, u), eps, step, tk);
                 }
             }
         }
@@ -487,7 +570,7 @@ __device__ __forceinline__ void pull_tiles(const PullPlan &pl, const PrState &p,
 // destinations [dst_lo, dst_hi)), or a device budget that has no room for it.
 __device__ __forceinline__ void pull_slots(const GraphView &rg, const unsigned long long *dpre, const SweepTiles &tiles,
                                            const TileWalk &walk, const uint32_t *colp, uint64_t slot_lo, uint32_t dst_lo,
-                                           uint32_t dst_hi, const PrState &p, const float *hot, uint32_t nhot, float eps,
+                                           uint32_t dst_hi, const PrState &p, const float *hot, uint32_t nhot, float eps, float step,
                                            SweepTileLds &sh, uint32_t &n_edges, PrTaken &tk) {
     const uint32_t lane = lane_id();
     float *const acc = reinterpret_cast<float *>(sh.base);  // base[] is dead once a tile's edges are loaded
@@ -514,7 +597,7 @@ __device__ __forceinline__ void pull_slots(const GraphView &rg, const unsigned l
             const uint32_t v = h.v0 + i;
             if (v < dst_lo || v >= dst_hi) continue;
             const bool cut = i == 0 || i + 1 == h.span;  // the list may go on in a neighbouring tile
-            pr_finish(p, v, acc[i], cut, pr_dest(p, v), eps, tk);
+            pr_finish(p, v, acc[i], cut, pr_dest(p, v), eps, step, tk);
         }
         wave_lds_sync();
     }
@@ -559,6 +642,10 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_step(GraphView g, PullPlan pl, 
         if (io.heavy_zero) *io.heavy_zero = 0;
         if (io.ecnt_zero) *io.ecnt_zero = 0;
         if (p.cnt_zero) *p.cnt_zero = 0;
+        if (mode == kPrAuto && p.pace_out) {
+            *p.sums_zero = PrSums{};
+            *p.pace_out = rd.next;
+        }
         if (io.log) {  // what round R - 1 produced, and whether round R pulls
             io.log[2 * ((io.round + kRoundLog - 1) % kRoundLog)] = rd.n_list + rd.n_pv;
             io.log[2 * (io.round % kRoundLog) + 1] = rd.pull ? 1u : 0u;
@@ -586,13 +673,13 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_step(GraphView g, PullPlan pl, 
                     walk.step -= nh;
                 }
             }
-            pull_tiles(pl, p, walk, sh.hot, nhot, eps, sh.tile[w], tk);
+            pull_tiles(pl, p, walk, sh.hot, nhot, eps, rd.step, sh.tile[w], tk);
         } else {
             const unsigned long long ntiles = (sl.rg.nv + sl.dpre[sl.rg.nv] + kSweepTile - 1) / kSweepTile;
             const TileWalk walk(sl.t_begin, min_u64(min_u64(sl.t_end, ntiles), sl.tiles.cap - 1), kPrWaves);
             uint32_t n_edges = 0;
             pull_slots(sl.rg, sl.dpre, sl.tiles, walk, sl.colp, sl.slot_lo, sl.dst_lo, sl.dst_hi, p, sh.hot, nhot, eps,
-                       sh.tile[w], n_edges, tk);
+                       rd.step, sh.tile[w], n_edges, tk);
             const unsigned long long ne = wave_sum_u64(n_edges);
             if (lane_id() == 0 && ne) atomicAdd(io.stats + 0, ne);
         }
@@ -604,7 +691,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_step(GraphView g, PullPlan pl, 
         for (uint64_t i = gwave * kWave + lane_id(); i < rd.n_list; i += nwaves * kWave) {
             const uint32_t u = io.in_list[i];  // listed once: no other lane holds u
             const PrDest d = pr_dest(p, u);
-            if (d.res != 0.0f) pr_take(p, u, d.res, d, tk);
+            if (d.res != 0.0f) pr_take(p, u, d.res, d, 1.0f, tk);
         }
         pr_count<kPrWaves>(tk, p, io, sh.red);
         return;
@@ -647,7 +734,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_tail(GraphView g, PullPlan pl, 
         auto finish = [&](uint32_t v) {
             const float total = p.accg[v];
             if (total != 0.0f) p.accg[v] = 0.0f;
-            pr_finish(p, v, total, false, pr_dest(p, v), eps, tk);
+            pr_finish(p, v, total, false, pr_dest(p, v), eps, rd.step, tk);
         };
         if constexpr (kPlan) {
             for (uint64_t t = first + 1; t < pl.ntiles; t += stride) {
@@ -693,7 +780,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_seed(uint32_t nv, PrState p, Pa
         const uint32_t v = (uint32_t)i;
         const float r = p.res[v];
         if (p.op.IsActiveNode(v, r, 0.0f) || (kBothSigns && p.op.IsActiveNode_INC(v, r, 0.0f)))
-            pr_take(p, v, r, pr_dest(p, v), tk);
+            pr_take(p, v, r, pr_dest(p, v), 1.0f, tk);
     }
     pr_count<kPrWaves>(tk, p, io, s_red);
 }
