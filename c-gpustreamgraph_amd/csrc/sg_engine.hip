@@ -84,7 +84,7 @@ public:
     float *accg_ = nullptr;
     PrSums *sums_ = nullptr;  // [3] rotating, as the round counters
     PrPace *pace_ = nullptr;  // [2]
-    static constexpr size_t kPaceBytes = 3 * sizeof(PrSums) + 2 * sizeof(PrPace);
+    static constexpr size_t kPaceWords = (3 * sizeof(PrSums) + 2 * sizeof(PrPace)) / 8;  // and the kept l
 
     uint64_t aux_device_bytes() const override { return rev_ ? rev_->dev_bytes_ : 0; }
     uint64_t aux_host_bytes() const override { return rev_ ? rev_->host_bytes_ : 0; }
@@ -112,8 +112,9 @@ public:
         accg_ = dalloc<float>(nv_);
         fill<uint32_t>((uint32_t *)accg_, nv_, 0u);
         if (!streams) {  // host-driven rounds (streamed pulls) are plain
-            sums_ = (PrSums *)dalloc<unsigned long long>(kPaceBytes / 8);
+            sums_ = (PrSums *)dalloc<unsigned long long>(kPaceWords + 1);
             pace_ = (PrPace *)(sums_ + 3);
+            fill<unsigned long long>((unsigned long long *)sums_, kPaceWords + 1, 0ull);
         }
         sync();
     }
@@ -156,7 +157,9 @@ public:
             p.sums_zero = sums_ + ((R + 2) % 3);
             p.pace_in = pace_ + (R & 1);
             p.pace_out = pace_ + ((R + 1) & 1);
+            p.kept = (double *)(pace_ + 2);
         }
+        p.in_deg = rev_->deg_;
         return p;
     }
     PassIO pr_io(PassIO io) const {
@@ -374,7 +377,8 @@ public:
     void seed() {
         frontier_reset();
         if (pulls()) {
-            if (pace_) fill<unsigned long long>((unsigned long long *)sums_, kPaceBytes / 8, 0ull);
+            // a static solve starts from nothing (kBothSigns: a snapshot, which keeps l)
+            if (pace_) fill<unsigned long long>((unsigned long long *)sums_, kPaceWords + (kBothSigns ? 0 : 1), 0ull);
             PassIO io = base_io();
             io.ecnt_out = ecnt_ + (R_ % 3);
             hipLaunchKernelGGL(k_pr_seed<kBothSigns>, dim3(pr_grid()), dim3(kPrBlock), 0, stream_, nv_, pr_state(R_ - 1), io);

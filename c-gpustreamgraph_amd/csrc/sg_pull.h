@@ -229,8 +229,12 @@ __device__ __forceinline__ float pr_eps(const api::PageRank &op, int mode) {
 // removes that part and leaves the rest a few times larger, which two or three
 // plain rounds make good. l is what the sums of the residuals taken in
 // successive rounds show. Rounds of a static solve of R-MAT graphs of 2^14 to
-// 2^18 vertices: 91 dense ones without, 17 with; of a snapshot: 41 and 16; the
+// 2^18 vertices: 91 dense ones without, 17 with; of a snapshot: 41 and 11; the
 // error against 64 bits is a fifth (solve) and the same (snapshot).
+// A snapshot's seed already takes a step, with the l of the last one that did
+// what it should on this engine's graph (a batch hardly changes l; without it
+// a snapshot takes 16 dense rounds). It is a guess like the round count that
+// sizes the batches: it decides how many rounds are run, not where they end.
 //
 // A step is taken when two successive ratios agree (the dominant part leads),
 // kPrStepWait rounds after the last one (their plain rounds shrink what the
@@ -241,6 +245,8 @@ __device__ __forceinline__ float pr_eps(const api::PageRank &op, int mode) {
 // 10 to 20 rounds more than without.
 constexpr uint32_t kPrStepWait = 5;
 constexpr double kPrStepAgree = 0.3;   // ratios may differ by this share of 1 - l
+constexpr double kPrStepLeast = 0.3;   // below this l plain rounds are as fast
+constexpr double kPrStepKeep = 0.5;    // an l above this is kept for the next snapshot's seed
 // Sums over the residuals that one round took (of their magnitudes: mag).
 struct PrSums {
     double sum, mag;
@@ -249,7 +255,7 @@ struct PrSums {
 struct PrPace {
     double sum;      // of the frontier before this one
     double ratio;    // of that one's sum to the one's before
-    double found;    // magnitude at the last step (0: none yet)
+    double found;    // magnitude at the last step (0: none yet; -1: the seed's, not known yet)
     double bound;    // what plain rounds would have left of it by now
     double l;        // the last step's l
     uint32_t since;  // rounds since then, or since the first
@@ -280,6 +286,8 @@ struct PrState {
     PrSums *sums_out, *sums_zero;
     const PrPace *pace_in;
     PrPace *pace_out;
+    double *kept;            // l for the next snapshot's seed (0: none)
+    const uint32_t *in_deg;  // in-degrees
 };
 
 // What a thread took: sources and their out-edges.
@@ -386,6 +394,7 @@ struct PrRound {
     uint32_t n_list, n_pv;
     bool idle, dense, pull;
     float step = 1.0f;  // the multiple of their residuals that destinations of a pull take
+    double keep = -1.0;  // a new kept l (negative: none)
     PrPace next{};
     __device__ __forceinline__ PrRound(const PrState &p, const PassIO &io, int mode) {
         n_list = mode == kPrAuto ? min(*io.in_cnt, io.in_cap) : 0u;
@@ -395,23 +404,28 @@ struct PrRound {
         const bool paced = mode == kPrAuto && p.pace_in;
         if (paced && p.pace_in->pull) dense = true;
         pull = dense && n_pv != 0;
-        if (paced && !idle) pace(*p.pace_in, *p.sums_in, p.op.m_alpha);
+        if (paced && !idle) pace(p, *p.pace_in, *p.sums_in);
     }
     // Frontiers that a push made have no sums: their ratios are 0 and agree with none.
-    __device__ __forceinline__ void pace(const PrPace &a, const PrSums &f, double alpha) {
+    __device__ __forceinline__ void pace(const PrState &p, const PrPace &a, const PrSums &f) {
         next = a;
         next.pull = 0;
         next.since = a.since + 1;
         next.sum = f.sum;
         next.ratio = a.sum != 0.0 ? f.sum / a.sum : 0.0;
         next.bound = a.bound * a.l;
+        if (a.found < 0.0) next.found = next.bound = f.mag;
         if (!pull || a.off || next.since < kPrStepWait) return;
-        if (a.found > 0.0 && f.mag > next.bound) {
-            next.off = 1;
-            return;
+        if (a.found > 0.0) {
+            if (f.mag > next.bound) {
+                next.off = 1;
+                if (*p.kept == a.l) keep = 0.0;
+                return;
+            }
+            if (a.l > kPrStepKeep) keep = a.l;
         }
         const double l = next.ratio;  // an eigenvalue is at most alpha
-        if (!(l > 0.0 && l < 0.5 * (1.0 + alpha)) || !(fabs(l - a.ratio) < kPrStepAgree * (1.0 - l))) return;
+        if (!(l > kPrStepLeast && l < 0.5 * (1.0 + p.op.m_alpha)) || !(fabs(l - a.ratio) < kPrStepAgree * (1.0 - l))) return;
         if (a.found > 0.0 && !(f.mag <= 0.5 * a.found)) return;
         step = (float)(1.0 / (1.0 - l));
         next.found = next.bound = f.mag;
@@ -645,6 +659,7 @@ __global__ void __launch_bounds__(kPrBlock) k_pr_step(GraphView g, PullPlan pl, 
         if (mode == kPrAuto && p.pace_out) {
             *p.sums_zero = PrSums{};
             *p.pace_out = rd.next;
+            if (rd.keep >= 0.0) *p.kept = rd.keep;
         }
         if (io.log) {  // what round R - 1 produced, and whether round R pulls
             io.log[2 * ((io.round + kRoundLog - 1) % kRoundLog)] = rd.n_list + rd.n_pv;
@@ -776,11 +791,21 @@ template <bool kBothSigns>
 __global__ void __launch_bounds__(kPrBlock) k_pr_seed(uint32_t nv, PrState p, PassIO io) {
     __shared__ unsigned long long s_red[kPrWaves][4];
     PrTaken tk;
+    const double l = kBothSigns && p.pace_out ? *p.kept : 0.0;
+    const float step = (float)(1.0 / (1.0 - l));
+    if (l > 0.0 && blockIdx.x == 0 && threadIdx.x == 0) {
+        PrPace a{};
+        a.l = l;
+        a.found = -1.0;
+        a.pull = 1;
+        *p.pace_out = a;
+    }
     for (uint64_t i = (uint64_t)blockIdx.x * kPrBlock + threadIdx.x; i < nv; i += (uint64_t)gridDim.x * kPrBlock) {
         const uint32_t v = (uint32_t)i;
         const float r = p.res[v];
         if (p.op.IsActiveNode(v, r, 0.0f) || (kBothSigns && p.op.IsActiveNode_INC(v, r, 0.0f)))
-            pr_take(p, v, r, pr_dest(p, v), 1.0f, tk);
+            // no pull comes to a vertex without in-edges: nothing of it may be left
+            pr_take(p, v, r, pr_dest(p, v), p.in_deg[v] ? step : 1.0f, tk);
     }
     pr_count<kPrWaves>(tk, p, io, s_red);
 }
