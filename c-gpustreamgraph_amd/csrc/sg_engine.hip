@@ -495,8 +495,7 @@ public:
         if (q == SG_Q_VALUE || q == SG_Q_BUFFER) {
             if (!value_) fail(SG_EINVAL, "no vertex state before sg_init");
             if (bytes < (size_t)nv_ * 4) fail(SG_EINVAL, "output too small");
-            SG_HIP(hipMemcpyAsync(out, q == SG_Q_VALUE ? value_ : buffer_, (size_t)nv_ * 4, hipMemcpyDeviceToHost, stream_));
-            sync();
+            read_back(out, q == SG_Q_VALUE ? value_ : buffer_, (size_t)nv_ * 4);
             return;
         }
         if (q == SG_Q_PARENT) {
@@ -866,8 +865,7 @@ public:
         hipLaunchKernelGGL(k_mextract, dim3(grid_for(nv_, 256, 16384)), dim3(256), 0, stream_, nv_,
                            (const unsigned long long *)best_, KP_, qi, tmp_, what == SG_Q_PARENT ? 1 : 0);
         SG_LAUNCHED();
-        SG_HIP(hipMemcpyAsync(out, tmp_, (size_t)nv_ * 4, hipMemcpyDeviceToHost, stream_));
-        sync();
+        read_back(out, tmp_, (size_t)nv_ * 4);
     }
 
     void word_source(uint32_t q, uint32_t qi, const uint32_t *&base, uint64_t &stride, uint32_t &word) override {

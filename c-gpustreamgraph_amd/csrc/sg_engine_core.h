@@ -21,6 +21,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <tuple>
 #include <type_traits>
@@ -768,6 +769,12 @@ public:
         release_graphs();
         for (auto &ev : events_) { (void)hipEventDestroy(ev.first); (void)hipEventDestroy(ev.second); }
         events_.clear();
+        for (auto &ev : rb_ev_) {
+            if (ev) (void)hipEventDestroy(ev);
+            ev = nullptr;
+        }
+        if (rb_) (void)hipHostFree(rb_);
+        rb_ = nullptr;
         if (pinned_) (void)hipHostFree(pinned_);
         pinned_ = nullptr;
         if (stream_ && own_stream_) (void)hipStreamDestroy(stream_);
@@ -955,6 +962,79 @@ public:
         }
     }
 
+    // Device words to the caller's memory, waited for. A copy of megabytes into
+    // pageable memory runs at what one core gets through page faults and a
+    // copy: chunks go to pinned staging, and threads take them from there while
+    // the next are on the link. 16 MB into pages already touched 950 -> 590 us,
+    // into new ones 1880 -> 810 us (the link alone: 300); chunks of 512 KiB 805
+    // and 965 us (a copy's start), 2 and 8 threads 20 to 30 % more on new pages.
+    // Below 2 MB the threads' start costs as much as they save.
+    static constexpr size_t kReadChunk = 1 << 20, kReadSlots = 8, kReadLeast = 2 << 20;
+    static constexpr uint32_t kReadThreads = 4;
+    char *rb_ = nullptr;
+    hipEvent_t rb_ev_[kReadSlots] = {};
+    void read_back(void *out, const void *src, size_t bytes) {
+        struct Readers {
+            std::atomic<size_t> next{0}, ready{0};  // chunks claimed, chunks in staging
+            std::atomic<bool> stop{false};
+            std::vector<std::thread> th;
+            ~Readers() {
+                stop = true;
+                for (auto &t : th) t.join();
+            }
+        };
+        const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
+        std::vector<std::atomic<uint8_t>> taken(rb_ && bytes >= kReadLeast ? n : 0);
+        auto take = [&, this](Readers &r) {
+            for (size_t i = r.next++; i < n; i = r.next++) {
+                while (r.ready.load(std::memory_order_acquire) <= i) {
+                    if (r.stop) return;
+                    __builtin_ia32_pause();
+                }
+                std::memcpy((char *)out + i * kReadChunk, rb_ + i % kReadSlots * kReadChunk,
+                            std::min(kReadChunk, bytes - i * kReadChunk));
+                taken[i].store(1, std::memory_order_release);
+            }
+        };
+        Readers r;
+        if (!taken.empty()) {
+            try {
+                for (uint32_t t = 0; t < kReadThreads && t < n; ++t) r.th.emplace_back([&] { take(r); });
+            } catch (const std::system_error &) {  // no more threads: those there are do
+            }
+        }
+        if (r.th.empty()) {
+            SG_HIP(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream_));
+            sync();
+            return;
+        }
+        for (size_t sent = 0, got = 0; got < n;) {
+            while (sent < n && (sent < kReadSlots || taken[sent - kReadSlots].load(std::memory_order_acquire))) {
+                SG_HIP(hipMemcpyAsync(rb_ + sent % kReadSlots * kReadChunk, (const char *)src + sent * kReadChunk,
+                                      std::min(kReadChunk, bytes - sent * kReadChunk), hipMemcpyDeviceToHost, stream_));
+                SG_HIP(hipEventRecord(rb_ev_[sent % kReadSlots], stream_));
+                ++sent;
+            }
+            if (got == sent) continue;
+            const hipError_t e = hipEventQuery(rb_ev_[got % kReadSlots]);
+            if (e == hipSuccess) r.ready.store(++got, std::memory_order_release);
+            else if (e != hipErrorNotReady) SG_HIP(e);
+        }
+        take(r);
+        for (auto &t : r.th) t.join();
+        r.th.clear();
+    }
+    // The staging of read_back, for engines whose results are that long (without it copies are plain).
+    void read_staging(size_t bytes) {
+        if (bytes < kReadLeast || rb_) return;
+        if (hipHostMalloc((void **)&rb_, kReadSlots * kReadChunk, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            rb_ = nullptr;
+            return;
+        }
+        for (auto &ev : rb_ev_) SG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    }
+
     template <class T>
     void fill(T *p, uint64_t n, T v) {
         if (n == 0) return;
@@ -1119,6 +1199,7 @@ public:
         st_.capacity = cap_;
         st_.host_edges = host_edges_ ? 1 : 0;
         st_.cache_slots = cache_slots_;
+        if (has_rounds()) read_staging((size_t)nv_ * 4);
         after_load(row, col);
     }
     // Stores an engine keeps beside its PMA (PageRank's in-edge store) are
@@ -1563,10 +1644,15 @@ public:
     // ---- batch prepare / commit -------------------------------------------------------
     void stage_host_batch(const uint32_t *ins, uint64_t nins, const uint32_t *del, uint64_t ndel,
                           const uint32_t *&d_ins, const uint32_t *&d_del) {
-        for (uint64_t i = 0; i < 2 * nins; ++i)
-            if (ins[i] >= nv_) fail(SG_EINVAL, "insert pair " + std::to_string(i / 2) + " has an id >= nv");
-        for (uint64_t i = 0; i < 2 * ndel; ++i)
-            if (del[i] >= nv_) fail(SG_EINVAL, "delete pair " + std::to_string(i / 2) + " has an id >= nv");
+        auto check = [&](const uint32_t *ids, uint64_t n, const char *what) {
+            uint32_t most = 0;  // (a loop without an exit: four ids at a time)
+            for (uint64_t i = 0; i < n; ++i) most = std::max(most, ids[i]);
+            if (most < nv_) return;
+            for (uint64_t i = 0; i < n; ++i)
+                if (ids[i] >= nv_) fail(SG_EINVAL, what + std::string(" pair ") + std::to_string(i / 2) + " has an id >= nv");
+        };
+        check(ins, 2 * nins, "insert");
+        check(del, 2 * ndel, "delete");
         ensure(raw_ins_, raw_ins_cap_, 2 * nins + 2);
         ensure(raw_del_, raw_del_cap_, 2 * ndel + 2);
         if (nins) SG_HIP(hipMemcpyAsync(raw_ins_, ins, 2 * nins * sizeof(uint32_t), hipMemcpyHostToDevice, stream_));
@@ -2050,10 +2136,10 @@ public:
     void gather_graph(uint32_t q, void *out, size_t bytes) {
         if (q == SG_Q_DEGREE) {
             if (bytes < (size_t)nv_ * 4) fail(SG_EINVAL, "output too small");
-            SG_HIP(hipMemcpyAsync(out, deg_, (size_t)nv_ * 4, hipMemcpyDeviceToHost, stream_));
+            read_back(out, deg_, (size_t)nv_ * 4);
         } else if (q == SG_Q_OFFSETS) {
             if (bytes < ((size_t)nv_ + 1) * 8) fail(SG_EINVAL, "output too small");
-            SG_HIP(hipMemcpyAsync(out, off_, ((size_t)nv_ + 1) * 8, hipMemcpyDeviceToHost, stream_));
+            read_back(out, off_, ((size_t)nv_ + 1) * 8);
         } else if (q == SG_Q_SLOTS) {
             if (bytes < (size_t)cap_ * 4) fail(SG_EINVAL, "output too small");
             SG_HIP(hipMemcpyAsync(out, col_, (size_t)cap_ * 4, hipMemcpyDefault, stream_));
@@ -2754,15 +2840,14 @@ struct TravProgram {
         if (!value) fail(SG_EINVAL, "no vertex state before sg_init");
         if (bytes < (size_t)e.nv_ * 4) fail(SG_EINVAL, "output too small");
         if (q == SG_Q_VALUE) {
-            SG_HIP(hipMemcpyAsync(out, value, (size_t)e.nv_ * 4, hipMemcpyDeviceToHost, e.stream_));
+            e.read_back(out, value, (size_t)e.nv_ * 4);
         } else {
             e.ensure(e.tmp_, e.tmp_cap_, e.nv_);
             hipLaunchKernelGGL(k_extract<Op>, dim3(grid_for(e.nv_, 256, 16384)), dim3(256), 0, e.stream_, e.nv_, buffer, e.tmp_,
                                q == SG_Q_BUFFER ? 1 : 0);
             SG_LAUNCHED();
-            SG_HIP(hipMemcpyAsync(out, e.tmp_, (size_t)e.nv_ * 4, hipMemcpyDeviceToHost, e.stream_));
+            e.read_back(out, e.tmp_, (size_t)e.nv_ * 4);
         }
-        e.sync();
     }
 };
 

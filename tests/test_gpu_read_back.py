@@ -1,0 +1,38 @@
+"""Results read through pinned staging: whole at the sizes where the chunks can go wrong.
+
+Chunks of 1 MiB through eight staging slots from 2 MiB on: a result just below,
+at and above a chunk and above the slots, read twice into fresh memory.
+Degrees are known without the device; OFFSETS are 8-byte words.
+"""
+import numpy as np
+import pytest
+
+import sgraph
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 18  # 4-byte words
+
+
+@pytest.mark.parametrize("nv", [2 * MB - 1, 2 * MB, 2 * MB + 1, 3 * MB, 8 * MB + 1, 9 * MB - 3, 17 * MB + 5])
+def test_results_come_whole(nv):
+    rng = np.random.default_rng(nv)
+    deg = rng.integers(0, 3, nv).astype(np.uint32)
+    row = np.zeros(nv + 1, np.uint64)
+    np.cumsum(deg, out=row[1:])
+    u = np.repeat(np.arange(nv, dtype=np.int64), deg)
+    k = np.arange(len(u)) - row[u].astype(np.int64)
+    col = ((u + 1 + k) % nv).astype(np.uint32)
+    eng = sgraph.Engine("cc")
+    try:
+        eng.load_csr(row, col)
+        for _ in range(2):
+            assert np.array_equal(eng.gather(sgraph.Q_DEGREE), deg)
+        off = eng.gather(sgraph.Q_OFFSETS)
+        assert off[-1] == eng.stats()["capacity"] and np.all(np.diff(off.astype(np.int64)) >= deg)
+        eng.init()
+        a = eng.values()
+        b = eng.gather_at(np.arange(nv, dtype=np.uint32))
+        assert np.array_equal(a, b)
+    finally:
+        eng.close()
