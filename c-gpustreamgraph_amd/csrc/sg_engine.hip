@@ -320,13 +320,12 @@ public:
     }
 
     void residual() {
-        SG_HIP(hipMemsetAsync(d_sum_, 0, 2 * sizeof(double), stream_));
+        fill<unsigned long long>((unsigned long long *)d_sum_, 2, 0ull);
         hipLaunchKernelGGL(k_pr_residual, dim3(grid_for(nv_, kBlock, 2048)), dim3(kBlock), 0, stream_, nv_, buffer_, d_sum_,
                            (unsigned long long *)(d_sum_ + 1));
         SG_LAUNCHED();
         double h[2];
-        SG_HIP(hipMemcpyAsync(h_u64_, d_sum_, 2 * sizeof(double), hipMemcpyDeviceToHost, stream_));
-        sync();
+        publish(h_u64_, d_sum_, 2 * sizeof(double));
         std::memcpy(h, h_u64_, sizeof h);
         st_.pr_residual_l1 = h[0];
         st_.pr_residual_max = h[1];

@@ -609,6 +609,38 @@ __global__ void k_extract(uint32_t nv, const typename Op::buffer_t *buffer, uint
         out[v] = hi ? (uint32_t)(buffer[v] >> 32) : (uint32_t)buffer[v];
 }
 
+// Words the host waits for: every block has stored its part into pinned memory
+// (any thread, before the call); the last one to arrive sets *word to val.
+// count: a zero word in device memory, zero again after.
+struct HostSignal {
+    uint32_t *word, *count;
+    uint32_t val;
+};
+__device__ __forceinline__ void signal_host(const HostSignal &s) {
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (atomicAdd(s.count, 1u) + 1 != gridDim.x) return;
+    *s.count = 0;
+    __threadfence_system();
+    __hip_atomic_store(s.word, s.val, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// n words to pinned memory.
+__global__ void __launch_bounds__(256) k_publish(const uint32_t *src, uint32_t n, uint32_t *dst, HostSignal s) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+    signal_host(s);
+}
+// k_gather_words with the ids read from pinned memory and the results stored there.
+__global__ void __launch_bounds__(256) k_gather_publish(const uint32_t *base, uint64_t stride, uint32_t word, uint32_t nv,
+                                                        const uint32_t *verts, uint32_t n, uint32_t *out, HostSignal s) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const uint32_t v = verts[i];
+        out[i] = v < nv ? base[(uint64_t)v * stride + word] : 0xFFFFFFFFu;
+    }
+    signal_host(s);
+}
+
 // Pointwise gather: out[i] = 32-bit word base[verts[i] * stride + word].
 __global__ void k_gather_words(const uint32_t *base, uint64_t stride, uint32_t word, uint32_t nv, const uint32_t *verts,
                                uint64_t n, uint32_t *out) {
@@ -895,6 +927,12 @@ public:
     Ctl *h_ctl_ = nullptr;
     uint32_t *h_blk_ = nullptr;   // host copy of the control block
     unsigned long long *h_u64_ = nullptr;  // [16]
+    uint32_t *h_word_ = nullptr;  // the last signal a kernel sent (HostSignal)
+    uint32_t *h_small_ = nullptr;  // [kSmallWords] ids and results of short reads
+    uint32_t *sig_count_ = nullptr;
+    uint32_t sig_ = 0;
+    static constexpr uint32_t kSmallWords = 128 << 10;
+    static constexpr size_t kPinnedBytes = 65536 + kSmallWords * 4;
     const unsigned long long *h_stats() const { return (const unsigned long long *)(h_blk_ + 8 + 2 * kRoundLog); }
     const unsigned long long *h_ecnt() const { return h_stats() + 16; }
     const uint32_t *h_pcnt() const { return (const uint32_t *)(h_ecnt() + 4); }
@@ -943,10 +981,43 @@ public:
             scratch_ = g_scratch_addr[cfg_.device];
         }
         SG_HIP(hipEventCreateWithFlags(&sync_ev_, hipEventDisableTiming));
-        SG_HIP(hipHostMalloc(&pinned_, 65536, hipHostMallocDefault));
+        SG_HIP(hipHostMalloc(&pinned_, kPinnedBytes, hipHostMallocMapped | hipHostMallocCoherent));
+        void *dp = nullptr;
+        SG_HIP(hipHostGetDevicePointer(&dp, pinned_, 0));
+        if (dp != pinned_) fail(SG_EDEVICE, "pinned host memory is not addressable by the device at its host address");
         h_ctl_ = (Ctl *)pinned_;
         h_blk_ = (uint32_t *)((char *)pinned_ + 4096);
         h_u64_ = (unsigned long long *)((char *)pinned_ + 16384);
+        h_word_ = (uint32_t *)((char *)pinned_ + 32768);
+        h_small_ = (uint32_t *)((char *)pinned_ + 65536);
+        *h_word_ = 0;
+        sig_count_ = dalloc<uint32_t>(1);
+        fill<uint32_t>(sig_count_, 1, 0u);
+    }
+    HostSignal next_signal() { return HostSignal{h_word_, sig_count_, ++sig_}; }
+    // Until the stream's last kernel has sent the signal.
+    void wait_signal() {
+        for (uint32_t spin = 1;; ++spin) {
+            if (__atomic_load_n(h_word_, __ATOMIC_ACQUIRE) == sig_) return;
+            __builtin_ia32_pause();
+            if (spin % 16384) continue;
+            const hipError_t e = hipStreamQuery(stream_);  // a fault would send no signal
+            if (e == hipErrorNotReady) continue;
+            SG_HIP(e);
+            if (__atomic_load_n(h_word_, __ATOMIC_ACQUIRE) == sig_) return;
+            fail(SG_EDEVICE, "the device finished without a signal");
+        }
+    }
+    // Words in device memory to dst in the pinned block, waited for. The kernel
+    // that copies them also stores the word the host polls: a copy, an event
+    // and its query took 10 us more per wait, and a snapshot waits three to
+    // six times.
+    void publish(void *dst, const void *src, size_t bytes) {
+        const uint32_t n = (uint32_t)(bytes / 4);
+        hipLaunchKernelGGL(k_publish, dim3(grid_for(n, 1024, 128)), dim3(256), 0, stream_, (const uint32_t *)src, n,
+                           (uint32_t *)dst, next_signal());
+        SG_LAUNCHED();
+        wait_signal();
     }
 
     // Wait for the stream by polling an event: the host resumes as soon as the
@@ -1002,6 +1073,11 @@ public:
                 for (uint32_t t = 0; t < kReadThreads && t < n; ++t) r.th.emplace_back([&] { take(r); });
             } catch (const std::system_error &) {  // no more threads: those there are do
             }
+        }
+        if (r.th.empty() && bytes <= kSmallWords * 4 && bytes % 4 == 0) {
+            publish(h_small_, src, bytes);
+            std::memcpy(out, h_small_, bytes);
+            return;
         }
         if (r.th.empty()) {
             SG_HIP(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream_));
@@ -1495,6 +1571,7 @@ public:
 
     // Harvest kernel timings of completed events (call after a sync).
     void harvest_events() {
+        if (ev_used_) sync();  // a signal says that the kernels are done, not that their events are
         for (size_t i = 0; i < ev_used_; ++i) {
             float ms = 0.f;
             SG_HIP(hipEventElapsedTime(&ms, events_[i].first, events_[i].second));
@@ -1511,8 +1588,7 @@ public:
 
     // Copy the control block to the host and wait.
     void read_block() {
-        SG_HIP(hipMemcpyAsync(h_blk_, cnt_, kCtlBlockBytes, hipMemcpyDeviceToHost, stream_));
-        sync();
+        publish(h_blk_, cnt_, kCtlBlockBytes);
     }
 
     // Run rounds from the frontier of round R_ until a round activates nothing
@@ -1780,8 +1856,7 @@ public:
                                reads_old_lists() ? 0 : 1, &ctl_->pad[1]);
             SG_LAUNCHED();
             if (host_edges_) {  // HBM holds only what this batch stages, not a copy of the edge array
-                SG_HIP(hipMemcpyAsync(h_ctl_, ctl_, sizeof(Ctl), hipMemcpyDeviceToHost, stream_));
-                sync();
+                publish(h_ctl_, ctl_, sizeof(Ctl));
                 ensure(tmp_, tmp_cap_, std::max<uint64_t>(h_ctl_->seqcur, 1));
             }
             begin_timed(timing(SG_KCLASS_MERGE), SG_KCLASS_MERGE);
@@ -1797,8 +1872,7 @@ public:
                                tinfo_, &ctl_->tcount, cpos_, newdeg_, leaf_dirty_, L_, leaf_cnt_, ctl_);
             SG_LAUNCHED();
         }
-        SG_HIP(hipMemcpyAsync(h_ctl_, ctl_, sizeof(Ctl), hipMemcpyDeviceToHost, stream_));
-        sync();
+        publish(h_ctl_, ctl_, sizeof(Ctl));
         if (h_ctl_->pad[0] || h_ctl_->pad[1]) fail(SG_EDEVICE, "internal touched/chunk list overflow");
         st_.dropped_updates += h_ctl_->dropped;
         return h_ctl_->overflow != 0;
@@ -2123,6 +2197,16 @@ public:
         uint64_t stride = 1;
         uint32_t word = 0;
         word_source(q, qi, base, stride, word);
+        if (n <= kSmallWords / 2) {
+            // no copies: 4096 ids 30 us with one each way and an event
+            std::memcpy(h_small_, verts, n * 4);
+            hipLaunchKernelGGL(k_gather_publish, dim3(grid_for(n, 256, 256)), dim3(256), 0, stream_, base, stride, word, nv_,
+                               (const uint32_t *)h_small_, (uint32_t)n, h_small_ + kSmallWords / 2, next_signal());
+            SG_LAUNCHED();
+            wait_signal();
+            std::memcpy(out, h_small_ + kSmallWords / 2, n * 4);
+            return;
+        }
         ensure(gat_v_, gat_v_cap_, n);
         ensure(gat_o_, gat_o_cap_, n);
         SG_HIP(hipMemcpyAsync(gat_v_, verts, n * 4, hipMemcpyHostToDevice, stream_));

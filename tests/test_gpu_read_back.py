@@ -2,7 +2,8 @@
 
 Chunks of 1 MiB through eight staging slots from 2 MiB on: a result just below,
 at and above a chunk and above the slots, read twice into fresh memory.
-Degrees are known without the device; OFFSETS are 8-byte words.
+Degrees are known without the device; OFFSETS are 8-byte words. Pointwise reads
+of up to 65536 ids go through pinned words without copies.
 """
 import numpy as np
 import pytest
@@ -34,5 +35,26 @@ def test_results_come_whole(nv):
         a = eng.values()
         b = eng.gather_at(np.arange(nv, dtype=np.uint32))
         assert np.array_equal(a, b)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 65535, 65536, 65537, 70001])
+def test_lookups_at_the_end_of_the_pinned_words(n):
+    nv = 3001
+    rng = np.random.default_rng(n)
+    u = rng.integers(0, nv - 1, 9000)
+    k = np.unique(u * nv + u + 1)
+    row = np.zeros(nv + 1, np.uint64)
+    np.cumsum(np.bincount(k // nv, minlength=nv).astype(np.uint64), out=row[1:])
+    eng = sgraph.Engine("cc")
+    try:
+        eng.load_csr(row, (k % nv).astype(np.uint32))
+        eng.init()
+        v = eng.values()
+        ids = rng.integers(0, nv + 5, n).astype(np.uint32)  # ids past the graph read as 0xFFFFFFFF
+        exp = np.where(ids < nv, v[np.minimum(ids, nv - 1)], 0xFFFFFFFF)
+        assert np.array_equal(eng.gather_at(ids), exp)
+        assert np.array_equal(eng.gather_at(ids[::-1]), exp[::-1])
     finally:
         eng.close()
