@@ -77,6 +77,7 @@ public:
     api::PageRank op_{};
     float *value_ = nullptr, *buffer_ = nullptr;
     double *d_sum_ = nullptr;
+    bool sum_clear_ = false;  // d_sum_ is zero
     // pull rounds (cfg.pull_divisor != UINT32_MAX): the in-edge store, the
     // push arrays of alternating rounds, the partial sums of cut in-lists
     std::unique_ptr<GraphStore> rev_;
@@ -219,7 +220,7 @@ public:
         const uint32_t R = R_;
         PrState p = pr_state(R);
         p.cnt_zero = nullptr;
-        hipLaunchKernelGGL(k_pr_amend_take, dim3(1024), dim3(256), 0, stream_, (const uint32_t *)touched_,
+        hipLaunchKernelGGL(k_pr_amend_take, dim3(grid_for((uint64_t)nins_ + ndel_, 256, 1024)), dim3(256), 0, stream_, (const uint32_t *)touched_,
                            (const uint32_t *)&ctl_->tcount, nv_, p, type, pv_[R & 1]);
         SG_LAUNCHED();
         PassIO io = base_io();
@@ -320,7 +321,8 @@ public:
     }
 
     void residual() {
-        fill<unsigned long long>((unsigned long long *)d_sum_, 2, 0ull);
+        if (!sum_clear_) fill<unsigned long long>((unsigned long long *)d_sum_, 2, 0ull);
+        sum_clear_ = false;
         hipLaunchKernelGGL(k_pr_residual, dim3(grid_for(nv_, kBlock, 2048)), dim3(kBlock), 0, stream_, nv_, buffer_, d_sum_,
                            (unsigned long long *)(d_sum_ + 1));
         SG_LAUNCHED();
@@ -374,10 +376,11 @@ public:
     // starts round R_.
     template <bool kBothSigns>
     void seed() {
-        frontier_reset();
+        // a static solve starts from nothing (kBothSigns: a snapshot, which keeps l)
+        frontier_reset(pace_ ? ZeroRange{(unsigned long long *)sums_, (uint32_t)kPaceWords + (kBothSigns ? 0 : 1)} : ZeroRange{},
+                       ZeroRange{(unsigned long long *)d_sum_, 2});
+        sum_clear_ = true;
         if (pulls()) {
-            // a static solve starts from nothing (kBothSigns: a snapshot, which keeps l)
-            if (pace_) fill<unsigned long long>((unsigned long long *)sums_, kPaceWords + (kBothSigns ? 0 : 1), 0ull);
             PassIO io = base_io();
             io.ecnt_out = ecnt_ + (R_ % 3);
             hipLaunchKernelGGL(k_pr_seed<kBothSigns>, dim3(pr_grid()), dim3(kPrBlock), 0, stream_, nv_, pr_state(R_ - 1), io);
@@ -400,7 +403,7 @@ public:
         if (!inited_) fail(SG_EINVAL, "sg_apply before sg_init");
         auto t0 = std::chrono::steady_clock::now();
         const bool overflow = prepare(d_ins, nins, d_del, ndel);
-        frontier_reset();
+        if (!pulls()) frontier_reset();
         const uint32_t R = R_;
         const uint32_t *tc = &ctl_->tcount;
         if (pulls()) {

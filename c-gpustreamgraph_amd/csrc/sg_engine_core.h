@@ -272,11 +272,14 @@ __device__ __forceinline__ uint64_t off_at(const uint64_t *off, uint32_t nv, uin
     return v >= nv ? cap : off[v];
 }
 
-// New degree of every touched vertex from the chunk prefix; vertices that
-// outgrow their range mark their leaf dirty. Leaf and edge totals follow.
+// New degree of every touched vertex and the positions of its chunks in its
+// list (the prefix of their counts: one chunk as a rule, the wave walks 64 at a
+// time of a vertex that has more); vertices that outgrow their range mark their
+// leaf dirty. Leaf and edge totals follow.
 __global__ void __launch_bounds__(kBlock) k_newdeg(GraphView g, const TInfo *tinfo, const uint32_t *tcount,
-                                                   const unsigned long long *cpos, uint32_t *newdeg, uint8_t *leaf_dirty,
-                                                   uint32_t L, unsigned long long *leaf_cnt, Ctl *ctl) {
+                                                   const unsigned long long *ccount, unsigned long long *cpos,
+                                                   uint32_t *newdeg, uint8_t *leaf_dirty, uint32_t L,
+                                                   unsigned long long *leaf_cnt, Ctl *ctl) {
     __shared__ unsigned long long s_sum[kWavesPerBlock];
     __shared__ bool s_over[kWavesPerBlock];
     const uint32_t n = *tcount;
@@ -285,9 +288,29 @@ __global__ void __launch_bounds__(kBlock) k_newdeg(GraphView g, const TInfo *tin
         const uint64_t t = base + threadIdx.x;
         long long delta = 0;
         bool over = false;
+        TInfo ti{};
+        if (t < n) ti = tinfo[t];
+        unsigned long long kept = 0;  // what the vertex's chunks hold
+        if (ti.nch == 1) {
+            kept = ccount[ti.cbase];
+            cpos[ti.cbase] = 0;
+        }
+        for (uint64_t m = __ballot(ti.nch > 1); m; m &= m - 1) {
+            const int l = __ffsll((unsigned long long)m) - 1;
+            const uint32_t cb = (uint32_t)__builtin_amdgcn_readlane((int)ti.cbase, l);
+            const uint32_t nc = (uint32_t)__builtin_amdgcn_readlane((int)ti.nch, l);
+            unsigned long long sum = 0;
+            for (uint32_t c0 = 0; c0 < nc; c0 += kWave) {
+                const uint32_t c = c0 + lane_id();
+                const unsigned long long x = c < nc ? ccount[cb + c] : 0ull;
+                const unsigned long long incl = wave_incl_scan(x);
+                if (c < nc) cpos[cb + c] = sum + incl - x;
+                sum += __shfl(incl, kWave - 1, kWave);
+            }
+            if ((int)lane_id() == l) kept = sum;
+        }
         if (t < n) {
-            const TInfo ti = tinfo[t];
-            const uint32_t nd = has_del(ti) ? (uint32_t)(cpos[ti.cbase + ti.nch] - cpos[ti.cbase]) : ti.d0 + ti.ni;
+            const uint32_t nd = has_del(ti) ? (uint32_t)kept : ti.d0 + ti.ni;
             newdeg[ti.u] = nd;
             if (nd > g.off[ti.u + 1] - g.off[ti.u]) {
                 leaf_dirty[ti.u / L] = 1;
@@ -422,8 +445,8 @@ __global__ void __launch_bounds__(kBlock) k_win_gather(GraphView g, BatchView bv
                                                        const unsigned long long *wv_off, uint64_t Wv,
                                                        const unsigned long long *P, const uint32_t *mark,
                                                        const uint32_t *tidx, const TInfo *tinfo,
-                                                       const unsigned long long *cpos, const MChunk *chunks,
-                                                       const uint32_t *merged, uint32_t *out) {
+                                                       const unsigned long long *ccount, const unsigned long long *cpos,
+                                                       const MChunk *chunks, const uint32_t *merged, uint32_t *out) {
     const uint64_t gw = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / kWave;
     const uint32_t lane = lane_id();
@@ -438,11 +461,11 @@ __global__ void __launch_bounds__(kBlock) k_win_gather(GraphView g, BatchView bv
         if (bit_test(mark, v)) {
             const TInfo ti = tinfo[tidx[v]];
             if (ti.de > ti.db && chunks[ti.cbase].ibase == kInPlace) {  // compacted where it lies
-                keep_old = (uint32_t)(cpos[ti.cbase + 1] - cpos[ti.cbase]);
+                keep_old = (uint32_t)ccount[ti.cbase];
             } else if (ti.de > ti.db) {  // survivors of old list + inserts, staged by the filter chunk by chunk
                 for (uint32_t c = ti.cbase; c < ti.cbase + ti.nch; ++c) {
                     const uint32_t *src = merged + chunks[c].ibase;
-                    const uint64_t at = cpos[c] - cpos[ti.cbase], cnt = cpos[c + 1] - cpos[c];
+                    const uint64_t at = cpos[c], cnt = ccount[c];
                     for (uint64_t k = lane; k < cnt; k += kWave) dst[at + k] = src[k];
                 }
                 continue;
@@ -485,6 +508,19 @@ __global__ void __launch_bounds__(kBlock) k_win_scatter(const Window *win, uint3
             deg[x.vlo + il] = (uint32_t)nd;
         }
     }
+}
+
+// Counters before a run of rounds, in one launch: the frontier counters, the
+// out-edge and push-array counters, the stats of timed rounds, and up to two
+// ranges of the caller's.
+struct ZeroRange {
+    unsigned long long *p;
+    uint32_t n;
+};
+__global__ void __launch_bounds__(256) k_reset(uint32_t *cnt, ZeroRange a, ZeroRange b, ZeroRange c, ZeroRange d) {
+    if (threadIdx.x < 8) cnt[threadIdx.x] = 0;  // word 7 stays zero: an empty list count
+    for (const ZeroRange &r : {a, b, c, d})
+        for (uint32_t i = threadIdx.x; i < r.n; i += blockDim.x) r.p[i] = 0;
 }
 
 __global__ void k_set_u64(uint64_t *p, uint64_t v) { *p = v; }
@@ -551,15 +587,23 @@ __global__ void __launch_bounds__(kBlock) k_inval_seed(Op op, const unsigned lon
     }
 }
 
-// Relax each inserted edge that survived the batch's deletes.
+// Seeds of a traversal recompute, in one launch: blocks [0, na) activate the
+// invalidated vertices that are active on their own and clear the bitmaps, the
+// others relax each inserted edge that survived the batch's deletes. (A vertex
+// that both find joins once: the stamp.)
 template <class Op>
-__global__ void __launch_bounds__(kBlock) k_insert_relax(Op op, BatchView bv, BatchRanges br, typename Op::buffer_t *buffer,
-                                                         uint32_t *stamp, uint32_t stamp_val, uint32_t wmode,
-                                                         uint64_t wseed, uint32_t *list, uint32_t *cnt, uint32_t cap,
-                                                         unsigned long long *stats) {
+__global__ void __launch_bounds__(kBlock) k_reseed(uint32_t nv, uint32_t na, uint32_t *inval, uint32_t *coarse, uint32_t cshift,
+                                                   const typename Op::value_t *value, Op op, BatchView bv, BatchRanges br,
+                                                   typename Op::buffer_t *buffer, uint32_t *stamp, uint32_t stamp_val,
+                                                   uint32_t wmode, uint64_t wseed, uint32_t *list, uint32_t *cnt,
+                                                   uint32_t cap, unsigned long long *stats) {
     __shared__ BlockAppend sh;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < bv.nins; base += stride) {
+    if (blockIdx.x < na) {
+        inval_activate(nv, op, inval, coarse, cshift, value, buffer, stamp, stamp_val, list, cnt, cap, stats + 3, blockIdx.x, na);
+        return;
+    }
+    const uint64_t stride = (uint64_t)(gridDim.x - na) * blockDim.x;
+    for (uint64_t base = (uint64_t)(blockIdx.x - na) * blockDim.x; base < bv.nins; base += stride) {
         const uint64_t i = base + threadIdx.x;
         bool p = false;
         uint32_t v = 0;
@@ -687,6 +731,7 @@ public:
     std::string last_error_ = "no error";
     hipStream_t stream_ = nullptr;
     bool own_stream_ = true;
+    const uint32_t *sort_relabel_ = nullptr;  // the batch sort records targets by these ids (k_relabel_pairs: larger batches)
     bool swap_pairs_ = false;  // batches are read as (v, u): the in-edge store of another engine
     sg_stats st_{};
 
@@ -1338,8 +1383,10 @@ public:
         SweepTiles t{tile_v_, tile_e_, std::min<uint64_t>(tile_v_cap_, tile_e_cap_)};
         hipLaunchKernelGGL(k_deg_block_sums, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, bsum_);
         SG_LAUNCHED();
-        hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, bsum_);
-        SG_LAUNCHED();
+        if (nb > kScanOwn) {
+            hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, bsum_, bsum_);
+            SG_LAUNCHED();
+        }
         hipLaunchKernelGGL(k_deg_scan_write, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, bsum_, dpre_);
         SG_LAUNCHED();
         const uint64_t ntiles = ((uint64_t)nv_ + ne_ + kSweepTile - 1) / kSweepTile;
@@ -1378,10 +1425,13 @@ public:
     // and spills into hq[R % 3]; it clears cnt[(R + 2) % 3] and hc[(R + 1) % 3],
     // whose readers have finished. Seed passes before round R append to
     // round R's frontier and spill into hq[(R + 2) % 3].
-    void frontier_reset() {  // word 7 stays zero: an empty list count
-        fill<uint32_t>(cnt_, 8, 0);
-        fill<unsigned long long>(ecnt_, 6, 0ull);  // and pcnt
+    void frontier_reset(ZeroRange a = {}, ZeroRange b = {}) {
+        hipLaunchKernelGGL(k_reset, dim3(1), dim3(256), 0, stream_, cnt_, ZeroRange{ecnt_, 6},  // and pcnt
+                           ZeroRange{stats_ + 8, 8}, a, b);
+        SG_LAUNCHED();
+        timed_clear_ = true;
     }
+    bool timed_clear_ = false;  // no timed round has counted since the last reset
 
     PassIO base_io() const {
         PassIO io{};
@@ -1627,7 +1677,8 @@ public:
         uint32_t k = std::max<uint32_t>(1, std::min<uint32_t>(k0, kRoundLog));
         const uint32_t maxr = cfg_.max_rounds ? cfg_.max_rounds : 1000000u;
         const bool do_time = timed && timing(SG_KCLASS_RELAX);
-        if (timed) fill<unsigned long long>(stats_ + 8, 8, 0ull);
+        if (timed && !timed_clear_) fill<unsigned long long>(stats_ + 8, 8, 0ull);
+        timed_clear_ = false;
         uint32_t rounds = 0;
         bool first = true;
         last_appended_ = 0;
@@ -1744,6 +1795,7 @@ public:
         sb.nv = nv_;
         sb.a = swap_pairs_ ? 1 : 0;
         sb.b = swap_pairs_ ? 0 : 1;
+        sb.relabel = sort_relabel_;
         sb.dropped = &ctl_->dropped;
         const uint32_t *const pairs[2] = {d_ins, d_del};
         const uint32_t n[2] = {nins, ndel};
@@ -1818,10 +1870,9 @@ public:
         ensure(chunks_, chunks_cap_, chunk_bound);
         ensure(ccount_, ccount_cap_, chunk_bound + 1);
         ensure(cpos_, cpos_cap_, chunk_bound + 1);
-        fill<uint8_t>((uint8_t *)ctl_, sizeof(Ctl), 0);
-        fill<unsigned long long>(ccount_, chunk_bound + 1, 0ull);
-        size_t b1 = 0, b2 = 0, b3 = 0;
-        SG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, b3, ccount_, cpos_, (int)(chunk_bound + 1), stream_));
+        static_assert(sizeof(Ctl) % 8 == 0, "cleared in words");
+        fill<unsigned long long>((unsigned long long *)ctl_, sizeof(Ctl) / 8, 0ull);
+        size_t b1 = 0, b2 = 0;
         // sort only the bits ids can hold: kb = bit length of nv, so a masked
         // kGap / ~0 (dropped pair) still compares above every valid key
         const int kb = nv_ ? 32 - __builtin_clz(nv_) : 1;
@@ -1829,7 +1880,7 @@ public:
             SG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b1, ins_k_, ins_k2_, ins_v_, ins_v2_, (int)nins, 0, kb, stream_));
             SG_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, b2, del_k_, del_k2_, (int)ndel, 0, 32 + kb, stream_));
         }
-        ensure(cub_tmp_, cub_cap_, std::max({b1, b2, b3}) + 256);
+        if (!own_sort) ensure(cub_tmp_, cub_cap_, std::max(b1, b2) + 256);
         size_t b = cub_cap_;
         if (own_sort) {
             sort_batch(d_ins, nins, d_del, ndel);
@@ -1860,16 +1911,14 @@ public:
                 ensure(tmp_, tmp_cap_, std::max<uint64_t>(h_ctl_->seqcur, 1));
             }
             begin_timed(timing(SG_KCLASS_MERGE), SG_KCLASS_MERGE);
-            hipLaunchKernelGGL(k_chunk_filter, dim3(kGridFilter), dim3(kBlock), 0, stream_, gview(), bv_,
+            hipLaunchKernelGGL(k_chunk_filter, dim3(chunk_grid(kGridFilter)), dim3(kBlock), 0, stream_, gview(), bv_,
                                (const MChunk *)chunks_, &ctl_->nchunks, (uint32_t)chunk_bound, ccount_, tmp_, col_);
             SG_LAUNCHED();
             end_timed(timing(SG_KCLASS_MERGE));
         }
-        b = cub_cap_;
-        SG_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp_, b, ccount_, cpos_, (int)(chunk_bound + 1), stream_));
         if (nins + ndel) {
             hipLaunchKernelGGL(k_newdeg, dim3(grid_for((uint64_t)nins + ndel, kBlock, 8192)), dim3(kBlock), 0, stream_, gview(),
-                               tinfo_, &ctl_->tcount, cpos_, newdeg_, leaf_dirty_, L_, leaf_cnt_, ctl_);
+                               tinfo_, &ctl_->tcount, (const unsigned long long *)ccount_, cpos_, newdeg_, leaf_dirty_, L_, leaf_cnt_, ctl_);
             SG_LAUNCHED();
         }
         publish(h_ctl_, ctl_, sizeof(Ctl));
@@ -1878,20 +1927,26 @@ public:
         return h_ctl_->overflow != 0;
     }
 
+    // Blocks of a kernel with one wave per chunk: vertices with deletes or more
+    // than kLaneIns inserts have chunks, one each and one more per kMergeChunk
+    // entries (an empty block of 8192 costs 1 to 2 ns: more than a small batch).
+    uint32_t chunk_grid(uint32_t most) const {
+        return grid_for(ndel_ + nins_ / kLaneIns + (ne_ + nins_) / kMergeChunk + 1, kWavesPerBlock, most);
+    }
+
     void commit(bool overflow) {
         const Ctl c = *h_ctl_;
         const uint64_t ne_new = ne_ + (uint64_t)(long long)c.ne_delta;
         if (nins_ + ndel_) {
             if (overflow) rebalance(ne_new);  // moves the touched vertices of its windows
             begin_timed(timing(SG_KCLASS_MERGE), SG_KCLASS_MERGE);
-            hipLaunchKernelGGL(k_chunk_place, dim3(kGridList), dim3(kBlock), 0, stream_, gview(), bv_, col_, tinfo_, chunks_,
-                               &ctl_->nchunks, (uint32_t)chunk_bound_, cpos_, tmp_, newdeg_, maximal_, nleaves_, L_,
-                               overflow ? 1 : 0);
+            const uint32_t nc = chunk_grid(kGridList);
+            hipLaunchKernelGGL(k_place, dim3(nc + grid_for(c.tcount, kBlock, 4096)), dim3(kBlock), 0, stream_, gview(), bv_,
+                               col_, tinfo_, &ctl_->tcount,
+                               ChunkPlace{chunks_, &ctl_->nchunks, (uint32_t)chunk_bound_, ccount_, cpos_}, nc, tmp_, newdeg_,
+                               deg_, PlaceSkip{maximal_, nleaves_, L_, overflow ? 1 : 0});
             SG_LAUNCHED();
             end_timed(timing(SG_KCLASS_MERGE));
-            hipLaunchKernelGGL(k_lane_place, dim3(grid_for(c.tcount, 256, 4096)), dim3(256), 0, stream_, gview(), bv_, col_,
-                               tinfo_, &ctl_->tcount, newdeg_, deg_, maximal_, nleaves_, L_, overflow ? 1 : 0);
-            SG_LAUNCHED();
             if (cache_slots_) {
                 hipLaunchKernelGGL(k_cache_drop, dim3(1024), dim3(256), 0, stream_, tinfo_, &ctl_->tcount, coff_);
                 SG_LAUNCHED();
@@ -1912,7 +1967,7 @@ public:
         }
         cache_rebuild();
         if (nins_ + ndel_ == 0) return;
-        hipLaunchKernelGGL(k_clear_ranges, dim3(1024), dim3(256), 0, stream_, tinfo_, &ctl_->tcount, br_, mark_);
+        hipLaunchKernelGGL(k_clear_ranges, dim3(grid_for((uint64_t)nins_ + ndel_, 256, 1024)), dim3(256), 0, stream_, tinfo_, &ctl_->tcount, br_, mark_);
         SG_LAUNCHED();
     }
 
@@ -1985,7 +2040,7 @@ public:
         ensure(tmp2_, tmp2_cap_, std::max<uint64_t>(ne_new, 1));
         const uint32_t gw = grid_for(Wv, kWavesPerBlock, 16384);
         hipLaunchKernelGGL(k_win_gather, dim3(gw), dim3(kBlock), 0, stream_, gview(), bv_, win_, nwin, wvoff_, Wv, P_arr_, mark_,
-                           tidx_, tinfo_, cpos_, (const MChunk *)chunks_, tmp_, tmp2_);
+                           tidx_, tinfo_, ccount_, cpos_, (const MChunk *)chunks_, tmp_, tmp2_);
         SG_LAUNCHED();
         uint32_t *dst = col_;
         if (resize) {
@@ -2373,7 +2428,8 @@ public:
     size_t rl_ins_cap_ = 0, rl_del_cap_ = 0;
     void init(const uint32_t *, uint32_t) override { fail(SG_EINVAL, "a graph store has no vertex program"); }
     void apply(const uint32_t *d_ins, uint64_t nins, const uint32_t *d_del, uint64_t ndel) override {
-        if (relabel_) {  // the batch's sources as the in-lists record them
+        sort_relabel_ = nins <= kSortMost && ndel <= kSortMost ? relabel_ : nullptr;
+        if (relabel_ && !sort_relabel_) {  // the batch's sources as the in-lists record them
             if (nins) {
                 ensure(rl_ins_, rl_ins_cap_, 2 * nins);
                 hipLaunchKernelGGL(k_relabel_pairs, dim3(grid_for(nins, 256, 4096)), dim3(256), 0, stream_, d_ins, nins,
@@ -2529,13 +2585,13 @@ public:
         const uint32_t nb = (uint32_t)(((uint64_t)nv_ + kScanSpan - 1) / kScanSpan);
         ensure(bsum_, bsum_cap_, (size_t)nb + 1);
         ensure(pl_cnt_, pl_cnt_cap_, (size_t)nb + 1);
-        hipLaunchKernelGGL(k_plan_sums, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, bsum_, pl_cnt_);
+        hipLaunchKernelGGL(k_plan_sums, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, bsum_, pl_cnt_, pl_heads_,
+                           std::max<uint64_t>(1, nt) * (kPullTile / 32));
         SG_LAUNCHED();
-        hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, bsum_);
-        SG_LAUNCHED();
-        hipLaunchKernelGGL(k_deg_scan_sums, dim3(1), dim3(1024), 0, stream_, nb, pl_cnt_);
-        SG_LAUNCHED();
-        fill<uint32_t>(pl_heads_, std::max<uint64_t>(1, nt) * (kPullTile / 32), 0u);
+        if (nb > kScanOwn) {
+            hipLaunchKernelGGL(k_deg_scan_sums, dim3(2), dim3(1024), 0, stream_, nb, bsum_, pl_cnt_);
+            SG_LAUNCHED();
+        }
         unsigned long long *const start = dpre_;  // nv + 1 words: the first edge of every list
         hipLaunchKernelGGL(k_plan_lists, dim3(nb), dim3(kScanBlock), 0, stream_, nv_, deg_, (const unsigned long long *)bsum_,
                            (const unsigned long long *)pl_cnt_, start, pl_dst_, pl_heads_, pl_n_);
@@ -2898,16 +2954,14 @@ struct TravProgram {
                                    e.coarse_, e.cshift_};
                 e.sweep_all(tl, op, (const typename Op::buffer_t *)buffer, ef, io);
             }
-            // invalidated vertices active on their own (CC: own label); clears the bitmaps
-            hipLaunchKernelGGL(k_inval_activate<Op>, dim3(grid_for((e.nv_ + 31) / 32, 256, 4096)), dim3(256), 0, e.stream_, e.nv_,
-                               op, e.inval_, e.coarse_, e.cshift_, value, buffer, e.stamp_, R, e.q_[R & 1], e.cnt_ + (R % 3),
-                               e.nv_, e.stats_ + 3);
-            SG_LAUNCHED();
         }
-        if (e.nins_) {
-            hipLaunchKernelGGL(k_insert_relax<Op>, dim3(grid_for(e.nins_, kBlock, 8192)), dim3(kBlock), 0, e.stream_, op, e.bv_,
-                               e.br_, buffer, e.stamp_, R, e.cfg_.weight_mode, e.cfg_.weight_seed, e.q_[R & 1],
-                               e.cnt_ + (R % 3), e.nv_, e.stats_);
+        // invalidated vertices active on their own (CC: own label); inserted edges
+        const uint32_t na = ninval ? grid_for((e.nv_ + 31) / 32, kBlock, 4096) : 0u;
+        const uint32_t ni = e.nins_ ? grid_for(e.nins_, kBlock, 8192) : 0u;
+        if (na + ni) {
+            hipLaunchKernelGGL(k_reseed<Op>, dim3(na + ni), dim3(kBlock), 0, e.stream_, e.nv_, na, e.inval_, e.coarse_,
+                               e.cshift_, value, op, e.bv_, e.br_, buffer, e.stamp_, R, e.cfg_.weight_mode,
+                               e.cfg_.weight_seed, e.q_[R & 1], e.cnt_ + (R % 3), e.nv_, e.stats_);
             SG_LAUNCHED();
         }
         return relax_rounds(e, true, phase_relax);

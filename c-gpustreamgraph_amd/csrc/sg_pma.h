@@ -16,8 +16,9 @@
 //             old list in kMergeChunk pieces when it has deletes, and the
 //             inserts in kMergeChunk pieces
 //   count     one wave per chunk counts its survivors (delete set staged in LDS)
-//   scan      exclusive prefix of the counts = each chunk's output position
-//   newdeg    per vertex; a vertex that outgrows its range marks its PMA leaf
+//   newdeg    per vertex: the prefix of its chunks' counts (each chunk's output
+//             position in its list) and the new degree; a vertex that outgrows
+//             its range marks its PMA leaf
 //   write     one wave per chunk writes survivors, in order, to a scratch array
 //   place     one wave per chunk copies them back into the vertex's range and
 //             turns the freed tail into gaps
@@ -325,30 +326,43 @@ __device__ __forceinline__ bool covered(const uint8_t *maximal, uint64_t nleaves
     return false;
 }
 
+// Vertices of re-spread windows: placed by the window pass, skipped here.
+struct PlaceSkip {
+    const uint8_t *maximal;
+    uint64_t nleaves;
+    uint32_t L;
+    int on;
+    __device__ bool operator()(uint32_t u) const { return on && covered(maximal, nleaves, L, u); }
+};
+// Where the chunks of the batch's vertices go (k_newdeg).
+struct ChunkPlace {
+    const MChunk *chunks;
+    const uint32_t *nchunks;
+    uint32_t cap;
+    const unsigned long long *count, *pos;  // survivors of a chunk, position in its vertex's list
+};
+
 // One wave per chunk: copy the chunk's survivors into the vertex's own range
 // (from `merged` when it has deletes, from the sorted inserts otherwise) and
-// gap-fill the freed tail. Vertices in a window are skipped; the window
-// re-spread moves them.
-__global__ void __launch_bounds__(kBlock) k_chunk_place(GraphView g, BatchView bv, uint32_t *col, const TInfo *tinfo,
-                                                        const MChunk *chunks, const uint32_t *nchunks, uint32_t chunk_cap,
-                                                        const unsigned long long *cpos, const uint32_t *merged,
-                                                        const uint32_t *newdeg, const uint8_t *maximal,
-                                                        uint64_t nleaves, uint32_t L, int skip_covered) {
-    const uint32_t n = min(*nchunks, chunk_cap);
+// gap-fill the freed tail.
+__device__ __forceinline__ void chunk_place(const BatchView &bv, uint32_t *col, const ChunkPlace &cp, const uint32_t *merged,
+                                            const uint32_t *newdeg, const PlaceSkip &skip, uint32_t block, uint32_t blocks) {
+    const MChunk *const chunks = cp.chunks;
+    const uint32_t n = min(*cp.nchunks, cp.cap);
     const uint32_t w = threadIdx.x / kWave, lane = lane_id();
-    const uint64_t gw = (uint64_t)blockIdx.x * kWavesPerBlock + w;
-    const uint64_t nw = (uint64_t)gridDim.x * kWavesPerBlock;
+    const uint64_t gw = (uint64_t)block * kWavesPerBlock + w;
+    const uint64_t nw = (uint64_t)blocks * kWavesPerBlock;
     MChunk mn = load_chunk(chunks, gw, n);
     for (uint64_t c = gw; c < n; c += nw) {
         const MChunk m = mn;
         mn = load_chunk(chunks, c + nw, n);
         const TInfo ti = chunk_info(m);
         if (m.ibase == kInPlace) continue;  // compacted by the filter
-        if (skip_covered && covered(maximal, nleaves, L, ti.u)) continue;
+        if (skip(ti.u)) continue;
         uint32_t *lst = col + m.base;
         const bool hd = has_del(ti);
-        const uint64_t p0 = (hd ? 0 : ti.d0) + (cpos[c] - cpos[ti.cbase]);
-        const uint64_t len = cpos[c + 1] - cpos[c];
+        const uint64_t p0 = (hd ? 0 : ti.d0) + cp.pos[c];
+        const uint64_t len = cp.count[c];
         const uint32_t *srcp = hd ? merged + m.ibase : bv.ins_val + ti.ib + m.lo;
         // len <= kMergeChunk: one load per lane and covered wave row, all in flight
         const uint32_t nj = (uint32_t)((len + kWave - 1) / kWave);
@@ -375,13 +389,13 @@ __global__ void __launch_bounds__(kBlock) k_chunk_place(GraphView g, BatchView b
 // One lane per touched vertex: an insert-only vertex with a short insert run
 // appends it in place; every touched vertex takes its new degree (vertices
 // in a re-spread window were written by the window pass).
-__global__ void k_lane_place(GraphView g, BatchView bv, uint32_t *col, const TInfo *tinfo, const uint32_t *tcount,
-                             const uint32_t *newdeg, uint32_t *deg, const uint8_t *maximal, uint64_t nleaves, uint32_t L,
-                             int skip_covered) {
+__device__ __forceinline__ void lane_place(const GraphView &g, const BatchView &bv, uint32_t *col, const TInfo *tinfo,
+                                           const uint32_t *tcount, const uint32_t *newdeg, uint32_t *deg,
+                                           const PlaceSkip &skip, uint32_t block, uint32_t blocks) {
     const uint32_t n = *tcount;
-    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t t = (uint64_t)block * blockDim.x + threadIdx.x; t < n; t += (uint64_t)blocks * blockDim.x) {
         const TInfo ti = tinfo[t];
-        if (skip_covered && covered(maximal, nleaves, L, ti.u)) continue;
+        if (skip(ti.u)) continue;
         if (!chunked(ti) && ti.ni) {
             uint32_t *dst = col + g.off[ti.u] + ti.d0;
             const uint32_t *src = bv.ins_val + ti.ib;
@@ -389,6 +403,15 @@ __global__ void k_lane_place(GraphView g, BatchView bv, uint32_t *col, const TIn
         }
         deg[ti.u] = newdeg[ti.u];
     }
+}
+
+// Both in one launch (they write different vertices' lists): blocks [0, nc)
+// place chunks.
+__global__ void __launch_bounds__(kBlock) k_place(GraphView g, BatchView bv, uint32_t *col, const TInfo *tinfo,
+                                                  const uint32_t *tcount, ChunkPlace cp, uint32_t nc, const uint32_t *merged,
+                                                  const uint32_t *newdeg, uint32_t *deg, PlaceSkip skip) {
+    if (blockIdx.x < nc) chunk_place(bv, col, cp, merged, newdeg, skip, blockIdx.x, nc);
+    else lane_place(g, bv, col, tinfo, tcount, newdeg, deg, skip, blockIdx.x - nc, gridDim.x - nc);
 }
 
 // ---- edge-centric sweep ----------------------------------------------------------
@@ -441,8 +464,12 @@ __global__ void __launch_bounds__(kScanBlock) k_deg_block_sums(uint32_t nv, cons
     if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-// Phase 2 (one block): exclusive scan of the nb block sums in place.
-__global__ void __launch_bounds__(1024) k_deg_scan_sums(uint32_t nb, unsigned long long *bsum) {
+// Phase 2, for more than kScanOwn blocks (one block per array): exclusive scan
+// of the nb block sums in place. Up to kScanOwn, phase 3's blocks add up the
+// sums before their own themselves: four loads a thread against a launch.
+constexpr uint32_t kScanOwn = 1024;
+__global__ void __launch_bounds__(1024) k_deg_scan_sums(uint32_t nb, unsigned long long *bsum_a, unsigned long long *bsum_b) {
+    unsigned long long *const bsum = blockIdx.x ? bsum_b : bsum_a;
     __shared__ unsigned long long s_w[1024 / kWave];
     __shared__ unsigned long long s_carry;
     if (threadIdx.x == 0) s_carry = 0;
@@ -466,12 +493,22 @@ __global__ void __launch_bounds__(1024) k_deg_scan_sums(uint32_t nb, unsigned lo
     }
 }
 
+// What the blocks before this one hold, from their sums (scanned by phase 2, or not).
+__device__ __forceinline__ unsigned long long block_before(const unsigned long long *bsum, uint32_t nb,
+                                                           unsigned long long *s_w) {
+    if (nb > kScanOwn) return bsum[blockIdx.x];
+    unsigned long long x = 0, total;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanBlock) x += bsum[i];
+    block_excl_scan(x, s_w, total);
+    return total;
+}
+
 // Phase 3: dpre[v] for v in [0, nv].
 __global__ void __launch_bounds__(kScanBlock) k_deg_scan_write(uint32_t nv, const uint32_t *deg,
                                                                const unsigned long long *bsum, unsigned long long *dpre) {
-    __shared__ unsigned long long s_w[2][kScanBlock / kWave];
+    __shared__ unsigned long long s_w[3][kScanBlock / kWave];
     const uint64_t base = (uint64_t)blockIdx.x * kScanSpan;
-    unsigned long long carry = bsum[blockIdx.x];
+    unsigned long long carry = block_before(bsum, gridDim.x, s_w[2]);
     for (uint32_t i = 0; i < kScanIters; ++i) {
         const uint64_t v = base + (uint64_t)i * kScanBlock + threadIdx.x;
         const uint32_t d = v < nv ? deg[v] : 0u;
@@ -864,12 +901,12 @@ __global__ void __launch_bounds__(kSweepBlock) k_sweep_edges(GraphView g, const 
 // frontier: one thread per bitmap word. The sweep has read the bitmap and its
 // coarse filter for the last time: both are cleared here for the next batch.
 template <class Op>
-__global__ void k_inval_activate(uint32_t nv, Op op, uint32_t *inval, uint32_t *coarse, uint32_t cshift,
-                                 const typename Op::value_t *value, const typename Op::buffer_t *buffer, uint32_t *stamp,
-                                 uint32_t stamp_val, uint32_t *list, uint32_t *cnt, uint32_t cap,
-                                 unsigned long long *overflow) {
+__device__ __forceinline__ void inval_activate(uint32_t nv, const Op &op, uint32_t *inval, uint32_t *coarse, uint32_t cshift,
+                                               const typename Op::value_t *value, const typename Op::buffer_t *buffer,
+                                               uint32_t *stamp, uint32_t stamp_val, uint32_t *list, uint32_t *cnt,
+                                               uint32_t cap, unsigned long long *overflow, uint32_t block, uint32_t blocks) {
     const uint32_t nw = (nv + 31) / 32;
-    for (uint64_t wd = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; wd < nw; wd += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t wd = (uint64_t)block * blockDim.x + threadIdx.x; wd < nw; wd += (uint64_t)blocks * blockDim.x) {
         uint32_t bits = inval[wd];
         if (bits) inval[wd] = 0;
         if ((wd & ((1ull << cshift) - 1)) == 0) coarse[wd >> cshift] = 0;  // coarse word c covers words c << cshift ..

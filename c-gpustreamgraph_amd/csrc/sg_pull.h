@@ -88,9 +88,10 @@ struct PullPlan {
 };
 __host__ __device__ constexpr uint64_t pull_tile_words(uint32_t bits) { return (uint64_t)kPullTile / 32 * bits; }
 
-// Lists and edges per kScanSpan vertices.
+// Lists and edges per kScanSpan vertices; clears the nh words of heads.
 __global__ void __launch_bounds__(kScanBlock) k_plan_sums(uint32_t nv, const uint32_t *deg, unsigned long long *bsum,
-                                                          unsigned long long *bcnt) {
+                                                          unsigned long long *bcnt, uint32_t *heads, uint64_t nh) {
+    for (uint64_t i = (uint64_t)blockIdx.x * kScanBlock + threadIdx.x; i < nh; i += (uint64_t)gridDim.x * kScanBlock) heads[i] = 0;
     __shared__ unsigned long long s_w[2][kScanBlock / kWave];
     const uint64_t base = (uint64_t)blockIdx.x * kScanSpan;
     unsigned long long x = 0, c = 0;
@@ -110,13 +111,13 @@ __global__ void __launch_bounds__(kScanBlock) k_plan_sums(uint32_t nv, const uin
     }
 }
 // start[r], dst[r] of every list r, its head bit, start[lists] = ne, *nlists
-// (bsum / bcnt scanned). heads is zero before.
+// (bsum / bcnt: k_plan_sums). heads is zero before.
 __global__ void __launch_bounds__(kScanBlock) k_plan_lists(uint32_t nv, const uint32_t *deg, const unsigned long long *bsum,
                                                            const unsigned long long *bcnt, unsigned long long *start,
                                                            uint32_t *dst, uint32_t *heads, uint32_t *nlists) {
-    __shared__ unsigned long long s_w[4][kScanBlock / kWave];
+    __shared__ unsigned long long s_w[6][kScanBlock / kWave];
     const uint64_t base = (uint64_t)blockIdx.x * kScanSpan;
-    unsigned long long e0 = bsum[blockIdx.x], r0 = bcnt[blockIdx.x];
+    unsigned long long e0 = block_before(bsum, gridDim.x, s_w[4]), r0 = block_before(bcnt, gridDim.x, s_w[5]);
     for (uint32_t i = 0; i < kScanIters; ++i) {
         const uint64_t v = base + (uint64_t)i * kScanBlock + threadIdx.x;
         const uint32_t d = v < nv ? deg[v] : 0u;

@@ -48,6 +48,7 @@ struct SortBatch {
     SortSide side[2];  // inserts, deletes
     uint32_t nv;
     int a, b;                   // column of the source and of the target
+    const uint32_t *relabel;    // id that the targets are recorded by (null: as given)
     unsigned long long *dropped;  // pairs with an id >= nv, counted once
 };
 
@@ -57,7 +58,12 @@ __device__ __forceinline__ unsigned long long sort_key(const SortBatch &sb, int 
     const uint32_t u = x.pairs[2ull * i + sb.a], v = x.pairs[2ull * i + sb.b];
     const bool ok = u < sb.nv && v < sb.nv;
     if (s == 0) return ((unsigned long long)(ok ? u : kGap) << 32) | i;
-    return ok ? ((unsigned long long)u << 32) | v : ~0ull;
+    return ok ? ((unsigned long long)u << 32) | (sb.relabel ? sb.relabel[v] : v) : ~0ull;
+}
+// Target of insert i as the store records it.
+__device__ __forceinline__ uint32_t sort_target(const SortBatch &sb, uint32_t i) {
+    const uint32_t v = sb.side[0].pairs[2ull * i + sb.b];
+    return sb.relabel && v < sb.nv ? sb.relabel[v] : v;
 }
 __device__ __forceinline__ bool sort_dropped(int s, unsigned long long key) {
     return s == 0 ? (uint32_t)(key >> 32) == kGap : key == ~0ull;
@@ -236,7 +242,7 @@ __global__ void __launch_bounds__(kSortBlock) k_sort_buckets(SortBatch sb) {
             x.out_del[i] = k;
         } else {
             x.out_key[i] = (uint32_t)(k >> 32);
-            x.out_val[i] = x.pairs[2ull * (uint32_t)k + sb.b];
+            x.out_val[i] = sort_target(sb, (uint32_t)k);
         }
     };
     for (uint32_t i = hi + threadIdx.x; i < end; i += kSortBlock) put(i, x.tmp[i]);
