@@ -346,14 +346,16 @@ __device__ __forceinline__ void stage_push_n(const bool (&pred)[N], const uint32
     const uint32_t incl = wave_incl_scan(c);
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
     if (st.n + total > st.cap) stage_flush(st, io);
-    if (total > st.cap) {  // more than a slice at once
+    if (total > st.cap) {  // more than a slice at once: straight to the list
+        uint32_t pos = 0;
+        if (lane_id() == 0) pos = atomicAdd(io.out_cnt, total);
+        pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)pos) + incl - c;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            const uint64_t m = __ballot(pred[j]);
-            const uint32_t n = (uint32_t)__popcll(m);
-            if (st.n + n > st.cap) stage_flush(st, io);
-            if (pred[j]) st.buf[st.n + (uint32_t)__popcll(m & lanemask_lt())] = item[j];
-            st.n += n;
+            if (!pred[j]) continue;
+            if (pos < io.out_cap) io.out_list[pos] = item[j];
+            else atomicOr(io.stats + 3, 1ull);
+            ++pos;
         }
         return;
     }
@@ -416,17 +418,33 @@ struct alignas(16) LightWave {
 // LDS accesses of another width than the array's
 typedef uint32_t lds_u32x2 __attribute__((ext_vector_type(2), may_alias));
 
-// One step of edges: all their updates, then what they activate. Nothing
-// waits between the edges of a lane: the loads, the destination updates and
-// the stamp exchanges of a step are each in flight together.
+// One step of edges: their updates, EFn::kUpdates of a lane at a time, then what
+// they activate. The loads of a step are in flight together, and so are the
+// destination updates and the stamp exchanges of a group.
 template <class EFn>
 __device__ __forceinline__ void apply_edges(const PassIO &io, const EFn &efn, const uint32_t (&src)[kIlp],
                                             const uint32_t (&v)[kIlp], const uint32_t (&push)[kIlp], OutStage &st) {
+    constexpr int kN = EFn::kUpdates;
     uint64_t peek[kIlp];
 #pragma unroll
     for (int j = 0; j < kIlp; ++j) peek[j] = efn.load(v[j] != kGap ? v[j] : 0u);
     bool enq[kIlp];
-    efn.template apply_n<kIlp>(src, v, push, peek, enq);
+#pragma unroll
+    for (int h = 0; h < kIlp; h += kN) {
+        uint32_t s[kN], x[kN], p[kN];
+        uint64_t b[kN];
+        bool q[kN];
+#pragma unroll
+        for (int j = 0; j < kN; ++j) {
+            s[j] = src[h + j];
+            x[j] = v[h + j];
+            p[j] = push[h + j];
+            b[j] = peek[h + j];
+        }
+        efn.template apply_n<kN>(s, x, p, b, q);
+#pragma unroll
+        for (int j = 0; j < kN; ++j) enq[h + j] = q[j];
+    }
     if constexpr (EFn::kAppendSource) stage_push_n<kIlp>(enq, src, st, io);
     else stage_push_n<kIlp>(enq, v, st, io);
 }
@@ -632,8 +650,13 @@ __device__ __forceinline__ void block_stats(const WaveStats &ws, unsigned long l
 // the edge updates of every operator are order-insensitive (min-relaxations,
 // residual pushes), so the spilled lists of round R-1 are walked in round R
 // and whatever they activate joins round R+1.
+// A round waits for memory 70 % of its waves' time (SSSP, 65 M edges), so waves
+// in flight count: with all eight updates of a lane in flight SSSP and BFS took
+// 210 registers (2 waves per SIMD) and CC 148 (3). Five or six waves spill and
+// are slower again.
+constexpr int kRoundWaves = 4;  // per SIMD
 template <class VFn, class EFn>
-__global__ void __launch_bounds__(kBlock) k_round(GraphView g, PassIO io, VFn vfn, EFn efn) {
+__global__ void __launch_bounds__(kBlock, kRoundWaves) k_round(GraphView g, PassIO io, VFn vfn, EFn efn) {
     __shared__ LightWave s_wave[kWavesPerBlock];
     __shared__ unsigned long long s_red[kWavesPerBlock][4];
     __shared__ uint32_t s_n[kWavesPerBlock + 1];
@@ -770,6 +793,12 @@ struct EdgeFold<api::CC> {
 template <class Op>
 struct ERelax {
     static constexpr bool kAppendSource = false;
+    // Groups of 2, 4 and 8 updates at 4 waves per SIMD (8: spilling, so 2 waves
+    // for SSSP and BFS, 3 for CC), static solves in us: SSSP on 65 M edges 1817,
+    // 1848, 2002; BFS on 65 M 1189, 1232, 1446, on 12 M 388, 407, 486, on 1 M
+    // 155, 168, 188; CC on 65 M 3360, 3333, 3557, on 4 M 653, 590, 589, on 1 M
+    // 373, 340, 360. One at a time: 4 to 20 % more than 2.
+    static constexpr int kUpdates = !Op::kTraversal ? kIlp : EdgeFold<Op>::kKind == kFoldMin ? 2 : 4;
     Op op;
     typename Op::buffer_t *buffer;
     uint32_t *stamp;
@@ -882,6 +911,7 @@ struct ERelaxInval {
 template <class Op>
 struct EInvalidate {
     static constexpr bool kAppendSource = false;
+    static constexpr int kUpdates = kIlp;
     Op op;
     typename Op::value_t *value;
     typename Op::buffer_t *buffer;

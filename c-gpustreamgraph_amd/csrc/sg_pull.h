@@ -1061,6 +1061,7 @@ __global__ void __launch_bounds__(kSweepBlock) k_mirror_fill(GraphView g, const 
 template <class Op>
 struct EPullSeed {
     static constexpr bool kAppendSource = true;
+    static constexpr int kUpdates = kIlp;
     Op op;
     typename Op::buffer_t *buffer;
     uint32_t *stamp;
