@@ -660,11 +660,11 @@ struct HostSignal {
     uint32_t *word, *count;
     uint32_t val;
 };
-__device__ __forceinline__ void signal_host(const HostSignal &s) {
+__device__ __forceinline__ void signal_host(const HostSignal &s, uint32_t blocks) {
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x != 0) return;
-    if (atomicAdd(s.count, 1u) + 1 != gridDim.x) return;
+    if (atomicAdd(s.count, 1u) + 1 != blocks) return;
     *s.count = 0;
     __threadfence_system();
     __hip_atomic_store(s.word, s.val, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -673,7 +673,21 @@ __device__ __forceinline__ void signal_host(const HostSignal &s) {
 __global__ void __launch_bounds__(256) k_publish(const uint32_t *src, uint32_t n, uint32_t *dst, HostSignal s) {
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
-    signal_host(s);
+    signal_host(s, gridDim.x);
+}
+// Chunks of `chunk` words (a multiple of 4; 16-byte aligned) of n words to pinned
+// memory, kPublishBlocks blocks each, chunk c flagged at s.word[c] (s.count[c]).
+constexpr uint32_t kPublishBlocks = 16;
+__global__ void __launch_bounds__(256) k_publish_chunks(const uint32_t *src, uint64_t n, uint32_t chunk, uint32_t *dst,
+                                                        HostSignal s) {
+    const uint32_t c = blockIdx.x / kPublishBlocks, b = blockIdx.x % kPublishBlocks;
+    const uint64_t base = (uint64_t)c * chunk;
+    const uint32_t len = (uint32_t)min_u64(chunk, n - base);
+    const uint4 *const from = reinterpret_cast<const uint4 *>(src + base);
+    uint4 *const to = reinterpret_cast<uint4 *>(dst + base);
+    for (uint32_t i = b * 256 + threadIdx.x; i < len / 4; i += kPublishBlocks * 256) to[i] = from[i];
+    if (b == 0 && threadIdx.x < len % 4) dst[base + len / 4 * 4 + threadIdx.x] = src[base + len / 4 * 4 + threadIdx.x];
+    signal_host(HostSignal{s.word + c, s.count + c, s.val}, kPublishBlocks);
 }
 // k_gather_words with the ids read from pinned memory and the results stored there.
 __global__ void __launch_bounds__(256) k_gather_publish(const uint32_t *base, uint64_t stride, uint32_t word, uint32_t nv,
@@ -682,7 +696,7 @@ __global__ void __launch_bounds__(256) k_gather_publish(const uint32_t *base, ui
         const uint32_t v = verts[i];
         out[i] = v < nv ? base[(uint64_t)v * stride + word] : 0xFFFFFFFFu;
     }
-    signal_host(s);
+    signal_host(s, gridDim.x);
 }
 
 // Pointwise gather: out[i] = 32-bit word base[verts[i] * stride + word].
@@ -846,10 +860,6 @@ public:
         release_graphs();
         for (auto &ev : events_) { (void)hipEventDestroy(ev.first); (void)hipEventDestroy(ev.second); }
         events_.clear();
-        for (auto &ev : rb_ev_) {
-            if (ev) (void)hipEventDestroy(ev);
-            ev = nullptr;
-        }
         if (rb_) (void)hipHostFree(rb_);
         rb_ = nullptr;
         if (pinned_) (void)hipHostFree(pinned_);
@@ -1080,18 +1090,32 @@ public:
 
     // Device words to the caller's memory, waited for. A copy of megabytes into
     // pageable memory runs at what one core gets through page faults and a
-    // copy: chunks go to pinned staging, and threads take them from there while
-    // the next are on the link. 16 MB into pages already touched 950 -> 590 us,
-    // into new ones 1880 -> 810 us (the link alone: 300); chunks of 512 KiB 805
-    // and 965 us (a copy's start), 2 and 8 threads 20 to 30 % more on new pages.
-    // Below 2 MB the threads' start costs as much as they save.
-    static constexpr size_t kReadChunk = 1 << 20, kReadSlots = 8, kReadLeast = 2 << 20;
-    static constexpr uint32_t kReadThreads = 4;
+    // copy. Here a kernel stores chunks into pinned staging and flags each, and
+    // this and other threads take them from there: 16 MB into pages already
+    // touched 950 -> 430 us, into new ones 1880 -> 430 to 600 us (the link alone:
+    // 300), 4 MB 248 -> 146 us, 2 MB 156 -> 100 us. (Copies of 1 MiB with an
+    // event each: 590, 810, 215 and 160 us.) The threads start while the first
+    // chunks are on the link.
+    static constexpr size_t kReadChunk = 512 << 10, kReadHalf = 8, kReadSlots = 2 * kReadHalf;
+    static constexpr uint32_t kReadThreads = 3;  // beside the caller's
     char *rb_ = nullptr;
-    hipEvent_t rb_ev_[kReadSlots] = {};
+    uint32_t *rb_word_ = nullptr, *rb_count_ = nullptr;  // [kReadSlots] flags (pinned), arrivals
     void read_back(void *out, const void *src, size_t bytes) {
+        if (bytes <= kSmallWords * 4 && bytes % 4 == 0) {
+            publish(h_small_, src, bytes);
+            std::memcpy(out, h_small_, bytes);
+            return;
+        }
+        if (!rb_ || bytes % 4) {
+            SG_HIP(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream_));
+            sync();
+            return;
+        }
+        const size_t n = (bytes + kReadChunk - 1) / kReadChunk, halves = (n + kReadHalf - 1) / kReadHalf;
+        const uint32_t sig0 = sig_ + 1;  // chunks of half h are flagged with sig0 + h
+        sig_ += (uint32_t)halves;
         struct Readers {
-            std::atomic<size_t> next{0}, ready{0};  // chunks claimed, chunks in staging
+            std::atomic<size_t> next{0};
             std::atomic<bool> stop{false};
             std::vector<std::thread> th;
             ~Readers() {
@@ -1099,12 +1123,30 @@ public:
                 for (auto &t : th) t.join();
             }
         };
-        const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
-        std::vector<std::atomic<uint8_t>> taken(rb_ && bytes >= kReadLeast ? n : 0);
-        auto take = [&, this](Readers &r) {
+        std::vector<std::atomic<uint8_t>> taken(n);
+        size_t sent = 0;  // halves
+        auto send = [&] {  // the next half, once the staging it takes is free
+            if (sent == halves) return;
+            for (size_t i = sent >= 2 ? (sent - 2) * kReadHalf : n; i < n && i < (sent - 1) * kReadHalf; ++i)
+                if (!taken[i].load(std::memory_order_acquire)) return;
+            const size_t c0 = sent * kReadHalf, c1 = std::min(n, c0 + kReadHalf), slot = c0 % kReadSlots;
+            hipLaunchKernelGGL(k_publish_chunks, dim3((uint32_t)(c1 - c0) * kPublishBlocks), dim3(256), 0, stream_,
+                               (const uint32_t *)((const char *)src + c0 * kReadChunk),
+                               (std::min(bytes, c1 * kReadChunk) - c0 * kReadChunk) / 4, (uint32_t)(kReadChunk / 4),
+                               (uint32_t *)(rb_ + slot * kReadChunk),
+                               HostSignal{rb_word_ + slot, rb_count_ + slot, sig0 + (uint32_t)sent});
+            SG_LAUNCHED();
+            ++sent;
+        };
+        Readers r;
+        auto ready = [&, this](size_t i) {
+            return __atomic_load_n(rb_word_ + i % kReadSlots, __ATOMIC_ACQUIRE) == sig0 + (uint32_t)(i / kReadHalf);
+        };
+        auto take = [&, this](auto &&waiting) {
             for (size_t i = r.next++; i < n; i = r.next++) {
-                while (r.ready.load(std::memory_order_acquire) <= i) {
+                while (!ready(i)) {
                     if (r.stop) return;
+                    waiting();
                     __builtin_ia32_pause();
                 }
                 std::memcpy((char *)out + i * kReadChunk, rb_ + i % kReadSlots * kReadChunk,
@@ -1112,48 +1154,50 @@ public:
                 taken[i].store(1, std::memory_order_release);
             }
         };
-        Readers r;
-        if (!taken.empty()) {
-            try {
-                for (uint32_t t = 0; t < kReadThreads && t < n; ++t) r.th.emplace_back([&] { take(r); });
-            } catch (const std::system_error &) {  // no more threads: those there are do
-            }
+        send();
+        send();
+        try {
+            for (uint32_t t = 0; t < kReadThreads && t + 1 < n; ++t) r.th.emplace_back([&] { take([] {}); });
+        } catch (const std::system_error &) {  // no more threads: those there are do
         }
-        if (r.th.empty() && bytes <= kSmallWords * 4 && bytes % 4 == 0) {
-            publish(h_small_, src, bytes);
-            std::memcpy(out, h_small_, bytes);
-            return;
+        uint32_t spin = 0;
+        auto last = std::chrono::steady_clock::now();  // the device was busy
+        auto waiting = [&] {
+            send();
+            if (++spin % 16384) return;
+            const hipError_t e = hipStreamQuery(stream_);  // a fault would flag nothing
+            const auto now = std::chrono::steady_clock::now();
+            if (e == hipErrorNotReady) last = now;
+            else SG_HIP(e);
+            if (now - last > std::chrono::seconds(60)) fail(SG_EDEVICE, "the device finished without a signal");
+        };
+        take(waiting);
+        while (sent < halves) {  // the others have claimed what is not sent yet
+            waiting();
+            __builtin_ia32_pause();
         }
-        if (r.th.empty()) {
-            SG_HIP(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream_));
-            sync();
-            return;
-        }
-        for (size_t sent = 0, got = 0; got < n;) {
-            while (sent < n && (sent < kReadSlots || taken[sent - kReadSlots].load(std::memory_order_acquire))) {
-                SG_HIP(hipMemcpyAsync(rb_ + sent % kReadSlots * kReadChunk, (const char *)src + sent * kReadChunk,
-                                      std::min(kReadChunk, bytes - sent * kReadChunk), hipMemcpyDeviceToHost, stream_));
-                SG_HIP(hipEventRecord(rb_ev_[sent % kReadSlots], stream_));
-                ++sent;
-            }
-            if (got == sent) continue;
-            const hipError_t e = hipEventQuery(rb_ev_[got % kReadSlots]);
-            if (e == hipSuccess) r.ready.store(++got, std::memory_order_release);
-            else if (e != hipErrorNotReady) SG_HIP(e);
-        }
-        take(r);
         for (auto &t : r.th) t.join();
         r.th.clear();
     }
     // The staging of read_back, for engines whose results are that long (without it copies are plain).
     void read_staging(size_t bytes) {
-        if (bytes < kReadLeast || rb_) return;
-        if (hipHostMalloc((void **)&rb_, kReadSlots * kReadChunk, hipHostMallocDefault) != hipSuccess) {
+        if (bytes <= kSmallWords * 4 || rb_) return;
+        const size_t words = kReadSlots * kReadChunk;
+        void *p = nullptr, *dp = nullptr;
+        if (hipHostMalloc(&p, words + kReadSlots * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
-            rb_ = nullptr;
             return;
         }
-        for (auto &ev : rb_ev_) SG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        if (hipHostGetDevicePointer(&dp, p, 0) != hipSuccess || dp != p) {
+            (void)hipGetLastError();
+            (void)hipHostFree(p);
+            return;
+        }
+        rb_ = (char *)p;
+        rb_word_ = (uint32_t *)(rb_ + words);
+        std::memset(rb_word_, 0, kReadSlots * 4);
+        rb_count_ = dalloc<uint32_t>(kReadSlots);
+        fill<uint32_t>(rb_count_, kReadSlots, 0u);
     }
 
     template <class T>

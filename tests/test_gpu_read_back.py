@@ -1,7 +1,8 @@
 """Results read through pinned staging: whole at the sizes where the chunks can go wrong.
 
-Chunks of 1 MiB through eight staging slots from 2 MiB on: a result just below,
-at and above a chunk and above the slots, read twice into fresh memory.
+Chunks of 512 KiB, eight to a launch, through sixteen staging slots: results just
+below, at and above a chunk, a launch and the slots (and below the 512 KiB that
+come in one piece), read twice into fresh memory.
 Degrees are known without the device; OFFSETS are 8-byte words. Pointwise reads
 of up to 65536 ids go through pinned words without copies.
 """
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 MB = 1 << 18  # 4-byte words
 
 
-@pytest.mark.parametrize("nv", [2 * MB - 1, 2 * MB, 2 * MB + 1, 3 * MB, 8 * MB + 1, 9 * MB - 3, 17 * MB + 5])
+@pytest.mark.parametrize("nv", [MB // 2 - 1, MB // 2, MB // 2 + 1, MB + 3, 4 * MB, 4 * MB + 1, 2 * MB - 1, 2 * MB, 2 * MB + 1, 3 * MB, 8 * MB + 1, 9 * MB - 3, 17 * MB + 5])
 def test_results_come_whole(nv):
     rng = np.random.default_rng(nv)
     deg = rng.integers(0, 3, nv).astype(np.uint32)
