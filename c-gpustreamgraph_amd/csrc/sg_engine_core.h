@@ -1787,8 +1787,11 @@ public:
                 finish_rounds(timed);
                 fail(SG_EDEVICE, "no convergence within " + std::to_string(maxr) + " rounds");
             }
-            // past the expected count the remaining rounds are few: restart small
-            k = adaptive && rounds == k ? 4u : std::min<uint32_t>(2 * k, 64);
+            // past the expected count the remaining rounds are few: restart
+            // small. With no count to go by, half of the rounds so far: a third
+            // of the launches at most find nothing to do (doubling: half).
+            if (adaptive || cfg_.rounds_per_sync) k = adaptive && rounds == k ? 4u : std::min<uint32_t>(2 * k, 64);
+            else k = std::min<uint32_t>(std::max<uint32_t>(4, rounds / 2), 64);
         }
     }
 
