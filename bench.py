@@ -678,7 +678,7 @@ def main():
     pulls = c3["pulls"]
     ms_pull = c3["ms_pull"]
     # memory traffic per dense pull launch, rocprofv3 FETCH_SIZE + WRITE_SIZE at C3 (committed summary)
-    traffic_c3, traffic_c3_src = measured_traffic("sg::k_pr_pull", "k_pr_pull_c3_prcc_rmat27.pmc.txt")
+    traffic_c3, traffic_c3_src = measured_traffic("sg::k_pr_step", "k_pr_step_c3_prcc_rmat27.pmc.txt")
     out = {
         "metric": "updated-edge GTEPS + p50/p99 snapshot latency, 1 MI355X, batched vs plain",
         "value": round(c3["batched"], 4),
@@ -709,7 +709,7 @@ def main():
                   "latency_p50_ms": pct([a + b for a, b in zip(res["pr"]["lat"], res["cc"]["lat"])], 50),
                   "latency_p99_ms": pct([a + b for a, b in zip(res["pr"]["lat"], res["cc"]["lat"])], 99)},
         "roofline": {
-            "kernel": "k_pr_pull + k_pr_pull_fix (PageRank pull rounds over the in-edge store: 8 B per in-edge + "
+            "kernel": "k_pr_step + k_pr_tail (PageRank pull rounds over the in-edge store: 8 B per in-edge + "
                       "24 B per vertex); in-lists read from a packed HBM copy, the rest from a packed host copy",
             "bound": "hbm",
             "achieved": round(c3["achieved"], 2) if c3["achieved"] else None,
