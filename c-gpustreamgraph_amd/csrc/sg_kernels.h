@@ -317,6 +317,7 @@ __device__ __forceinline__ void stage_flush(OutStage &st, const PassIO &io) {
         if (pos < io.out_cap) io.out_list[pos] = st.buf[i];
         else atomicOr(io.stats + 3, 1ull);
     }
+    wave_lds_sync();  // read by every lane before the slice fills again
     st.n = 0;
 }
 
