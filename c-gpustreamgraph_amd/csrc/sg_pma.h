@@ -265,8 +265,8 @@ __device__ __forceinline__ bool survives(uint32_t x, const BatchView &bv, const 
 // order, to out[ibase ...] and count them; an in-place chunk (kInPlace)
 // compacts its survivors into the vertex's own slots instead (every load is
 // in registers before the first store, a survivor only moves left, and slots
-// already holding their survivor are not rewritten) and gap-fills the freed
-// tail. Chunks of insert-only vertices keep everything: counted without reads
+// of the old list already holding their survivor are not rewritten) and
+// gap-fills the freed tail. Chunks of insert-only vertices keep everything: counted without reads
 // (they are placed straight from the sorted batch).
 __global__ void __launch_bounds__(kBlock) k_chunk_filter(GraphView g, BatchView bv, const MChunk *chunks,
                                                          const uint32_t *nchunks, uint32_t chunk_cap,
@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(kBlock) k_chunk_filter(GraphView g, BatchView 
             const bool keep = i < m.hi && survives(x[j], bv, ti, s_del[w], s_mask[w], ns);
             const uint64_t b = __ballot(keep);
             const uint32_t pos = cnt + (uint32_t)__popcll(b & lanemask_lt());
-            if (keep && (!inpl || pos != i)) dst[pos] = x[j];
+            if (keep && (!inpl || pos != i || i >= ti.d0)) dst[pos] = x[j];  // (an insert is in no slot yet)
             cnt += (uint32_t)__popcll(b);
         }
         if (inpl)

@@ -2,8 +2,9 @@
 that need no GPU: what a kernel reads and writes out of bounds, and the lists
 and results it makes.
 
-`library` builds it once per session; while the fixture is in use, sgraph calls
-it instead of libsgraph.so.
+While the `emulated` fixture is in use, sgraph calls that library (built once
+per session) instead of libsgraph.so; `backend` runs a test on it and, marked
+gpu, on the device.
 """
 import ctypes
 import os
@@ -57,3 +58,8 @@ def emulated(emulated_path, monkeypatch):
     so.emulation_reset()
     yield so
     so.emulation_reset()
+
+
+@pytest.fixture(params=["emulated", pytest.param("device", marks=pytest.mark.gpu)])
+def backend(request):
+    return request.getfixturevalue("emulated") if request.param == "emulated" else None

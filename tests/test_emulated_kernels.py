@@ -1,6 +1,9 @@
 """The engine's kernels on the CPU: every program on small graphs under update
 batches, its lists and results against the oracle, every access checked against
 the allocation it falls in.
+
+Odd batches hold what generated streams seldom do: deletes of edges that are not
+there, also from sources without edges; deletes of the batch's own inserts.
 """
 import numpy as np
 import pytest
@@ -24,13 +27,16 @@ def graph(r, nv, per_vertex):
     return row, p[:, 1].astype(np.uint32)
 
 
-def batch(r, nv, row, col, nins, ndel):
+def batch(r, nv, row, col, nins, ndel, odd):
     src = np.repeat(np.arange(nv), np.diff(row.astype(np.int64)))
     ins = r.integers(0, nv, (nins, 2))
     ins[:, 0] = np.where(r.random(nins) < 0.3, r.integers(0, nv), ins[:, 0])  # one source gains a third
     ins = ins[ins[:, 0] != ins[:, 1]]
     k = r.integers(0, len(col), ndel)
     dele = np.stack([src[k], col[k]], 1)
+    if odd:
+        dele = np.where((r.random(ndel) < 0.5)[:, None], r.integers(0, nv, (ndel, 2)), dele)
+        dele = np.where((r.random(ndel) < 0.2)[:, None], ins[r.integers(0, len(ins), ndel)], dele)
     return ins.astype(np.uint32), dele.astype(np.uint32)
 
 
@@ -60,7 +66,7 @@ def check_values(eng, algo, queries, row, col, tag):
         assert np.array_equal(eng.values(), exp), tag
 
 
-def run(algo, nv, per_vertex, sizes, seed, nq=0, **cfg):
+def run(algo, nv, per_vertex, sizes, seed, nq=0, odd=False, **cfg):
     r = np.random.default_rng(seed)
     row, col = graph(r, nv, per_vertex)
     queries = [(["bfs", "sssp"][i % 2], int(r.integers(0, nv))) for i in range(nq)]
@@ -73,7 +79,7 @@ def run(algo, nv, per_vertex, sizes, seed, nq=0, **cfg):
             eng.init(0 if algo in ("bfs", "sssp") else None)
         check_values(eng, algo, queries, row, col, "G0")
         for t, (nins, ndel) in enumerate(sizes):
-            ins, dele = batch(r, nv, row, col, nins, ndel)
+            ins, dele = batch(r, nv, row, col, nins, ndel, odd)
             eng.apply(ins, dele)
             row, col = O.apply_updates(row, col, ins, dele)
             check_lists(eng, row, col, f"G{t + 1}")
@@ -85,21 +91,21 @@ def run(algo, nv, per_vertex, sizes, seed, nq=0, **cfg):
 SIZES = [(400, 400), (5, 40), (2500, 2500)]
 
 
-@pytest.mark.parametrize("density", [0.25, 1.0])
+@pytest.mark.parametrize("density,odd", [(0.25, False), (0.25, True), (1.0, False), (1.0, True)])
 @pytest.mark.parametrize("algo,cfg", [
     ("bfs", {}), ("sssp", dict(flags=sgraph.FLAG_IN_EDGES)), ("cc", {}), ("cc", dict(flags=HOST, segments=5, cache_level=4)),
     ("pr", {}), ("pr", dict(pull_divisor=sgraph.PULL_ALWAYS)), ("pr", dict(pull_divisor=sgraph.PULL_NEVER)),
     ("prcc", dict(flags=HOST, segments=5, edge_budget_gb=2e-5)),
 ])
-def test_programs(emulated, algo, cfg, density):
-    run(algo, 700, 5, SIZES, seed=31, pma_density=density, **cfg)
+def test_programs(emulated, algo, cfg, density, odd):
+    run(algo, 700, 5, SIZES, seed=31, odd=odd, pma_density=density, **cfg)
 
 
 def test_streamed_pulls(emulated):
     run("pr", 200, 5, SIZES[:2], seed=33, flags=HOST | sgraph.FLAG_PULL_STREAM, segments=2, pull_divisor=sgraph.PULL_ALWAYS)
 
 
-@pytest.mark.parametrize("density", [0.25, 1.0])
+@pytest.mark.parametrize("density,odd", [(0.25, False), (0.25, True), (1.0, True)])
 @pytest.mark.parametrize("nq", [3, 20, 70])  # one light group, one group of 32, two of 64
-def test_batched_queries(emulated, nq, density):
-    run("multi", 700, 5, SIZES, seed=32, nq=nq, pma_density=density)
+def test_batched_queries(emulated, nq, density, odd):
+    run("multi", 700, 5, SIZES, seed=32, nq=nq, odd=odd, pma_density=density)
