@@ -460,9 +460,10 @@ __global__ void __launch_bounds__(kBlock) k_win_gather(GraphView g, BatchView bv
         uint64_t ntail = 0;
         if (bit_test(mark, v)) {
             const TInfo ti = tinfo[tidx[v]];
-            if (ti.de > ti.db && chunks[ti.cbase].ibase == kInPlace) {  // compacted where it lies
+            // (with deletes but an empty sequence it has no chunk, and cbase is another's)
+            if (has_del(ti) && ti.nch == 1 && chunks[ti.cbase].ibase == kInPlace) {  // compacted where it lies
                 keep_old = (uint32_t)ccount[ti.cbase];
-            } else if (ti.de > ti.db) {  // survivors of old list + inserts, staged by the filter chunk by chunk
+            } else if (has_del(ti)) {  // survivors of old list + inserts, staged by the filter chunk by chunk
                 for (uint32_t c = ti.cbase; c < ti.cbase + ti.nch; ++c) {
                     const uint32_t *src = merged + chunks[c].ibase;
                     const uint64_t at = cpos[c], cnt = ccount[c];

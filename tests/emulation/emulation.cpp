@@ -62,6 +62,7 @@ void *lane_arg;
 int error = hipSuccess;
 std::string fail_kernel;  // emulation_fail_launch
 int fail_after = -1;
+bool backwards = false;  // emulation_backwards
 struct Range {
     char *map, *user;
     size_t mapped, bytes;
@@ -211,7 +212,10 @@ void run(const void *kernel, dim3 grid, dim3 block, void (*fn)(void *), void *ar
     blockDim = block;
     lane_fn = fn;
     lane_arg = arg;
-    for (blockIdx.x = 0; blockIdx.x < grid.x && !error; ++blockIdx.x) run_block((int)block.x);
+    for (uint32_t b = 0; b < grid.x && !error; ++b) {
+        blockIdx.x = backwards ? grid.x - 1 - b : b;
+        run_block((int)block.x);
+    }
     cur = nullptr;
     if (error) new_stacks();
 }
@@ -246,7 +250,10 @@ extern "C" {
 void emulation_reset() {
     emulation::error = hipSuccess;
     emulation::fail_after = -1;
+    emulation::backwards = false;
 }
+// Blocks run from the last to the first.
+void emulation_backwards() { emulation::backwards = true; }
 void emulation_fail_launch(const char *kernel, int after) {
     emulation::fail_kernel = kernel;
     emulation::fail_after = after;
