@@ -1068,16 +1068,7 @@ public:
     // that copies them also stores the word the host polls: a copy, an event
     // and its query took 10 us more per wait, and a snapshot waits three to
     // six times.
-    // Engines with their edges in host memory wait and copy through the runtime
-    // (their kernels take milliseconds): a run of the largest such configuration
-    // faulted in an update with signals, and the cause is not known.
-    bool signals() const { return !host_edges_; }
     void publish(void *dst, const void *src, size_t bytes) {
-        if (!signals()) {
-            SG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_));
-            sync();
-            return;
-        }
         const uint32_t n = (uint32_t)(bytes / 4);
         hipLaunchKernelGGL(k_publish, dim3(grid_for(n, 1024, 128)), dim3(256), 0, stream_, (const uint32_t *)src, n,
                            (uint32_t *)dst, next_signal());
@@ -1111,7 +1102,7 @@ public:
     char *rb_ = nullptr;
     uint32_t *rb_word_ = nullptr, *rb_count_ = nullptr;  // [kReadSlots] flags (pinned), arrivals
     void read_back(void *out, const void *src, size_t bytes) {
-        if (signals() && bytes <= kSmallWords * 4 && bytes % 4 == 0) {
+        if (bytes <= kSmallWords * 4 && bytes % 4 == 0) {
             publish(h_small_, src, bytes);
             std::memcpy(out, h_small_, bytes);
             return;
@@ -1191,7 +1182,7 @@ public:
     }
     // The staging of read_back, for engines whose results are that long (without it copies are plain).
     void read_staging(size_t bytes) {
-        if (!signals() || bytes <= kSmallWords * 4 || rb_) return;
+        if (bytes <= kSmallWords * 4 || rb_) return;
         const size_t words = kReadSlots * kReadChunk;
         void *p = nullptr, *dp = nullptr;
         if (hipHostMalloc(&p, words + kReadSlots * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
@@ -2309,7 +2300,7 @@ public:
         uint64_t stride = 1;
         uint32_t word = 0;
         word_source(q, qi, base, stride, word);
-        if (signals() && n <= kSmallWords / 2) {
+        if (n <= kSmallWords / 2) {
             // no copies: 4096 ids 30 us with one each way and an event
             std::memcpy(h_small_, verts, n * 4);
             hipLaunchKernelGGL(k_gather_publish, dim3(grid_for(n, 256, 256)), dim3(256), 0, stream_, base, stride, word, nv_,
