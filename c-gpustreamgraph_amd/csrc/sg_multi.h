@@ -138,13 +138,11 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t m, uint32_t r) {
     return pos;
 }
 
-// Target in slot s of u's list. An entry that is no vertex (no live list holds
-// one) reads as u itself: weights are 1 at least, so the edge improves nothing,
-// and no vertex is its own tree parent.
-__device__ __forceinline__ uint32_t target_at(const GraphView &g, uint64_t s, uint32_t u) {
-    const uint32_t v = edge_at(g, s);
-    return v != kGap ? v : u;
-}
+// Entry v of u's list as a vertex. An entry that is none (no live list holds
+// one) stands for u itself: weights are 1 at least, so the edge improves
+// nothing, and no vertex is its own tree parent. (Applied where an id is used:
+// right after its load it would wait for the ids fetched ahead.)
+__device__ __forceinline__ uint32_t target_of(uint32_t v, uint32_t u) { return v != kGap ? v : u; }
 
 // A wave takes the lists of up to 64 (vertex, group) items at a time: lane i
 // holds item i's words, the lists are then walked one after the other, each
@@ -211,7 +209,7 @@ __device__ __forceinline__ void mwalk_sparse(const GraphView &g, const MultiStat
     const uint32_t lane = lane_id();
     for (uint32_t e0 = 0; e0 < len; e0 += kWave) {
         const bool in = e0 + lane < len;
-        const uint32_t v = e0 == 0 ? vv : target_at(g, start + min(e0 + lane, len - 1), u);
+        const uint32_t v = target_of(e0 == 0 ? vv : edge_at(g, start + min(e0 + lane, len - 1)), u);
         unsigned long long *const p = &ms.best[(uint64_t)v * ms.KP + grp * ms.QS];
         unsigned long long b[kSparseSlots];
 #pragma unroll
@@ -265,8 +263,7 @@ __device__ __forceinline__ void mwalk_items(const GraphView &g, const MultiState
     // comes later sets its bit again
     auto ids = [&](uint32_t i) {
         const uint32_t len = (uint32_t)__builtin_amdgcn_readlane((int)it.len, (int)i);
-        const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)it.u, (int)i);
-        return len ? target_at(g, read_lane_u64(it.start, (int)i) + min(lane, len - 1), u) : 0u;
+        return len ? edge_at(g, read_lane_u64(it.start, (int)i) + min(lane, len - 1)) : 0u;
     };
     auto dist = [&](uint32_t i) {
         const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)it.u, (int)i);
@@ -315,8 +312,9 @@ __device__ __forceinline__ void mwalk_items(const GraphView &g, const MultiState
         const uint64_t ones = wlog == 6 ? ~0ull : (1ull << (1u << wlog)) - 1;
         for (uint32_t e0 = 0; e0 < len; e0 += kWave) {
             const uint32_t ne = min(len - e0, (uint32_t)kWave);
+            vv = target_of(vv, u);
             const uint32_t wv = kMode == 0 ? sg_weight(ms.wmode, ms.wseed, u, vv) : 0u;
-            const uint32_t vnext = e0 + kWave < len ? target_at(g, start + min(e0 + kWave + lane, len - 1), u) : 0u;
+            const uint32_t vnext = e0 + kWave < len ? edge_at(g, start + min(e0 + kWave + lane, len - 1)) : 0u;
             uint64_t hit = 0;  // ranks of this lane's edge
             // edges past the last repeat it (lanes past ne hold its id): their
             // updates change nothing, their marks fall on the same vertex
