@@ -1115,15 +1115,8 @@ public:
         const size_t n = (bytes + kReadChunk - 1) / kReadChunk, halves = (n + kReadHalf - 1) / kReadHalf;
         const uint32_t sig0 = sig_ + 1;  // chunks of half h are flagged with sig0 + h
         sig_ += (uint32_t)halves;
-        struct Readers {
-            std::atomic<size_t> next{0};
-            std::atomic<bool> stop{false};
-            std::vector<std::thread> th;
-            ~Readers() {
-                stop = true;
-                for (auto &t : th) t.join();
-            }
-        };
+        std::atomic<size_t> next{0};
+        std::atomic<bool> stop{false};
         std::vector<std::atomic<uint8_t>> taken(n);
         size_t sent = 0;  // halves
         auto send = [&] {  // the next half, once the staging it takes is free
@@ -1139,14 +1132,13 @@ public:
             SG_LAUNCHED();
             ++sent;
         };
-        Readers r;
         auto ready = [&, this](size_t i) {
             return __atomic_load_n(rb_word_ + i % kReadSlots, __ATOMIC_ACQUIRE) == sig0 + (uint32_t)(i / kReadHalf);
         };
         auto take = [&, this](auto &&waiting) {
-            for (size_t i = r.next++; i < n; i = r.next++) {
+            for (size_t i = next++; i < n; i = next++) {
                 while (!ready(i)) {
-                    if (r.stop) return;
+                    if (stop) return;
                     waiting();
                     __builtin_ia32_pause();
                 }
@@ -1155,10 +1147,18 @@ public:
                 taken[i].store(1, std::memory_order_release);
             }
         };
+        struct Readers {  // gone before what they use
+            std::atomic<bool> &stop;
+            std::vector<std::thread> th;
+            ~Readers() {
+                stop = true;
+                for (auto &t : th) t.join();
+            }
+        } readers{stop, {}};
         send();
         send();
         try {
-            for (uint32_t t = 0; t < kReadThreads && t + 1 < n; ++t) r.th.emplace_back([&] { take([] {}); });
+            for (uint32_t t = 0; t < kReadThreads && t + 1 < n; ++t) readers.th.emplace_back([&] { take([] {}); });
         } catch (const std::system_error &) {  // no more threads: those there are do
         }
         uint32_t spin = 0;
@@ -1173,12 +1173,13 @@ public:
             if (now - last > std::chrono::seconds(60)) fail(SG_EDEVICE, "the device finished without a signal");
         };
         take(waiting);
-        while (sent < halves) {  // the others have claimed what is not sent yet
-            waiting();
-            __builtin_ia32_pause();
-        }
-        for (auto &t : r.th) t.join();
-        r.th.clear();
+        // what the others have claimed: only this thread sends the rest, and sees a
+        // device that will flag nothing more
+        for (size_t i = 0; i < n; ++i)
+            while (!taken[i].load(std::memory_order_acquire)) {
+                if (!ready(i)) waiting();
+                __builtin_ia32_pause();
+            }
     }
     // The staging of read_back, for engines whose results are that long (without it copies are plain).
     void read_staging(size_t bytes) {

@@ -215,7 +215,7 @@ static inline hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, in
     return hipSuccess;
 }
 static inline hipError_t hipMemcpy(void *to, const void *from, size_t n, int kind) { return hipMemcpyAsync(to, from, n, kind); }
-static inline hipError_t hipGetLastError() { return emulation::status(); }
+static inline hipError_t hipGetLastError() { return hipSuccess; }  // a failed kernel shows at a wait, a copy or a query
 static inline hipError_t hipSetDevice(int) { return hipSuccess; }
 static inline hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 static inline hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
