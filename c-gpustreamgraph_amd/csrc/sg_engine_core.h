@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <sched.h>
+
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -737,6 +739,13 @@ static void parallel_for(uint64_t n, Fn fn) {
     for (auto &x : th) x.join();
 }
 
+// Cores that the calling thread may run on.
+static uint32_t usable_cores() {
+    cpu_set_t set;
+    if (sched_getaffinity(0, sizeof set, &set) == 0) return (uint32_t)std::max(1, CPU_COUNT(&set));
+    return std::max(1u, std::thread::hardware_concurrency());
+}
+
 class Engine {
 public:
     explicit Engine(const sg_config &cfg) : cfg_(cfg) {}
@@ -1098,7 +1107,7 @@ public:
     // event each: 590, 810, 215 and 160 us.) The threads start while the first
     // chunks are on the link.
     static constexpr size_t kReadChunk = 512 << 10, kReadHalf = 8, kReadSlots = 2 * kReadHalf;
-    static constexpr uint32_t kReadThreads = 3;  // beside the caller's
+    static constexpr uint32_t kReadThreads = 3;  // beside the caller's, where there are cores for them
     char *rb_ = nullptr;
     uint32_t *rb_word_ = nullptr, *rb_count_ = nullptr;  // [kReadSlots] flags (pinned), arrivals
     void read_back(void *out, const void *src, size_t bytes) {
@@ -1158,7 +1167,12 @@ public:
         send();
         send();
         try {
-            for (uint32_t t = 0; t < kReadThreads && t + 1 < n; ++t) readers.th.emplace_back([&] { take([] {}); });
+            const uint32_t others = std::min<uint32_t>(kReadThreads, usable_cores() - 1);
+            for (uint32_t t = 0; t < others && t + 1 < n; ++t)
+                readers.th.emplace_back([&] {
+                    uint32_t spin = 0;  // the cores may have others waiting for them
+                    take([&] { if (++spin % 64 == 0) std::this_thread::yield(); });
+                });
         } catch (const std::system_error &) {  // no more threads: those there are do
         }
         uint32_t spin = 0;
