@@ -2575,10 +2575,15 @@ public:
 
     // PageRank owners: the pull plan (sg_pull.h). Resident store: all its ids,
     // where the device budget has room (it is given back when something else
-    // needs the memory; pulls then read the slots). Store in pinned host
+    // needs the memory; pulls then read the slots, until a later batch finds
+    // room again). Store in pinned host
     // memory: HBM holds as many tiles of ids as the edge budget allows, the
     // rest are packed straight into pinned host memory.
-    bool want_plan_ = false, plan_ok_ = false, plan_refused_ = false;
+    bool want_plan_ = false, plan_ok_ = false;
+    // Batches to go without a plan after it was given back or found no room: 1, 2,
+    // 4, ... up to kPlanMostWait, so that memory which stays short costs little.
+    static constexpr uint32_t kPlanMostWait = 64;
+    uint32_t plan_wait_ = 0, plan_next_wait_ = 1;
     PullPlan plan_{};
     uint32_t *pl_ids_ = nullptr, *pl_tail_ = nullptr, *pl_heads_ = nullptr, *pl_dst_ = nullptr;
     PullTileMeta *pl_meta_ = nullptr;
@@ -2608,7 +2613,8 @@ public:
         pl_meta_ = nullptr;
         pl_ids_cap_ = pl_heads_cap_ = pl_meta_cap_ = 0;
         plan_ok_ = false;
-        plan_refused_ = true;
+        plan_wait_ = plan_next_wait_;
+        plan_next_wait_ = std::min(2 * plan_next_wait_, kPlanMostWait);
     }
     bool plan_building_ = false;
     bool give_back() override {
@@ -2619,7 +2625,10 @@ public:
     }
     bool refresh_plan() {
         plan_ok_ = false;
-        if (plan_refused_) return false;
+        if (plan_wait_) {
+            --plan_wait_;
+            return false;
+        }
         const uint32_t b = mbits_ = id_bits();
         const uint64_t nt = (ne_ + kPullTile - 1) / kPullTile, words = pull_tile_words(b);
         const uint64_t in_hbm = host_edges_ ? std::min(nt, budget_words() / words) : nt;
