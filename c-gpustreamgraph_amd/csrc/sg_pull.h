@@ -1004,19 +1004,6 @@ __device__ __forceinline__ void copy_run(uint32_t *arr, unsigned long long i0, u
     }
 }
 
-// First tile whose edges reach past live-edge index x (every tile before it
-// ends at or below x); nt when none.
-__device__ __forceinline__ unsigned long long tile_reaching(const SweepTiles &tiles, unsigned long long nt,
-                                                            unsigned long long x) {
-    unsigned long long lo = 0, hi = nt;
-    while (lo < hi) {
-        const unsigned long long mid = (lo + hi) / 2;
-        if (tiles.e[mid + 1] > x) hi = mid;
-        else lo = mid + 1;
-    }
-    return lo;
-}
-
 // HBM copy of the store's leading live edges, read from the store in host
 // memory through the tile sweep (live slots only, coalesced): copy id k = live
 // edge k (merge-path order) for k < mlive. g must carry no copy itself, and a
