@@ -28,7 +28,8 @@ def build(out_dir):
         pytest.skip("no clang++ to build the kernels for the CPU")
     inc = ["-I", HERE, "-I", os.path.join(ROOT, "include"), "-I", os.path.join(PKG, "csrc"), "-I", os.path.join(PKG, "host")]
     flags = ["-std=c++17", "-O1", "-fPIC", "-w", "-x", "c++"]
-    sources = [os.path.join(PKG, "csrc", "sg_engine.hip"), os.path.join(HERE, "emulation.cpp"),
+    sources = [os.path.join(HERE, "plan.cpp"),  # with sg_engine.hip
+               os.path.join(HERE, "emulation.cpp"),
                os.path.join(PKG, "host", "sg_io.cpp"), os.path.join(PKG, "host", "sg_server.cpp")]
 
     def compile_one(src):
