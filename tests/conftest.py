@@ -9,6 +9,8 @@ for p in (PKG, os.path.join(ROOT, "oracle")):
     if p not in sys.path:
         sys.path.insert(0, p)
 
+from emulated import backend, emulated, emulated_path  # noqa: E402,F401 (fixtures)
+
 GOLDEN = os.path.join(ROOT, "tests", "golden")
 
 

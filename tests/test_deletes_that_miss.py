@@ -11,7 +11,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import backend, emulated, emulated_path  # noqa: F401 (fixtures)
 
 OLD = (0, 1, 5, 63, 64, 65, 130)  # entries before the batch
 NEW = (1, 2, 63, 64, 65, 129)     # inserts

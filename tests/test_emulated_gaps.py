@@ -8,7 +8,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import emulated, emulated_path  # noqa: F401 (fixtures)
 
 GAP = 0xFFFFFFFF
 

@@ -10,7 +10,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import emulated, emulated_path  # noqa: F401 (fixtures)
 
 PR_REL_TOL = 5e-5
 HOST = sgraph.FLAG_HOST_EDGES

@@ -10,7 +10,6 @@ import ctypes
 import numpy as np
 import pytest
 
-from emulated import emulated, emulated_path  # noqa: F401 (fixtures)
 
 TILE = 512  # kPullTile
 

@@ -12,7 +12,6 @@ import sys
 
 import pytest
 
-from emulated import emulated_path  # noqa: F401 (fixture)
 
 CHILD = """
 import ctypes, sys

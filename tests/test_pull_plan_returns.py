@@ -9,7 +9,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import backend, emulated, emulated_path  # noqa: F401 (fixtures)
 
 PR_REL_TOL = 5e-5
 NV, NE = 700, 20000

@@ -10,7 +10,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import backend, emulated, emulated_path  # noqa: F401 (fixtures)
 
 
 def csr(lists, nv):

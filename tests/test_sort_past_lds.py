@@ -10,7 +10,6 @@ import pytest
 
 import oracle as O
 import sgraph
-from emulated import backend, emulated, emulated_path  # noqa: F401 (fixtures)
 
 NV = 3000
 BUCKET, OVER, MOST_SPLIT, LDS = 768, 8, 512, 8192  # sg_sort.h: kSortBucket, kSortOver, kSortMaxSplit, kSortLds
